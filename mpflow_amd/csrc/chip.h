@@ -1,0 +1,42 @@
+// On-chip PCG (chip.hip): whole solves of the meshes whose Krylov vectors fit one CU.
+#pragma once
+
+#include "jobs.h"
+
+namespace mpf {
+
+// A workgroup keeps one (job, harmonic) and a group of G right-hand-side lanes: p in LDS
+// (80 KB), r, x and q in registers, K rows x G lanes per thread.
+constexpr int kChipMaxRows = 20480;   // padded rows of the largest mesh (G = 1)
+constexpr int kChipMaxWidth = 32;     // padded ELL width (2 bits of 8-slot groups)
+constexpr int kChipCus = 256;         // one workgroup each
+
+struct ChipShape {
+    int G = 0, K = 0, threads = 0;
+};
+// The shape for np padded rows when a solve has `lanes` (job, harmonic, lane) triples in
+// all.  Enough lanes to fill the chip: the largest group, 512 threads; fewer: the smallest
+// group that keeps every workgroup on a CU of its own, 1024 threads.
+ChipShape chip_shape(int np, long long lanes);
+
+// gst flags of a lane group
+constexpr int kChipCapped = 1, kChipNan = 2, kChipEmpty = 4;
+
+// pos -> row and row -> pos of the chip order (each tile's rows by aggregate, 64 positions
+// per aggregate, padding rows in the holes); *bad is set when an aggregate has more than 64 rows
+void launch_chip_order(int n, int np, const uint8_t* aggq, uint16_t* rowof, uint16_t* posof, int* bad,
+                       hipStream_t st);
+// column positions of the ELL in chip order: [width / 8][np] x 8 ids of 16 bits; octs[np / 64]:
+// 8-slot groups in use per 64 positions
+void launch_chip_ids(int np, int width, const int32_t* ids, const uint8_t* gw, const uint16_t* rowof,
+                     const uint16_t* posof, uint4* cid, uint8_t* octs, hipStream_t st);
+// values S + alpha_c R of every (job, slice) pair of the list: J.cval [C][width / 8][2][np] float4
+void launch_chip_pack(const JobDev* d_jobs, const int2* d_js, int njs, int max_np, hipStream_t st);
+// one phase over `n` items (job, slice, lane group, index of the pair's first group state):
+// phase 0 runs every lane group from its start to its own stop test; phase 1 takes the
+// groups behind their pair's largest step count (gin) on to it.  gout receives every group's
+// (steps, flags).
+void launch_chip(const JobDev* d_jobs, const int4* d_items, int n, const ChipShape& c, const int2* gin, int2* gout,
+                 int phase, hipStream_t st);
+
+}  // namespace mpf

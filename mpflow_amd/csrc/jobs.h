@@ -75,6 +75,12 @@ struct JobDev {
     float* csc;                  // [4 ntiles] Sc^-1/2 (written after each assembly)
     float* cy;                   // [C][4 ntiles][Rp] coarse correction Einv W^T r
     float* cg;                   // [C][4 ntiles][Rp] Sc^-1/2 W^T r of the current iteration
+    // on-chip PCG (chip.hip; set by the Krylov driver for jobs that fit): the matrix in chip
+    // order, positions of 16 bits
+    const uint16_t* crow;        // [np] device row of each position
+    const uint4* cid;            // [width / 8][np] positions of 8 neighbours
+    const uint8_t* cocts;        // [np / 64] groups of 8 slots in use
+    float4* cval;                // [C][width / 8][2][np] S + alpha_c R
 };
 
 // PCG search direction of iteration k (k4 = k % kRing)

@@ -45,18 +45,20 @@ KrylovDriver::KrylovDriver(mpf_ctx* c, std::vector<std::vector<JobDev>*> sources
     hipStream_t s0 = ctx->stream;
     MPF_HIP(hipMemsetAsync(st.p, 0, st.bytes(), s0));
     // groups by (lane count, padded width)
-    std::vector<int4> all_tiles;
-    std::vector<int2> all_js;
+    std::vector<int4> all_tiles, str_tiles;
+    std::vector<int2> all_js, str_js;
     for (int j = 0; j < nj; ++j) {
         const JobDev& J = h[j];
+        const bool chip = J.np <= kChipMaxRows && J.width <= kChipMaxWidth && J.gw;
         Group* g = nullptr;
         for (auto& q : groups)
-            if (q.lg == J.lg && q.wpad == J.width) g = &q;
+            if (q.lg == J.lg && q.wpad == J.width && q.chip == chip) g = &q;
         if (!g) {
             groups.emplace_back();
             g = &groups.back();
             g->lg = J.lg;
             g->wpad = J.width;
+            g->chip = chip;
         }
         g->jobs.push_back(j);
         // the 128-bit gather kernels keep byte offsets of a slice vector in 31 bits
@@ -64,6 +66,9 @@ KrylovDriver::KrylovDriver(mpf_ctx* c, std::vector<std::vector<JobDev>*> sources
         for (int c = 0; c < J.C; ++c) {
             all_js.push_back(make_int2(j, c));
             for (int t = 0; t < J.ntiles; ++t) all_tiles.push_back(make_int4(j, c, t, 0));
+            if (chip) continue;
+            str_js.push_back(make_int2(j, c));
+            for (int t = 0; t < J.ntiles; ++t) str_tiles.push_back(make_int4(j, c, t, 0));
         }
     }
     size_t total = 0;
@@ -122,6 +127,17 @@ KrylovDriver::KrylovDriver(mpf_ctx* c, std::vector<std::vector<JobDev>*> sources
     init_tiles.upload(ordered.data(), ordered.size(), s0);
     init_js.alloc(n_init_js);
     init_js.upload(all_js.data(), all_js.size(), s0);
+    n_stream_tiles = (int)str_tiles.size();
+    n_stream_js = (int)str_js.size();
+    if (n_stream_js) {
+        std::vector<int4> so(str_tiles.size());
+        xcd_order(str_tiles.data(), n_stream_tiles, so.data());
+        stream_tiles.alloc(n_stream_tiles);
+        stream_tiles.upload(so.data(), so.size(), s0);
+        stream_js.alloc(n_stream_js);
+        stream_js.upload(str_js.data(), str_js.size(), s0);
+        MPF_HIP(hipStreamSynchronize(s0));   // so goes out of scope
+    }
     MPF_HIP(hipHostMalloc((void**)&h_active, sizeof(int), hipHostMallocDefault));
     MPF_HIP(hipHostMalloc((void**)&h_st, st.bytes(), hipHostMallocDefault));
     std::memset(h_st, 0, st.bytes());
@@ -136,6 +152,178 @@ KrylovDriver::~KrylovDriver() {
     if (h_active) (void)hipHostFree(h_active);
     if (h_st) (void)hipHostFree(h_st);
     if (h_tiles) (void)hipHostFree(h_tiles);
+    if (h_gst) (void)hipHostFree(h_gst);
+    for (auto& c : chips) {
+        if (c.done) (void)hipEventDestroy(c.done);
+        if (c.stream) (void)hipStreamDestroy(c.stream);
+    }
+    if (chip_fork) (void)hipEventDestroy(chip_fork);
+}
+
+// Tables of the on-chip PCG (chip.hip), once per driver: the chip order and 16-bit matrix of
+// every mesh, room for the values of every (job, slice), and the work items per class.
+bool KrylovDriver::ensure_chip() {
+    if (chip_tried) return chip_ok;
+    chip_tried = true;
+    const int nj = (int)h.size();
+    chip_mesh_of.assign(nj, -1);
+    cval_off.assign(nj, 0);
+    std::vector<int> jobs_on;
+    for (const auto& g : groups)
+        if (g.chip) jobs_on.insert(jobs_on.end(), g.jobs.begin(), g.jobs.end());
+    if (jobs_on.empty()) return false;
+    std::sort(jobs_on.begin(), jobs_on.end());
+    hipStream_t s0 = ctx->stream;
+    try {
+        DBuf<int> bad(1);
+        int hbad = 0;
+        bad.upload(&hbad, 1, s0);
+        size_t nval = 0;
+        for (int j : jobs_on) {
+            const JobDev& J = h[j];
+            int m = -1;
+            for (size_t i = 0; i < chip_meshes.size(); ++i)
+                if (chip_meshes[i]->ids == J.ids) m = (int)i;
+            if (m < 0) {
+                m = (int)chip_meshes.size();
+                chip_meshes.emplace_back(new ChipMesh);
+                ChipMesh& M = *chip_meshes.back();
+                M.ids = J.ids;
+                M.crow.alloc(J.np);
+                M.cpos.alloc(J.np);
+                M.cid.alloc((size_t)J.width / 8 * J.np);
+                M.octs.alloc(J.np / 64);
+                launch_chip_order(J.n, J.np, J.aggq, M.crow.p, M.cpos.p, bad.p, s0);
+                launch_chip_ids(J.np, J.width, J.ids, J.gw, M.crow.p, M.cpos.p, M.cid.p, M.octs.p, s0);
+            }
+            chip_mesh_of[j] = m;
+            cval_off[j] = nval;
+            nval += (size_t)J.C * J.width / 4 * J.np;
+            chip_max_np = std::max(chip_max_np, J.np);
+        }
+        cval.alloc(nval);
+        MPF_HIP(hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, s0));
+        MPF_HIP(hipStreamSynchronize(s0));
+        if (hbad) return false;   // an aggregate of more than 64 rows: streamed
+        long long lanes = 0;
+        for (int j : jobs_on) lanes += (long long)h[j].C * h[j].R;
+        // the longest pairs (low harmonics) first
+        int total = 0, cmax = 0;
+        for (int j : jobs_on) cmax = std::max(cmax, h[j].C);
+        for (int c = 0; c < cmax; ++c)
+            for (int j : jobs_on) {
+                const JobDev& J = h[j];
+                if (c >= J.C) continue;
+                const ChipShape sh = chip_shape(J.np, lanes);
+                ChipClass* cl = nullptr;
+                for (auto& q : chips)
+                    if (q.shape.G == sh.G && q.shape.K == sh.K && q.shape.threads == sh.threads) cl = &q;
+                if (!cl) {
+                    chips.emplace_back();
+                    cl = &chips.back();
+                    cl->shape = sh;
+                }
+                h_chip_js.push_back(make_int2(j, c));
+                chip_first.push_back(total);
+                for (int g = 0; g < J.Rp / sh.G; ++g) cl->h_items.push_back(make_int4(j, c, g, total));
+                total += J.Rp / sh.G;
+            }
+        // the groups of a pair on one XCD (block b runs on XCD b % 8), which then reads the
+        // pair's matrix into its L2 once: pair i goes to XCD i % 8
+        for (auto& cl : chips) {
+            std::vector<std::vector<int4>> on(kXcds);
+            int pairs = -1, last = -1;
+            for (const int4& it : cl.h_items) {
+                if (it.w != last) { ++pairs; last = it.w; }
+                on[pairs % kXcds].push_back(it);
+            }
+            cl.h_items.clear();
+            size_t longest = 0;          // pairs of 16 and of 32 lanes have different group counts
+            for (const auto& x : on) longest = std::max(longest, x.size());
+            for (size_t i = 0; i < longest; ++i)
+                for (const auto& x : on)
+                    if (i < x.size()) cl.h_items.push_back(x[i]);
+        }
+        chip_first.push_back(total);
+        size_t listed = 0;
+        for (const auto& cl : chips) listed += cl.h_items.size();
+        MPF_REQUIRE((int)listed == total, "krylov: on-chip work list incomplete");
+        std::sort(chips.begin(), chips.end(), [](const ChipClass& a, const ChipClass& b) {
+            return a.shape.K * a.shape.threads > b.shape.K * b.shape.threads;
+        });
+        for (size_t i = 0; i < chips.size(); ++i) {
+            ChipClass& c = chips[i];
+            c.items.alloc(c.h_items.size());
+            c.items.upload(c.h_items.data(), c.h_items.size(), s0);
+            if (i == 0) continue;
+            MPF_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
+            MPF_HIP(hipEventCreateWithFlags(&c.done, hipEventDisableTiming));
+        }
+        if (chips.size() > 1) MPF_HIP(hipEventCreateWithFlags(&chip_fork, hipEventDisableTiming));
+        chip_js.alloc(h_chip_js.size());
+        chip_js.upload(h_chip_js.data(), h_chip_js.size(), s0);
+        gst[0].alloc(total);
+        gst[1].alloc(total);
+        MPF_HIP(hipMemsetAsync(gst[0].p, 0, gst[0].bytes(), s0));
+        MPF_HIP(hipMemsetAsync(gst[1].p, 0, gst[1].bytes(), s0));
+        MPF_HIP(hipHostMalloc((void**)&h_gst, sizeof(int2) * total, hipHostMallocDefault));
+        MPF_HIP(hipStreamSynchronize(s0));
+    } catch (const Error& e) {
+        if (e.code != MPF_ENOMEM) throw;
+        // no room for the tables: the jobs are streamed
+        cval.release();
+        chip_meshes.clear();
+        return false;
+    }
+    chip_ok = true;
+    return true;
+}
+
+// One solve of every on-chip pair: phase 0, then phase 1 until the lane groups of every pair
+// have taken the same number of steps (usually once: it takes every group on to the step at
+// which the pair's slowest group stopped).  Step counts and flags go to h_st.
+void KrylovDriver::run_chip() {
+    hipStream_t s0 = ctx->stream;
+    launch_chip_pack(jobs.p, chip_js.p, (int)h_chip_js.size(), chip_max_np, s0);
+    const int total = chip_first.back();
+    auto phase = [&](int ph, int in) {
+        if (chips.size() > 1) MPF_HIP(hipEventRecord(chip_fork, s0));
+        for (auto& c : chips) {
+            hipStream_t s = c.stream ? c.stream : s0;
+            if (c.stream) MPF_HIP(hipStreamWaitEvent(s, chip_fork, 0));
+            launch_chip(jobs.p, c.items.p, (int)c.h_items.size(), c.shape, gst[in].p, gst[in ^ 1].p, ph, s);
+            if (c.stream) {
+                MPF_HIP(hipEventRecord(c.done, s));
+                MPF_HIP(hipStreamWaitEvent(s0, c.done, 0));
+            }
+        }
+    };
+    phase(0, 1);
+    int in = 0;
+    for (bool open = true; open;) {
+        phase(1, in);
+        in ^= 1;
+        MPF_HIP(hipMemcpyAsync(h_gst, gst[in].p, sizeof(int2) * total, hipMemcpyDeviceToHost, s0));
+        MPF_HIP(hipStreamSynchronize(s0));
+        open = false;
+        for (size_t i = 0; i < h_chip_js.size() && !open; ++i) {
+            int steps = 0;
+            for (int g = chip_first[i]; g < chip_first[i + 1]; ++g) steps = std::max(steps, h_gst[g].x);
+            for (int g = chip_first[i]; g < chip_first[i + 1]; ++g)
+                if (!h_gst[g].y && h_gst[g].x != steps) open = true;
+        }
+    }
+    for (size_t i = 0; i < h_chip_js.size(); ++i) {
+        int steps = 0, flags = 0;
+        for (int g = chip_first[i]; g < chip_first[i + 1]; ++g) {
+            steps = std::max(steps, h_gst[g].x);
+            flags |= h_gst[g].y & (kChipCapped | kChipNan);
+        }
+        int* sp = &h_st[((size_t)h_chip_js[i].x * kMaxSlices + h_chip_js[i].y) * kStInts];
+        sp[0] = 0;
+        sp[1] = steps;
+        sp[2] = flags ? 1 : 0;
+    }
 }
 
 void KrylovDriver::drop_graph() {
@@ -197,6 +385,14 @@ void KrylovDriver::tune(Group& g) {
     g.order = choice >> 4;
 }
 
+// whether every group's SpMV choice is in the context's cache
+bool KrylovDriver::tuned() {
+    std::lock_guard<std::mutex> lk(ctx->tune.mu);
+    for (const auto& g : groups)
+        if (!ctx->tune.spmv.count(g.key)) return false;
+    return true;
+}
+
 bool KrylovDriver::run(const mpf_solve_opts& o, int rule, double tol, bool use_rhs, bool ref_b,
                        mpf_solve_stats* stats) {
     hipStream_t s0 = ctx->stream;
@@ -206,6 +402,8 @@ bool KrylovDriver::run(const mpf_solve_opts& o, int rule, double tol, bool use_r
     const bool want_coarse = !bicg && o.preconditioner == MPF_PRECOND_TWO_LEVEL;
     if (want_coarse != coarse) drop_graph();
     coarse = want_coarse && init_nchunk > 0;
+    // small meshes run on chip; profiled runs stream, their SpMV launches are what is timed
+    const bool chip = !bicg && !ctx->prof && ensure_chip();
     for (int j = 0; j < nj; ++j) {
         JobDev& J = h[j];
         J = (*src[origin[j].first])[origin[j].second];
@@ -216,17 +414,36 @@ bool KrylovDriver::run(const mpf_solve_opts& o, int rule, double tol, bool use_r
         J.maxit = o.max_iter > 0 ? o.max_iter : 10 * J.n;
         J.use_rhs = use_rhs ? 1 : 0;
         J.ref_b = ref_b ? 1 : 0;
+        if (chip && chip_mesh_of[j] >= 0) {
+            const ChipMesh& M = *chip_meshes[chip_mesh_of[j]];
+            J.crow = M.crow.p;
+            J.cid = M.cid.p;
+            J.cocts = M.octs.p;
+            J.cval = cval.p + cval_off[j];
+        }
     }
     jobs.upload(h.data(), h.size(), s0);
     MPF_HIP(hipMemsetAsync(active.p, 0, sizeof(int), s0));
-    if (bicg) launch_bicg_init(jobs.p, init_tiles.p, n_init_tiles, init_js.p, n_init_js, active.p, 0, s0);
-    else launch_pcg_init(jobs.p, init_tiles.p, n_init_tiles, init_js.p, n_init_js, active.p, s0,
-                         coarse ? init_nchunk : 0);
+    const int4* itiles = chip ? stream_tiles.p : init_tiles.p;
+    const int2* ijs = chip ? stream_js.p : init_js.p;
+    const int nit = chip ? n_stream_tiles : n_init_tiles, nij = chip ? n_stream_js : n_init_js;
+    if (bicg) {
+        launch_bicg_init(jobs.p, init_tiles.p, n_init_tiles, init_js.p, n_init_js, active.p, 0, s0);
+    } else {
+        if (chip && !tuned()) {
+            // the candidates are timed on initialised pairs, streamed or not
+            launch_pcg_init(jobs.p, init_tiles.p, n_init_tiles, init_js.p, n_init_js, active.p, s0,
+                            coarse ? init_nchunk : 0);
+            for (auto& g : groups) tune(g);
+            MPF_HIP(hipMemsetAsync(active.p, 0, sizeof(int), s0));
+        }
+        if (nij) launch_pcg_init(jobs.p, itiles, nit, ijs, nij, active.p, s0, coarse ? init_nchunk : 0);
+    }
     for (auto& g : groups) {
         if (!bicg) tune(g);
         else g.order = 0;
         g.cur = g.tiles_o[g.order].p;
-        g.ncur = g.nall;
+        g.ncur = chip && g.chip ? 0 : g.nall;
         g.fcur = g.ftiles.p;
         g.nfcur = g.nfall;
     }
@@ -237,7 +454,7 @@ bool KrylovDriver::run(const mpf_solve_opts& o, int rule, double tol, bool use_r
     for (const auto& J : h) maxit = std::max(maxit, J.maxit);
     drop_graph();
     int it = 0;
-    while (true) {
+    while (nij > 0 || bicg) {
         if (graphs) {
             if (!gexec || gbicg != bicg || gevery != every) {
                 drop_graph();
@@ -271,6 +488,7 @@ bool KrylovDriver::run(const mpf_solve_opts& o, int rule, double tol, bool use_r
         // compact the work lists: always without graphs, otherwise once a quarter of the
         // listed tiles belong to finished pairs (finished pairs' blocks exit at once)
         for (auto& g : groups) {
+            if (chip && g.chip) continue;
             // the survivors in (job, slice, tile) or (job, tile, slice) order (a filter of
             // the unstriped list keeps its order), then striped over the XCDs again so that
             // XCD x gets a contiguous run of them
@@ -306,7 +524,8 @@ bool KrylovDriver::run(const mpf_solve_opts& o, int rule, double tol, bool use_r
         }
     }
     drop_graph();
-    if (!bicg) launch_pcg_flush(jobs.p, init_tiles.p, n_init_tiles, s0);
+    if (!bicg && nij) launch_pcg_flush(jobs.p, itiles, nit, s0);
+    if (chip) run_chip();
     bool capped = false;
     int64_t slice_iters = 0;
     double bytes = 0.0;

@@ -4,10 +4,11 @@
 #pragma once
 
 #include <map>
+#include <memory>
 #include <mutex>
 #include <vector>
 
-#include "jobs.h"
+#include "chip.h"
 
 struct mpf_ctx;
 
@@ -50,6 +51,7 @@ class KrylovDriver {
     struct Group {
         int lg = 0, wpad = 0, variant = 0;
         int order = 0;                // work-list order: 0 (job, slice, tile), 1 (job, tile, slice)
+        bool chip = false;            // jobs the on-chip PCG takes (CG without profiling)
         bool wide = false;            // a slice vector of >= 2^31 - 2^16 bytes: 32-bit-gather SpMV only
         long long key = 0;
         std::vector<int> jobs;        // indices into h
@@ -70,10 +72,39 @@ class KrylovDriver {
         const int4* fcur = nullptr;
         size_t fhoff = 0;
     };
+    // jobs of the on-chip PCG that share the lane group and the rows per thread
+    struct ChipClass {
+        ChipShape shape;
+        std::vector<int4> h_items;    // (job, slice, lane group, index of the pair's first group)
+        DBuf<int4> items;
+        hipStream_t stream = nullptr; // classes after the first run beside it
+        hipEvent_t done = nullptr;
+    };
+    struct ChipMesh {                 // one per ELL pattern
+        const int32_t* ids = nullptr;
+        DBuf<uint16_t> crow, cpos;
+        DBuf<uint4> cid;
+        DBuf<uint8_t> octs;
+    };
+    bool ensure_chip();               // false: no job fits, or no room for the tables
+    void run_chip();
+    bool chip_tried = false, chip_ok = false;
+    std::vector<ChipClass> chips;
+    std::vector<std::unique_ptr<ChipMesh>> chip_meshes;
+    std::vector<int> chip_mesh_of;    // per job (-1: streamed)
+    std::vector<int2> h_chip_js;      // the on-chip (job, slice) pairs
+    std::vector<int> chip_first;      // first group index of each pair; then the total
+    DBuf<int2> chip_js, gst[2];
+    DBuf<float4> cval;
+    std::vector<size_t> cval_off;     // per job
+    int chip_max_np = 0;
+    int2* h_gst = nullptr;            // pinned
+    hipEvent_t chip_fork = nullptr;
     void launch_group_iter(Group& g, int iter, bool bicg, hipStream_t s, hipEvent_t e0, hipEvent_t e1);
     bool coarse = false;              // this run uses the two-level preconditioner
     int init_nchunk = 0;
     void tune(Group& g);
+    bool tuned();
     void drop_graph();
 
     mpf_ctx* ctx;
@@ -84,7 +115,9 @@ class KrylovDriver {
     DBuf<int> st, active;
     DBuf<int4> init_tiles;            // every tile of every job (init kernels take any width)
     DBuf<int2> init_js;
-    int n_init_tiles = 0, n_init_js = 0;
+    DBuf<int4> stream_tiles;          // the same without the on-chip jobs
+    DBuf<int2> stream_js;
+    int n_init_tiles = 0, n_init_js = 0, n_stream_tiles = 0, n_stream_js = 0;
     std::vector<Group> groups;
     int* h_active = nullptr;          // pinned
     int* h_st = nullptr;              // pinned [njobs][kMaxSlices][kStInts]
