@@ -515,11 +515,11 @@ int mpf_spd_solve(mpf_ctx* ctx, int32_t n, const float* d_G, double shift, const
         MPF_REQUIRE(n > 0, "mpf_spd_solve: n <= 0");
         set_device(ctx);
         mpf::DBuf<double> A((size_t)n * n);
-        mpf::DBuf<int2> pairs(mpf::cholesky_pairs(n));
+        mpf::DBuf<double> fw(mpf::spd_factor_work(n, 1));
         mpf::DBuf<int> info(1);
         MPF_HIP(hipMemsetAsync(info.p, 0, sizeof(int), ctx->stream));
-        mpf::launch_cholesky(n, d_G, 0, shift, A.p, 0, 1, info.p, pairs.p, ctx->stream);
-        mpf::launch_potrs(n, A.p, 0, d_b, 0, d_y, 0, 1, ctx->stream);
+        mpf::launch_spd_factor(n, d_G, 0, shift, A.p, 0, 1, info.p, fw.p, ctx->stream);
+        mpf::launch_spd_solve(n, A.p, 0, d_b, 0, d_y, 0, 1, fw.p, ctx->stream);
         int h = 0;
         MPF_HIP(hipMemcpyAsync(&h, info.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         MPF_HIP(hipStreamSynchronize(ctx->stream));
@@ -540,7 +540,7 @@ int mpf_normal_solve(mpf_ctx* ctx, int32_t rows, int32_t cols, const float* d_J,
         mpf::DBuf<float> G((size_t)m * m);
         mpf::DBuf<double> A((size_t)m * m), y(m), dy(m), res(m), vE(E);
         mpf::DBuf<double> work(mpf::gemv_n_workspace(m, E, 1) / sizeof(double) + 1);
-        mpf::DBuf<int2> pairs(mpf::cholesky_pairs(m));
+        mpf::DBuf<double> fw(mpf::spd_factor_work(m, 1));
         mpf::DBuf<int> info(1);
         if (mpf::gram_nt_applies(m, ldj)) {
             mpf::DBuf<char> gw(mpf::gram_nt_workspace_bytes(m, E, 1));
@@ -552,12 +552,12 @@ int mpf_normal_solve(mpf_ctx* ctx, int32_t rows, int32_t cols, const float* d_J,
             MPF_HIP(hipStreamSynchronize(st));
         }
         MPF_HIP(hipMemsetAsync(info.p, 0, sizeof(int), st));
-        mpf::launch_cholesky(m, G.p, 0, shift, A.p, 0, 1, info.p, pairs.p, st);
-        mpf::launch_potrs(m, A.p, 0, d_r, 0, y.p, 0, 1, st);
+        mpf::launch_spd_factor(m, G.p, 0, shift, A.p, 0, 1, info.p, fw.p, st);
+        mpf::launch_spd_solve(m, A.p, 0, d_r, 0, y.p, 0, 1, fw.p, st);
         for (int k = 0; k < gn_refine; ++k) {
             mpf::launch_gemv_t(m, E, d_J, ldj, 0, y.p, 0, vE.p, 0, 1, st);
             mpf::launch_gemv_n(m, E, d_J, ldj, 0, vE.p, 0, shift, y.p, 0, d_r, 0, res.p, 0, 1, work.p, st);
-            mpf::launch_potrs(m, A.p, 0, res.p, 0, dy.p, 0, 1, st);
+            mpf::launch_spd_solve(m, A.p, 0, res.p, 0, dy.p, 0, 1, fw.p, st);
             mpf::launch_add_to(m, y.p, dy.p, st);
         }
         mpf::launch_gemv_t(m, E, d_J, ldj, 0, y.p, 0, d_delta, 0, 1, st);

@@ -70,14 +70,20 @@ void launch_gemv_n(int rows, int cols, const float* A, int lda, size_t strideA, 
                    size_t striderhs, double* out, size_t strideout, int batch, double* work,
                    hipStream_t st);
 
-// device int2 entries launch_cholesky needs for its update list (filled on the device)
+// FP64 solves of G + shift I (spd.hip).  Factor: A (n x n per batch entry, column-major, no
+// padding) receives X = L^-1 in its lower and X^T in its upper triangle; *d_info is set to 1
+// when a pivot is not positive; work: spd_factor_work doubles.
+size_t spd_factor_work(int n, int batch);
+void launch_spd_factor(int n, const float* G, size_t strideG, double shift, double* A, size_t strideA, int batch,
+                       int* d_info, double* work, hipStream_t st);
+// y = X^T (X b) for every batch entry (strideA 0: one factor for all); work: batch x n doubles;
+// y may be b
+void launch_spd_solve(int n, const double* A, size_t strideA, const double* b, size_t strideb, double* y,
+                      size_t stridey, int batch, double* work, hipStream_t st);
+// device int2 entries launch_cholesky_z needs for its update list (filled on the device)
 size_t cholesky_pairs(int n);
-void launch_cholesky(int n, const float* G, size_t strideG, double shift, double* A, size_t strideA,
-                     int batch, int* d_info, int2* d_pairs, hipStream_t st);
-void launch_potrs(int n, const double* A, size_t strideA, const double* b, size_t strideb, double* y,
-                  size_t stridey, int batch, hipStream_t st);
 // complex symmetric (not Hermitian) A = L L^T in place and its solves, FP64; A holds
-// both triangles of the already shifted matrices; d_pairs as for launch_cholesky
+// both triangles of the already shifted matrices; d_pairs: cholesky_pairs entries
 void launch_cholesky_z(int n, zd* A, size_t strideA, int batch, int* d_info, int2* d_pairs, hipStream_t st);
 void launch_potrs_z(int n, const zd* A, size_t strideA, const zd* b, size_t strideb, zd* y, size_t stridey,
                     int batch, hipStream_t st);

@@ -634,19 +634,8 @@ __global__ void __launch_bounds__(256) k_gemv_n_reduce(int rows, int nslab, cons
 // --------------------------------------------------------------------------------
 constexpr int kCB = 32;
 
-// A64 = G + shift I (and zero the strictly upper triangle is not needed)
-__global__ void __launch_bounds__(256) k_to64_shift(int n, const float* __restrict__ G, size_t strideG,
-                                                    double shift, double* __restrict__ A, size_t strideA) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const int b = blockIdx.y;
-    if (i >= (size_t)n * n) return;
-    const int r = (int)(i % n), c = (int)(i / n);
-    A[b * strideA + i] = (double)G[b * strideG + i] + (r == c ? shift : 0.0);
-}
-
-// The blocked L L^T kernels below are templates over the scalar T: double for the real
-// symmetric positive definite normal equations, zd for the complex symmetric ones of the
-// complex-conductivity model (the same formulas without conjugation).
+// L L^T of the complex symmetric normal equations of the complex-conductivity model (plain
+// transposes, no conjugation); the real ones are factored in spd.hip.
 //
 // factor the diagonal block kb in place
 template <class T>
@@ -1181,32 +1170,9 @@ __global__ void __launch_bounds__(256) k_chol_pairs(int nblk, int2* __restrict__
         for (int ib = jb; ib < nblk; ++ib) pairs[i++] = make_int2(ib, jb);
 }
 
-void launch_cholesky(int n, const float* G, size_t strideG, double shift, double* A, size_t strideA,
-                     int batch, int* d_info, int2* d_pairs, hipStream_t st) {
-    dim3 g0((unsigned)(((size_t)n * n + 255) / 256), batch);
-    k_to64_shift<<<g0, 256, 0, st>>>(n, G, strideG, shift, A, strideA);
-    const int nblk = (n + kCB - 1) / kCB;
-    k_chol_pairs<<<(nblk + 255) / 256, 256, 0, st>>>(nblk, d_pairs);
-    for (int kb = 0; kb < nblk; ++kb) {
-        k_potrf_diag<double><<<dim3(1, 1, batch), 256, 0, st>>>(n, A, strideA, kb, d_info);
-        if (kb + 1 < nblk) {
-            k_potrf_panel<double><<<dim3(nblk - kb - 1, 1, batch), 256, 0, st>>>(n, A, strideA, kb);
-            const int p0 = chol_pair_start(nblk, kb), np = chol_pair_start(nblk, kb + 1) - p0;
-            k_potrf_update<double><<<dim3(np, 1, batch), 256, 0, st>>>(n, A, strideA, kb, d_pairs + p0);
-        }
-    }
-    check_launch();
-}
-
 size_t cholesky_pairs(int n) {
     const int nblk = (n + kCB - 1) / kCB;
     return (size_t)nblk * nblk * nblk / 2 + 16;
-}
-
-void launch_potrs(int n, const double* A, size_t strideA, const double* b, size_t strideb, double* y,
-                  size_t stridey, int batch, hipStream_t st) {
-    k_potrs<double><<<batch, kTrsvThreads, 0, st>>>(n, A, strideA, b, strideb, y, stridey);
-    check_launch();
 }
 
 // complex symmetric A = L L^T in place (A: shifted FP64 matrices, both triangles)

@@ -408,7 +408,7 @@ void Model::ensure_gn() {
     work_n.alloc(gemv_n_workspace(m, S.E, frames) / sizeof(double) + 1);
     gram_work.alloc(std::max({gram_workspace_bytes(m, S.E), gram_nt_workspace_bytes(m, S.E, frames),
                               Jb.p ? gram_bf16_workspace_bytes(m, S.E, frames) : (size_t)0}));
-    pairs.alloc(cholesky_pairs(m));
+    spd_work.alloc(spd_factor_work(m, frames));
     info.alloc(1);
 }
 
@@ -447,7 +447,7 @@ void Model::gn_dense(float* d_gamma, const double* d_Umeas, double lambda, int g
             launch_gram(Jm.p + (size_t)f * m * E, 0, m, E, m, G.p + (size_t)f * m * m, gram_work.p, st0);
     const double lam2 = (S.ref * lambda) * (S.ref * lambda);
     MPF_HIP(hipMemsetAsync(info.p, 0, sizeof(int), st0));
-    launch_cholesky(m, G.p, (size_t)m * m, lam2, A64.p, (size_t)m * m, frames, info.p, pairs.p, st0);
+    launch_spd_factor(m, G.p, (size_t)m * m, lam2, A64.p, (size_t)m * m, frames, info.p, spd_work.p, st0);
     normal_solve(Jm.p, (size_t)m * E, A64.p, (size_t)m * m, lam2, frames, gn_refine);
     // delta = J^T y ; gamma += delta   (solver.cpp:222)
     launch_gemv_t(m, E, Jm.p, m, (size_t)m * E, y.p, m, vE.p, E, frames, st0);
@@ -504,7 +504,7 @@ void Model::normal_solve(const float* Jp, size_t strideJ, const double* A, size_
                          int gn_refine) {
     hipStream_t st0 = ctx->stream;
     const int m = S.mrows, E = S.E;
-    launch_potrs(m, A, strideA, rgn.p, m, y.p, m, nb, st0);
+    launch_spd_solve(m, A, strideA, rgn.p, m, y.p, m, nb, spd_work.p, st0);
     // FP64 refinement of (J J^T + lam I) y = r with residuals from the FP32 Jacobian: at
     // most gn_refine passes, fewer once every frame's remaining error, predicted from the
     // last two corrections (|dy_k|^2 / |dy_k-1|, relative to |y|, the refinement converging
@@ -520,7 +520,7 @@ void Model::normal_solve(const float* Jp, size_t strideJ, const double* A, size_
             launch_gemv_t(m, E, Jp, m, strideJ, y.p, m, vE.p, E, nb, st0);
             launch_gemv_n(m, E, Jp, m, strideJ, vE.p, E, lam2, y.p, m, rgn.p, m, res.p, m, nb, work_n.p, st0);
         }
-        launch_potrs(m, A, strideA, res.p, m, dy.p, m, nb, st0);
+        launch_spd_solve(m, A, strideA, res.p, m, dy.p, m, nb, spd_work.p, st0);
         launch_add_to_ratio(m, nb, y.p, dy.p, ratio.p, st0);
         if (k + 1 == gn_refine) break;
         MPF_HIP(hipMemcpyAsync(ratio_h.data(), ratio.p, sizeof(double) * nb, hipMemcpyDeviceToHost, st0));
@@ -554,7 +554,7 @@ void Model::laplacian_cg(const float* K, size_t strideK, const double* A, size_t
     // z = (K^T K + mu I)^-1 v = (v - K^T (K K^T + mu I)^-1 K v) / mu
     auto precond = [&](const double* v, double* z) {
         launch_gemv_n(m, E, K, m, strideK, v, E, 0.0, nullptr, 0, nullptr, 0, cg_t.p, m, nb, work_n.p, st0);
-        launch_potrs(m, A, strideA, cg_t.p, m, cg_s.p, m, nb, st0);
+        launch_spd_solve(m, A, strideA, cg_t.p, m, cg_s.p, m, nb, spd_work.p, st0);
         launch_gemv_t(m, E, K, m, strideK, cg_s.p, m, cg_u.p, E, nb, st0);
         launch_axmy(NE, 1.0 / mu, v, cg_u.p, z, st0);
     };
@@ -707,7 +707,7 @@ void Model::diff_prepare(const float* d_gamma_ref, double lambda, const mpf_solv
         launch_gram(diff_J.p, 0, m, E, m, G.p, gram_work.p, st0);
     diff_lam2 = (S.ref * lambda) * (S.ref * lambda);
     MPF_HIP(hipMemsetAsync(info.p, 0, sizeof(int), st0));
-    launch_cholesky(m, G.p, 0, diff_lam2, diff_A.p, 0, 1, info.p, pairs.p, st0);
+    launch_spd_factor(m, G.p, 0, diff_lam2, diff_A.p, 0, 1, info.p, spd_work.p, st0);
     int hinfo = 0;
     MPF_HIP(hipMemcpyAsync(&hinfo, info.p, sizeof(int), hipMemcpyDeviceToHost, st0));
     MPF_HIP(hipStreamSynchronize(st0));

@@ -69,7 +69,7 @@ struct Model {
     DBuf<double> ratio;                 // per frame: |dy| / |y| of the last refinement pass
     std::vector<double> ratio_h;
     DBuf<char> gram_work;
-    DBuf<int2> pairs;
+    DBuf<double> spd_work;              // factorisation panels, intermediate vectors of the solves
     DBuf<int> info;
 
     Model(mpf_ctx* c, const mpf_model_desc& d);

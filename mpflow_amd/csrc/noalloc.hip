@@ -3,6 +3,7 @@
 // harnesses that forbid hipMalloc).  Its work space lives in a file-scope device array of
 // fixed size; each GPU holds its own copy for the life of the process, and every call on
 // that GPU shares it: calls that overlap on one GPU race.
+#include <algorithm>
 #include <mutex>
 
 #include "dense.h"
@@ -38,7 +39,7 @@ size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 // offsets of the work-space parts for an m x E problem
 struct NaLayout {
-    size_t G, A, y, dy, res, vE, gemv, gram, pairs, info, total;
+    size_t G, A, y, dy, res, vE, gemv, gram, info, total;
 };
 
 NaLayout na_layout(int m, int E) {
@@ -50,9 +51,10 @@ NaLayout na_layout(int m, int E) {
     L.dy = o;    o += align256((size_t)m * sizeof(double));
     L.res = o;   o += align256((size_t)m * sizeof(double));
     L.vE = o;    o += align256((size_t)E * sizeof(double));
-    L.gemv = o;  o += align256(gemv_n_workspace(m, E, 1));
+    // the factorisation's panel and the solves' intermediate vector share this part with the
+    // products' partial sums: none of them is live across another's launches
+    L.gemv = o;  o += align256(std::max(gemv_n_workspace(m, E, 1), spd_factor_work(m, 1) * sizeof(double)));
     L.gram = o;  o += align256(gram_nt_workspace_bytes(m, E, 1, kNaGramSlabs));
-    L.pairs = o; o += align256(cholesky_pairs(m) * sizeof(int2));
     L.info = o;  o += align256(sizeof(int));
     L.total = o;
     return L;
@@ -90,7 +92,6 @@ void normal_solve_noalloc(mpf_ctx* ctx, int rows, int cols, const float* d_J, in
     double* vE = (double*)(base + L.vE);
     double* work = (double*)(base + L.gemv);
     void* gw = base + L.gram;
-    int2* pairs = (int2*)(base + L.pairs);
     int* info = (int*)(base + L.info);
     hipStream_t st = ctx->stream;
     const int m = rows, E = cols;
@@ -98,12 +99,12 @@ void normal_solve_noalloc(mpf_ctx* ctx, int rows, int cols, const float* d_J, in
     launch_gram_nt(d_J, 0, m, E, ldj, G, 0, 1, gw, st, kNaGramSlabs);
     k_na_zero_int<<<1, 64, 0, st>>>(info);
     MPF_HIP(hipGetLastError());
-    launch_cholesky(m, G, 0, shift, A, 0, 1, info, pairs, st);
-    launch_potrs(m, A, 0, d_r, 0, y, 0, 1, st);
+    launch_spd_factor(m, G, 0, shift, A, 0, 1, info, work, st);
+    launch_spd_solve(m, A, 0, d_r, 0, y, 0, 1, work, st);
     for (int k = 0; k < gn_refine; ++k) {
         launch_gemv_t(m, E, d_J, ldj, 0, y, 0, vE, 0, 1, st);
         launch_gemv_n(m, E, d_J, ldj, 0, vE, 0, shift, y, 0, d_r, 0, res, 0, 1, work, st);
-        launch_potrs(m, A, 0, res, 0, dy, 0, 1, st);
+        launch_spd_solve(m, A, 0, res, 0, dy, 0, 1, work, st);
         launch_add_to(m, y, dy, st);
     }
     launch_gemv_t(m, E, d_J, ldj, 0, y, 0, d_delta, 0, 1, st);
