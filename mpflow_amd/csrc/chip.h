@@ -22,10 +22,9 @@ ChipShape chip_shape(int np, long long lanes);
 // gst flags of a lane group
 constexpr int kChipCapped = 1, kChipNan = 2, kChipEmpty = 4;
 
-// pos -> row and row -> pos of the chip order (each tile's rows by aggregate, 64 positions
-// per aggregate, padding rows in the holes); *bad is set when an aggregate has more than 64 rows
-void launch_chip_order(int n, int np, const uint8_t* aggq, uint16_t* rowof, uint16_t* posof, int* bad,
-                       hipStream_t st);
+// pos -> row and row -> pos of the chip order: each tile's rows by their place in the node
+// bisection (null: row order), 64 positions per aggregate
+void launch_chip_order(int np, const uint8_t* tpos, uint16_t* rowof, uint16_t* posof, hipStream_t st);
 // column positions of the ELL in chip order: [width / 8][np] x 8 ids of 16 bits; octs[np / 64]:
 // 8-slot groups in use per 64 positions
 void launch_chip_ids(int np, int width, const int32_t* ids, const uint8_t* gw, const uint16_t* rowof,

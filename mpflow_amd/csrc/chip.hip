@@ -30,41 +30,13 @@ namespace mpf {
 // --------------------------------------------------------------------------------
 // chip order and matrix
 // --------------------------------------------------------------------------------
-__global__ void __launch_bounds__(kTileRows) k_chip_order(int n, int np, const uint8_t* __restrict__ aggq,
+__global__ void __launch_bounds__(kTileRows) k_chip_order(const uint8_t* __restrict__ tpos,
                                                           uint16_t* __restrict__ rowof,
-                                                          uint16_t* __restrict__ posof, int* __restrict__ bad) {
-    const int tile0 = blockIdx.x * kTileRows, t = threadIdx.x, row = tile0 + t;
-    __shared__ int agg[kTileRows];
-    __shared__ int held[kTileRows];
-    const int q = row >= n ? -1 : (aggq ? (int)aggq[row] : t / kAggRows);
-    agg[t] = q;
-    held[t] = -1;
-    rowof[row] = posof[row] = (uint16_t)row;   // every entry is valid also where *bad is set
-    __syncthreads();
-    // real rows: rank within the aggregate in row order
-    int rank = 0;
-    for (int u = 0; u < t; ++u) rank += agg[u] == q ? 1 : 0;
-    const bool fits = q >= 0 && q < kAggPerTile && rank < kAggRows;
-    if (q >= 0 && !fits) atomicOr(bad, 1);
-    if (fits) {
-        held[q * kAggRows + rank] = t;
-        posof[row] = (uint16_t)(tile0 + q * kAggRows + rank);
-        rowof[tile0 + q * kAggRows + rank] = (uint16_t)row;
-    }
-    __syncthreads();
-    // padding rows: the rank-th hole
-    if (q < 0) {
-        int hole = 0;
-        for (int u = 0; u < kTileRows; ++u) {
-            if (held[u] >= 0) continue;
-            if (hole == rank) {
-                posof[row] = (uint16_t)(tile0 + u);
-                rowof[tile0 + u] = (uint16_t)row;
-                break;
-            }
-            ++hole;
-        }
-    }
+                                                          uint16_t* __restrict__ posof) {
+    const int row = blockIdx.x * kTileRows + threadIdx.x;
+    const int pos = tpos ? blockIdx.x * kTileRows + tpos[row] : row;
+    posof[row] = (uint16_t)pos;
+    rowof[pos] = (uint16_t)row;
 }
 
 // one 64-thread block per 64 positions
@@ -693,9 +665,8 @@ ChipShape chip_shape(int np, long long lanes) {
     return c;
 }
 
-void launch_chip_order(int n, int np, const uint8_t* aggq, uint16_t* rowof, uint16_t* posof, int* bad,
-                       hipStream_t st) {
-    k_chip_order<<<np / kTileRows, kTileRows, 0, st>>>(n, np, aggq, rowof, posof, bad);
+void launch_chip_order(int np, const uint8_t* tpos, uint16_t* rowof, uint16_t* posof, hipStream_t st) {
+    k_chip_order<<<np / kTileRows, kTileRows, 0, st>>>(tpos, rowof, posof);
     check_launch();
 }
 

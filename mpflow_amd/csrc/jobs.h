@@ -75,6 +75,11 @@ struct JobDev {
     float* csc;                  // [4 ntiles] Sc^-1/2 (written after each assembly)
     float* cy;                   // [C][4 ntiles][Rp] coarse correction Einv W^T r
     float* cg;                   // [C][4 ntiles][Rp] Sc^-1/2 W^T r of the current iteration
+    // block-diagonal part of the two-level preconditioner (blockjac.hip; null: the diagonal):
+    // M^-1 = D^-1/2 B D^-1/2 + W Einv W^T, B the inverses of the kBlkRows-row diagonal blocks of
+    // the unit-diagonal matrix at sigma = 1
+    const uint8_t* tpos;         // [np] place of each row in its tile
+    const float* bloc;           // [C][np / 32][4][64][4] operand order of the FP32 MFMA
     // on-chip PCG (chip.hip; set by the Krylov driver for jobs that fit): the matrix in chip
     // order, positions of 16 bits
     const uint16_t* crow;        // [np] device row of each position
@@ -121,11 +126,12 @@ constexpr int kSpmvVariants = 3;
 // d_js lists the group's (job, slice) pairs and `nchunk` the largest job's 32-tile
 // chunks: after the SpMV a small launch sums p.q and 1^T p per chunk, and between update
 // and pupdate one launch applies the two-level coarse correction (jobs that have one) and
-// sums r.z and r.r per chunk, so update and pupdate reduce chunk partials only.
+// sums r.z and r.r per chunk, so update and pupdate reduce chunk partials only.  blocks: every
+// job has inverse diagonal blocks.
 void launch_pcg_iter(const JobDev* d_jobs, const int4* d_tiles, int ntiles, int* d_active, int iter,
                      int lg, int wpad, int variant, hipStream_t st, hipEvent_t ev0 = nullptr,
                      hipEvent_t ev1 = nullptr, const int2* d_js = nullptr, int njs = 0, int nchunk = 0,
-                     const int4* d_ftiles = nullptr, int nftiles = 0);
+                     const int4* d_ftiles = nullptr, int nftiles = 0, bool blocks = false);
 // per-tile conductivity scale of the two-level preconditioner (after assembly); d1: the
 // model's per-tile sigma = 1 diagonal sums; work items with slice != 0 are skipped
 void launch_coarse_scale(const JobDev* d_jobs, const int4* d_tiles, int ntiles, const double* d1,

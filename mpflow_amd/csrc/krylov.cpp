@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "blockjac.h"
 #include "model.h"
 
 namespace mpf {
@@ -175,9 +176,6 @@ bool KrylovDriver::ensure_chip() {
     std::sort(jobs_on.begin(), jobs_on.end());
     hipStream_t s0 = ctx->stream;
     try {
-        DBuf<int> bad(1);
-        int hbad = 0;
-        bad.upload(&hbad, 1, s0);
         size_t nval = 0;
         for (int j : jobs_on) {
             const JobDev& J = h[j];
@@ -193,7 +191,7 @@ bool KrylovDriver::ensure_chip() {
                 M.cpos.alloc(J.np);
                 M.cid.alloc((size_t)J.width / 8 * J.np);
                 M.octs.alloc(J.np / 64);
-                launch_chip_order(J.n, J.np, J.aggq, M.crow.p, M.cpos.p, bad.p, s0);
+                launch_chip_order(J.np, J.tpos, M.crow.p, M.cpos.p, s0);
                 launch_chip_ids(J.np, J.width, J.ids, J.gw, M.crow.p, M.cpos.p, M.cid.p, M.octs.p, s0);
             }
             chip_mesh_of[j] = m;
@@ -202,9 +200,6 @@ bool KrylovDriver::ensure_chip() {
             chip_max_np = std::max(chip_max_np, J.np);
         }
         cval.alloc(nval);
-        MPF_HIP(hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, s0));
-        MPF_HIP(hipStreamSynchronize(s0));
-        if (hbad) return false;   // an aggregate of more than 64 rows: streamed
         long long lanes = 0;
         for (int j : jobs_on) lanes += (long long)h[j].C * h[j].R;
         // the longest pairs (low harmonics) first
@@ -338,7 +333,7 @@ void KrylovDriver::launch_group_iter(Group& g, int iter, bool bicg, hipStream_t 
         launch_bicg_iter(jobs.p, g.cur, g.ncur, active.p, iter, g.lg, g.wpad, s, e0, e1);
     else
         launch_pcg_iter(jobs.p, g.cur, g.ncur, active.p, iter, g.lg, g.wpad, g.variant, s, e0, e1, g.js.p, g.njs,
-                        g.nchunk, g.fcur, g.nfcur);
+                        g.nchunk, g.fcur, g.nfcur, g.blocks);
 }
 
 // Time each SpMV candidate that supports the group's width on the live job data (the
@@ -408,6 +403,7 @@ bool KrylovDriver::run(const mpf_solve_opts& o, int rule, double tol, bool use_r
         JobDev& J = h[j];
         J = (*src[origin[j].first])[origin[j].second];
         if (!coarse) J.cinv = nullptr;
+        if (!J.cinv) J.bloc = nullptr;
         J.st = st.p + (size_t)j * kMaxSlices * kStInts;
         J.rule = rule;
         J.tol = tol;
@@ -422,8 +418,20 @@ bool KrylovDriver::run(const mpf_solve_opts& o, int rule, double tol, bool use_r
             J.cval = cval.p + cval_off[j];
         }
     }
+    for (auto& g : groups) {
+        g.blocks = !(chip && g.chip);
+        for (int j : g.jobs) g.blocks = g.blocks && h[j].bloc;
+        if (!g.blocks)
+            for (int j : g.jobs) h[j].bloc = nullptr;
+    }
     jobs.upload(h.data(), h.size(), s0);
     MPF_HIP(hipMemsetAsync(active.p, 0, sizeof(int), s0));
+    // the start: jobs with inverse blocks by their own kernel, the others by k_pcg_init
+    auto start = [&](const int4* lt, int nt, const int2* lj, int nj2) {
+        for (auto& g : groups)
+            if (g.blocks) launch_block_init(jobs.p, g.tiles_o[0].p, g.nall, g.lg, s0);
+        launch_pcg_init(jobs.p, lt, nt, lj, nj2, active.p, s0, coarse ? init_nchunk : 0);
+    };
     const int4* itiles = chip ? stream_tiles.p : init_tiles.p;
     const int2* ijs = chip ? stream_js.p : init_js.p;
     const int nit = chip ? n_stream_tiles : n_init_tiles, nij = chip ? n_stream_js : n_init_js;
@@ -432,12 +440,11 @@ bool KrylovDriver::run(const mpf_solve_opts& o, int rule, double tol, bool use_r
     } else {
         if (chip && !tuned()) {
             // the candidates are timed on initialised pairs, streamed or not
-            launch_pcg_init(jobs.p, init_tiles.p, n_init_tiles, init_js.p, n_init_js, active.p, s0,
-                            coarse ? init_nchunk : 0);
+            start(init_tiles.p, n_init_tiles, init_js.p, n_init_js);
             for (auto& g : groups) tune(g);
             MPF_HIP(hipMemsetAsync(active.p, 0, sizeof(int), s0));
         }
-        if (nij) launch_pcg_init(jobs.p, itiles, nit, ijs, nij, active.p, s0, coarse ? init_nchunk : 0);
+        if (nij) start(itiles, nit, ijs, nij);
     }
     for (auto& g : groups) {
         if (!bicg) tune(g);

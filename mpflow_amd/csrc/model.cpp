@@ -8,6 +8,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "blockjac.h"
 #include "cem.h"
 #include "model.h"
 #include "fem.h"
@@ -45,6 +46,7 @@ Model::Model(mpf_ctx* c, const mpf_model_desc& d) : ctx(c) {
     diag_slot.alloc(np); diag_slot.upload(S.diag_slot.data(), np, st0);
     gw.alloc(np / 16); gw.upload(S.group_width.data(), np / 16, st0);
     aggq.alloc(np); aggq.upload(S.agg_q.data(), np, st0);
+    tpos.alloc(np); tpos.upload(S.tile_pos.data(), np, st0);
     ctb_off.alloc(S.ctb_off.size()); ctb_off.upload(S.ctb_off.data(), S.ctb_off.size(), st0);
     ctb_elem.alloc(S.ctb_elem.size()); ctb_elem.upload(S.ctb_elem.data(), S.ctb_elem.size(), st0);
     ctb_k.alloc(S.ctb_k.size()); ctb_k.upload(S.ctb_k.data(), S.ctb_k.size(), st0);
@@ -163,6 +165,7 @@ Model::Model(mpf_ctx* c, const mpf_model_desc& d) : ctx(c) {
         J.diag_slot = diag_slot.p;
         J.gw = gw.p;
         J.aggq = aggq.p;
+        J.tpos = tpos.p;
         if (nct) {
             J.cinv = cinv.p;
             J.cld = S.coarse_ld;
@@ -244,12 +247,40 @@ void Model::prepare(const mpf_solve_opts& o) {
         // Dirichlet rows, or the contact term of every mode: no constant mode
         if (S.fixed || S.cem_coupled) { J.dc = -1; J.dc_rank1 = 0; }
     }
+    const bool two_level = S.coarse_nt && o.preconditioner == MPF_PRECOND_TWO_LEVEL && o.krylov == MPF_KRYLOV_CG;
+    if (two_level) ensure_blocks();
     upload_jobs();
     launch_assemble(jobs.p, asm_items.p, nasm, st0);
     launch_dinv(jobs.p, tiles.p, ntiles, st0);
     if (S.fixed) launch_fixed_rhs(jobs.p, frames, fixdev(), st0);
-    if (S.coarse_nt && o.preconditioner == MPF_PRECOND_TWO_LEVEL && o.krylov == MPF_KRYLOV_CG)
-        launch_coarse_scale(jobs.p, tiles.p, ntiles, cd1.p, st0);
+    if (two_level) launch_coarse_scale(jobs.p, tiles.p, ntiles, cd1.p, st0);
+}
+
+// The inverse diagonal blocks of a mesh that the streaming PCG solves (the on-chip one keeps
+// the diagonal: its iterations are cheap next to a block product).  Without room for them, or
+// with a block that is not positive definite, the diagonal stays.
+void Model::ensure_blocks() {
+    if (bloc_tried || S.np <= kChipMaxRows) return;
+    bloc_tried = true;
+    hipStream_t st0 = ctx->stream;
+    try {
+        bloc.alloc(block_inverse_floats(S.C, S.np));
+    } catch (const Error& e) {
+        if (e.code != MPF_ENOMEM) throw;
+        return;
+    }
+    DBuf<int> bad(1);
+    int hbad = 0;
+    bad.upload(&hbad, 1, st0);
+    upload_jobs();
+    launch_block_inverse(jobs.p, S.C, S.np, bloc.p, bad.p, st0);
+    MPF_HIP(hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, st0));
+    MPF_HIP(hipStreamSynchronize(st0));
+    if (hbad) {
+        bloc.release();
+        return;
+    }
+    for (auto& J : hjobs) J.bloc = bloc.p;
 }
 
 // FP64 refinement report, voltages and (optionally) the Jacobian after the solves.

@@ -38,10 +38,13 @@ struct Model {
     DBuf<int32_t> cpl_off, cpl_node, cpl_elem, drow_off, drow_node, drow_elem;
     DBuf<double> cpl_k, cpl_m, drow_k, drow_m, fslice, cur;
     DBuf<int32_t> node_of_row;   // [np] device row -> caller's node (identity past the mesh nodes)
-    DBuf<uint8_t> gw, aggq;
+    DBuf<uint8_t> gw, aggq, tpos;
     DBuf<double> ctb_k, ctb_m, F, w_val, colscale;
     DBuf<float> cinv, csc, cy, cg;          // two-level preconditioner (allocated if the mesh has one)
     DBuf<double> cd1;
+    DBuf<float> bloc;                       // inverse diagonal blocks (first two-level solve of a large mesh)
+    bool bloc_tried = false;
+    void ensure_blocks();
     DBuf<float> ek, em;
     DBuf<int32_t> jac_order;     // elements sorted by their first device node (locality)
     // per-frame state

@@ -206,12 +206,13 @@ static void edge_integrals(int kb, const double* sp, double (*m)[3], double* v) 
 // patch of the mesh: most gathers of its SpMV rows stay inside it, consecutive tiles are
 // neighbouring patches (the XCD-striped work lists keep them in one L2).  Each tile is
 // then bisected the same way into leaves of kAggRows nodes (a part holding a whole number
-// of them first): the kAggPerTile aggregates of the two-level preconditioner, quarter[node]
-// = the leaf's index in its tile.  The tile's rows are then sorted by descending degree
+// of them first): the kAggPerTile aggregates of the two-level preconditioner; each of those
+// into leaves of kBlkRows, the blocks of its block-diagonal part.  tpos[node] = the node's
+// index within its tile in that order (aggregate tpos / kAggRows, block tpos / kBlkRows).  The tile's rows are then sorted by descending degree
 // (the aggregates are sets, not row ranges) so the 16-row groups of the SpMV have
 // near-uniform ELL widths.  Returns perm[node] = row.
 static std::vector<int32_t> device_order(int N, const double* xy, int E, int k, const int32_t* el,
-                                         std::vector<uint8_t>& quarter) {
+                                         std::vector<uint8_t>& tpos) {
     std::vector<int32_t> deg(N, 0);
     {
         std::vector<std::vector<int32_t>> nb(N);
@@ -258,11 +259,12 @@ static std::vector<int32_t> device_order(int N, const double* xy, int E, int k, 
     };
     split(0, N, kTileRows);
     auto by_degree = [&](int a, int c) { return deg[a] != deg[c] ? deg[a] > deg[c] : a < c; };
-    quarter.assign(N, 0);
+    tpos.assign(N, 0);
     for (int w = 0; w < N; w += kTileRows) {
         const int e = std::min(N, w + kTileRows);
         split(w, e, kAggRows);
-        for (int i = w; i < e; ++i) quarter[order[i]] = (uint8_t)((i - w) / kAggRows);
+        for (int a = w; a < e; a += kAggRows) split(a, std::min(e, a + kAggRows), kBlkRows);
+        for (int i = w; i < e; ++i) tpos[order[i]] = (uint8_t)(i - w);
         std::sort(order.begin() + w, order.begin() + e, by_degree);
     }
     std::vector<int32_t> perm(N);
@@ -466,16 +468,16 @@ void build_setup(const mpf_model_desc& caller, MeshSetup& s) {
     std::vector<double> nodes_r;
     std::vector<int32_t> el_r, bd_r;
     // aggregate of each caller node within its tile (kept order: consecutive kAggRows runs)
-    std::vector<uint8_t> quarter(caller.n_nodes);
+    std::vector<uint8_t> tpos(caller.n_nodes);
     if (caller.keep_node_order) {
         s.perm.resize(caller.n_nodes);
         for (int n = 0; n < caller.n_nodes; ++n) {
             s.perm[n] = n;
-            quarter[n] = (uint8_t)((n % kTileRows) / kAggRows);
+            tpos[n] = (uint8_t)(n % kTileRows);
         }
     } else {
         s.perm = device_order(caller.n_nodes, caller.nodes, caller.n_elements, caller.nodes_per_element,
-                              caller.elements, quarter);
+                              caller.elements, tpos);
         nodes_r.resize((size_t)2 * caller.n_nodes);
         for (int n = 0; n < caller.n_nodes; ++n) {
             nodes_r[2 * (size_t)s.perm[n]] = caller.nodes[2 * (size_t)n];
@@ -508,11 +510,13 @@ void build_setup(const mpf_model_desc& caller, MeshSetup& s) {
     const int Nu = N + (cem && !coupled ? d.n_ports : 0);
     s.N = Nu; s.E = E; s.k = k;
     s.np = round_up(Nu, kTileRows);
-    // aggregate within the tile of every row: the mesh nodes' from the ordering, the
-    // electrode rows (harmonic-wise electrode model) and padding rows by position
+    // place within the tile of every row (a permutation of the tile): the mesh nodes' from the
+    // ordering, the electrode rows (harmonic-wise electrode model) and padding rows by position
+    s.tile_pos.resize(s.np);
+    for (int r = 0; r < s.np; ++r) s.tile_pos[r] = (uint8_t)(r % kTileRows);
+    for (int n = 0; n < N; ++n) s.tile_pos[s.perm[n]] = tpos[n];
     s.agg_q.resize(s.np);
-    for (int r = 0; r < s.np; ++r) s.agg_q[r] = (uint8_t)((r % kTileRows) / kAggRows);
-    for (int n = 0; n < N; ++n) s.agg_q[s.perm[n]] = quarter[n];
+    for (int r = 0; r < s.np; ++r) s.agg_q[r] = (uint8_t)(s.tile_pos[r] / kAggRows);
     s.P = d.n_ports; s.D = d.n_drive; s.M = d.n_meas; s.R = s.D + s.M;
     MPF_REQUIRE(s.R <= 64, "model: D + M > 64 is not supported");
     // Pi = [I*Dpat | Mpat] (sources.cpp:57-71); columns that are scalar multiples of an

@@ -13,6 +13,7 @@
 // Dot products are accumulated in FP64 per lane, combined across row groups and
 // wavefronts in a fixed order into one partial per tile, and summed per (job, slice)
 // by a one-block reduction in tile order: every scalar is deterministic run to run.
+#include "blockjac.h"
 #include "krylov_dev.h"
 
 namespace mpf {
@@ -72,6 +73,7 @@ __global__ void __launch_bounds__(kEwBlock) k_pcg_init(const JobDev* __restrict_
                                                        const int4* __restrict__ tiles) {
     const int4 t = tiles[blockIdx.x];
     const JobDev& J = jobs[t.x];
+    if (J.bloc) return;   // k_block_init
     const int s = t.y;
     const Ew L = ew_of(J);
     const float* dinv = J.dinv + (size_t)s * J.np;
@@ -765,7 +767,9 @@ __global__ void __launch_bounds__(kUpdBlock, 6) k_pcg_pupdate4(const JobDev* __r
     }
     const size_t base = (size_t)s * J.np * LPR;
     const MPF_GLOBAL float* dinv = gp((const float*)J.dinv) + (size_t)s * J.np;
-    const MPF_GLOBAL float4* Rr = (const MPF_GLOBAL float4*)gp((const float*)J.rv) + base;
+    // z = D^-1 r, or as the block update left it in q
+    const bool blk = J.bloc != nullptr;
+    const MPF_GLOBAL float4* Rr = (const MPF_GLOBAL float4*)gp((const float*)(blk ? J.q : J.rv)) + base;
     // p_k is read from this iteration's buffer, p_{k+1} written to the next one
     const MPF_GLOBAL float4* Pk = (const MPF_GLOBAL float4*)gp((const float*)pbuf(J, k4)) + base;
     MPF_GLOBAL float4* Pn = (MPF_GLOBAL float4*)gp(pbuf(J, (k4 + 1) & (kRing - 1))) + base;
@@ -802,7 +806,7 @@ __global__ void __launch_bounds__(kUpdBlock, 6) k_pcg_pupdate4(const JobDev* __r
                 for (int j = 0; j < 4; ++j) xv[j] = xz[q][j] ? 0.0f : xv[j] + a[q][j] * pv[j];
             }
             X[i] = make_float4(xv[0], xv[1], xv[2], xv[3]);
-            const float d = dinv[row];
+            const float d = blk ? 1.0f : dinv[row];
             const float w = row < J.n ? 1.0f : 0.0f;
             const float4 y4 = sh_y[row_agg(J, row)][c4];
             Pn[i] = make_float4(zero[0] ? 0.0f : d * r4.x + w * y4.x + b[0] * p4.x,
@@ -815,7 +819,7 @@ __global__ void __launch_bounds__(kUpdBlock, 6) k_pcg_pupdate4(const JobDev* __r
     for (int row = t.z * kTileRows + r0; row < (t.z + 1) * kTileRows; row += ROWS) {
         const size_t i = (size_t)row * LPR + c4;
         const float4 r4 = Rr[i], p4 = Pk[i];
-        const float d = dinv[row];
+        const float d = blk ? 1.0f : dinv[row];
         const float w = row < J.n ? 1.0f : 0.0f;
         const float4 y4 = sh_y[row_agg(J, row)][c4];
         Pn[i] = make_float4(zero[0] ? 0.0f : d * r4.x + w * y4.x + b[0] * p4.x,
@@ -1168,7 +1172,7 @@ void launch_pcg_spmv(const JobDev* d_jobs, const int4* d_tiles, int ntiles, int 
 
 void launch_pcg_iter(const JobDev* d_jobs, const int4* d_tiles, int ntiles, int* d_active, int iter,
                      int lg, int wpad, int variant, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1,
-                     const int2* d_js, int njs, int nchunk, const int4* d_ftiles, int nftiles) {
+                     const int2* d_js, int njs, int nchunk, const int4* d_ftiles, int nftiles, bool blocks) {
     if (ev0) MPF_HIP(hipEventRecord(ev0, st));
     if (variant == 2) {
         MPF_REQUIRE(d_ftiles, "pcg iteration: the harmonic-fused SpMV needs a (job, tile) list");
@@ -1181,7 +1185,8 @@ void launch_pcg_iter(const JobDev* d_jobs, const int4* d_tiles, int ntiles, int*
     if (lg == 6) chunks_launch<6>(d_jobs, d_js, njs, nchunk, st);
     else if (lg == 5) chunks_launch<5>(d_jobs, d_js, njs, nchunk, st);
     else chunks_launch<4>(d_jobs, d_js, njs, nchunk, st);
-    if (lg == 6) k_pcg_update4<6><<<ntiles, kUpdBlock, 0, st>>>(d_jobs, d_tiles, iter);
+    if (blocks) launch_block_update(d_jobs, d_tiles, ntiles, iter, lg, st);
+    else if (lg == 6) k_pcg_update4<6><<<ntiles, kUpdBlock, 0, st>>>(d_jobs, d_tiles, iter);
     else if (lg == 5) k_pcg_update4<5><<<ntiles, kUpdBlock, 0, st>>>(d_jobs, d_tiles, iter);
     else k_pcg_update4<4><<<ntiles, kUpdBlock, 0, st>>>(d_jobs, d_tiles, iter);
     // coarse correction where the job has one; chunk sums of r.z and r.r for every job
