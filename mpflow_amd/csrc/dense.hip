@@ -556,13 +556,13 @@ constexpr int kNSlab = 256;
 
 // partial[slab][r] = sum_{c in slab} A[r + c*lda] (sum_r' A[r' + c*lda] x[r']): A (A^T x)
 // in one pass over A (rows <= 1024, rows, lda and strideA multiples of 4).  A block owns
-// the kNSlab columns of its slab, kTnCols at a time: thread t loads rows 4t..4t+3 of each
+// the sw columns of its slab, kTnCols at a time: thread t loads rows 4t..4t+3 of each
 // column (128-bit), the block reduces the column dots in FP64, and the same registers
 // then give the rows' partial sums, so every element of A is read once.
 constexpr int kTnCols = 8;
 __global__ void __launch_bounds__(256) k_gemv_tn_part(int rows, int cols, const float* __restrict__ A, int lda,
                                                       size_t strideA, const double* __restrict__ x,
-                                                      size_t stridex, double* __restrict__ part) {
+                                                      size_t stridex, double* __restrict__ part, int sw) {
     const int slab = blockIdx.x, b = blockIdx.y;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r0 = 4 * threadIdx.x;
@@ -573,7 +573,7 @@ __global__ void __launch_bounds__(256) k_gemv_tn_part(int rows, int cols, const 
         for (int i = 0; i < 4; ++i) xv[i] = x[b * stridex + r0 + i];
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
     __shared__ double red[4][kTnCols];
-    const int c0 = slab * kNSlab, c1 = min(cols, c0 + kNSlab);
+    const int c0 = slab * sw, c1 = min(cols, c0 + sw);
     for (int cb = c0; cb < c1; cb += kTnCols) {
         float4 p[kTnCols];
 #pragma unroll
@@ -615,16 +615,26 @@ __global__ void __launch_bounds__(256) k_gemv_n_part(int rows, int cols, const f
     part[((size_t)b * gridDim.y + slab) * rows + r] = s;
 }
 
-// y = part-sum (+ shift * z) ; out = rhs - y when rhs given
+// y = part-sum (+ shift * z) ; out = rhs - y when rhs given.  A block takes 16 rows, thread group
+// g (of 16) the slabs g, g + 16, ..., then the groups' sums are added in order: the few
+// hundred partials of a single frame are read by 64 workgroups at once.
 __global__ void __launch_bounds__(256) k_gemv_n_reduce(int rows, int nslab, const double* __restrict__ part,
                                                        double shift, const double* __restrict__ z, size_t stridez,
                                                        const double* __restrict__ rhs, size_t striderhs,
                                                        double* __restrict__ out, size_t strideout) {
-    const int r = blockIdx.x * 256 + threadIdx.x;
+    const int o = threadIdx.x & 15, g = threadIdx.x >> 4, r = blockIdx.x * 16 + o;
     const int b = blockIdx.y;
-    if (r >= rows) return;
     double s = 0.0;
-    for (int q = 0; q < nslab; ++q) s += part[((size_t)b * nslab + q) * rows + r];
+    if (r < rows) {
+#pragma unroll 4
+        for (int q = g; q < nslab; q += 16) s += part[((size_t)b * nslab + q) * rows + r];
+    }
+    __shared__ double red[16][17];
+    red[g][o] = s;
+    __syncthreads();
+    if (g != 0 || r >= rows) return;
+#pragma unroll
+    for (int q = 1; q < 16; ++q) s += red[q][o];
     if (z) s += shift * z[b * stridez + r];
     out[b * strideout + r] = rhs ? rhs[b * striderhs + r] - s : s;
 }
@@ -1123,13 +1133,26 @@ bool gemv_tn_applies(int rows, int lda, size_t strideA, const float* A) {
     return rows > 0 && rows <= 1024 && rows % 4 == 0 && lda % 4 == 0 && strideA % 4 == 0 && ((uintptr_t)A & 15) == 0;
 }
 
+// columns per block: kNSlab, fewer where that leaves the chip idle (below 512 blocks; one frame of
+// 9600 columns: 38 blocks and 126 us before, 400 and 17 us now)
+static int gemv_tn_slab(int cols, int batch) {
+    const int want = (512 + batch - 1) / batch;
+    const int sw = round_up((cols + want - 1) / want, kTnCols);
+    return std::min(kNSlab, sw);
+}
+
+size_t gemv_tn_workspace(int rows, int cols, int batch) {
+    const int sw = gemv_tn_slab(cols, batch);
+    return (size_t)batch * ((cols + sw - 1) / sw) * rows * sizeof(double);
+}
+
 void launch_gemv_tn(int rows, int cols, const float* A, int lda, size_t strideA, const double* x,
                     size_t stridex, double shift, const double* rhs, size_t striderhs, double* out,
                     size_t strideout, int batch, double* work, hipStream_t st) {
     MPF_REQUIRE(gemv_tn_applies(rows, lda, strideA, A), "gemv_tn: rows <= 1024, multiples of 4, aligned A");
-    const int nslab = (cols + kNSlab - 1) / kNSlab;
-    k_gemv_tn_part<<<dim3(nslab, batch), 256, 0, st>>>(rows, cols, A, lda, strideA, x, stridex, work);
-    dim3 g2((rows + 255) / 256, batch);
+    const int sw = gemv_tn_slab(cols, batch), nslab = (cols + sw - 1) / sw;
+    k_gemv_tn_part<<<dim3(nslab, batch), 256, 0, st>>>(rows, cols, A, lda, strideA, x, stridex, work, sw);
+    dim3 g2((rows + 15) / 16, batch);
     k_gemv_n_reduce<<<g2, 256, 0, st>>>(rows, nslab, work, shift, x, stridex, rhs, striderhs, out, strideout);
     check_launch();
 }
@@ -1145,7 +1168,7 @@ void launch_gemv_n(int rows, int cols, const float* A, int lda, size_t strideA, 
     const int nslab = (cols + kNSlab - 1) / kNSlab;
     dim3 g1((rows + 255) / 256, nslab, batch);
     k_gemv_n_part<<<g1, 256, 0, st>>>(rows, cols, A, lda, strideA, x, stridex, work);
-    dim3 g2((rows + 255) / 256, batch);
+    dim3 g2((rows + 15) / 16, batch);
     k_gemv_n_reduce<<<g2, 256, 0, st>>>(rows, nslab, work, shift, z, stridez, rhs, striderhs, out, strideout);
     check_launch();
 }

@@ -436,7 +436,7 @@ void Model::ensure_gn() {
     ratio.alloc(frames);
     rgn.alloc((size_t)frames * m);
     vE.alloc((size_t)frames * S.E);
-    work_n.alloc(gemv_n_workspace(m, S.E, frames) / sizeof(double) + 1);
+    work_n.alloc(std::max(gemv_n_workspace(m, S.E, frames), gemv_tn_workspace(m, S.E, frames)) / sizeof(double) + 1);
     gram_work.alloc(std::max({gram_workspace_bytes(m, S.E), gram_nt_workspace_bytes(m, S.E, frames),
                               Jb.p ? gram_bf16_workspace_bytes(m, S.E, frames) : (size_t)0}));
     spd_work.alloc(spd_factor_work(m, frames));

@@ -15,9 +15,11 @@
 // factorisations for one frame (64 dependent columns each), by FP64 MFMA for many.
 //
 // Measured (MI355X, n = 1024, against the 32-column factorisation in three launches per block
-// column and one-workgroup substitutions): factorisation of one matrix 1.5 -> 1.1 ms (the
-// diagonal tiles take 40 us of each step's 65), of 64 matrices 4.4 -> 5.2 ms; one solve
-// 1140 -> 16 us, 64 solves 1610 -> 153 us (3.5 TB/s), 64 against one factor 1120 -> 100 us.
+// column and one-workgroup substitutions): the first diagonal tile 41 -> 24 us, a step's panel
+// 16.8 -> 7.4 us and update 48 -> 28 us (64 matrices 294 -> 138 us), the arrows from this file's
+// first form (whole-tile eliminations, operands loaded one by one), which matched the former
+// factorisation; one solve 1140 -> 16 us, 64 solves 1610 -> 153 us (3.5 TB/s), 64 against one
+// factor 1120 -> 100 us.
 #include "dense.h"
 
 namespace mpf {
@@ -42,16 +44,30 @@ __global__ void __launch_bounds__(256) k_spd_shift(int n, const float* __restric
     A[b * strideA + i] = (double)G[b * strideG + i] + (r == c ? shift : 0.0);
 }
 
-// tile at rows r0, columns c0 of the column-major a (ld entries per column) as t[column][row];
-// entries past n are 0 (1 on the diagonal of a diagonal tile when `unit`)
+// A 64 x 64 tile's elements, 16 per thread: every load is issued (from a clamped place) before the
+// first is used; a guarded load per element would wait for each in turn (16 us per launch
+// instead of 7).
+struct SpdElems {
+    double v[kSB * kSB / 256];
+    // element u of the thread: place (u * 256 + thread) of the tile
+    static __device__ __forceinline__ int place(int u) { return u * 256 + threadIdx.x; }
+    template <class F>
+    __device__ __forceinline__ void load(F&& at) {
+#pragma unroll
+        for (int u = 0; u < kSB * kSB / 256; ++u) v[u] = *at(place(u) % kSB, place(u) / kSB);
+    }
+};
+
+// rows r0.., columns c0.. of the column-major a (ld entries per column, rows and nc columns
+// valid) as t[column][row]; entries past them are 0 (1 on the diagonal when `unit`)
 __device__ __forceinline__ void tile_load(SpdTile& t, const double* a, size_t ld, int n, int r0, int c0, int nc,
                                           bool unit) {
-#pragma unroll 4
-    for (int i = threadIdx.x; i < kSB * kSB; i += 256) {
-        const int r = i % kSB, c = i / kSB;
-        double v = unit && r == c ? 1.0 : 0.0;
-        if (r0 + r < n && c0 + c < nc) v = a[(size_t)(r0 + r) + (size_t)(c0 + c) * ld];
-        t[c][r] = v;
+    SpdElems e;
+    e.load([&](int r, int c) { return a + (size_t)min(r0 + r, n - 1) + (size_t)min(c0 + c, nc - 1) * ld; });
+#pragma unroll
+    for (int u = 0; u < kSB * kSB / 256; ++u) {
+        const int r = e.place(u) % kSB, c = e.place(u) / kSB;
+        t[c][r] = r0 + r < n && c0 + c < nc ? e.v[u] : (unit && r == c ? 1.0 : 0.0);
     }
 }
 
@@ -89,82 +105,119 @@ __device__ __forceinline__ void tile_put(SpdTile& t, const v4d (&acc)[2][2]) {
             for (int v = 0; v < 4; ++v) t[wj + 16 * j + o][wi + 16 * i + 4 * v + q] = acc[i][j][v];
 }
 
-// L L^T of the tile t (its lower triangle, t[column][row]) and X = L^-1 written to rows and
-// columns d0.. of a, mirrored.  A thread owns 4 x 4 entries of the tile and of X, rows ty + 16 u
-// and columns tx + 16 w; step j publishes column j of the tile and row j of X (two buffers,
-// one barrier per step).
-__device__ __forceinline__ void diag_factor(SpdTile& t, double (*colb)[kSB], double (*rowb)[kSB], double* a, int n,
-                                            int d0, int* info) {
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    double A[4][4], X[4][4];
+// LDS accesses of one wavefront made visible to its own lanes
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// L L^T of the 16 x 16 diagonal block of t at o and its inverse into w's, by one wavefront: lane
+// r + 16 g holds columns 4 g .. 4 g + 3 of row r of both; step j passes column j and row j of the
+// inverse through LDS (two buffers, no block barrier)
+__device__ __forceinline__ void factor16(const SpdTile& t, SpdTile& w, int o, double (*colb)[16], double (*rowb)[16],
+                                         int* info) {
+    const int l = threadIdx.x & 63, r = l & 15, g = l >> 4;
+    double A[4], X[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int q = 0; q < 4; ++q) {
+        const int c = 4 * g + q;
+        A[q] = r >= c ? t[o + c][o + r] : t[o + r][o + c];
+        X[q] = r == c ? 1.0 : 0.0;
+    }
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const int r = ty + 16 * u, c = tx + 16 * w;
-            A[u][w] = r >= c ? t[c][r] : t[r][c];
-            X[u][w] = r == c ? 1.0 : 0.0;
+    for (int j = 0; j < 16; ++j) {
+        const int b = j & 1;
+        if (g == j / 4) colb[b][r] = A[j % 4];
+        if (r == j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) rowb[b][4 * g + q] = X[q];
+        wave_sync();
+        double d = colb[b][j];
+        if (!(d > 0.0)) {
+            if (l == 0) atomicExch(info, 1);
+            d = 1e-300;
         }
+        const double rs = rsqrt(d), lr = r > j ? colb[b][r] * rs : 0.0;
 #pragma unroll
-    for (int jb = 0; jb < 4; ++jb) {
-#pragma unroll 1
-        for (int jj = 0; jj < 16; ++jj) {
-            const int j = 16 * jb + jj, buf = j & 1;
-            if (tx == jj)
-#pragma unroll
-                for (int u = 0; u < 4; ++u) colb[buf][ty + 16 * u] = A[u][jb];
-            if (ty == jj)
-#pragma unroll
-                for (int w = 0; w < 4; ++w) rowb[buf][tx + 16 * w] = X[jb][w];
-            __syncthreads();
-            double d = colb[buf][j];
-            if (!(d > 0.0)) {
-                if (threadIdx.x == 0) atomicExch(info, 1);
-                d = 1e-300;
-            }
-            const double rs = rsqrt(d);
-            double lr[4], lc[4], xr[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int r = ty + 16 * u;
-                lr[u] = r > j ? colb[buf][r] * rs : 0.0;
-                const int c = tx + 16 * u;
-                lc[u] = c > j ? colb[buf][c] * rs : 0.0;
-                xr[u] = rowb[buf][c] * rs;
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    A[u][w] -= lr[u] * lc[w];
-                    X[u][w] = ty + 16 * u == j ? xr[w] : X[u][w] - lr[u] * xr[w];
-                }
+        for (int q = 0; q < 4; ++q) {
+            const double x = rowb[b][4 * g + q] * rs;
+            A[q] -= lr * (colb[b][4 * g + q] * rs);
+            X[q] = r == j ? x : X[q] - lr * x;
         }
     }
-    // X through LDS (t[column][row]) for contiguous writes of both triangles
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[o + 4 * g + q][o + r] = 4 * g + q <= r ? X[q] : 0.0;
+}
+
+// one wavefront's 16 x 16 product over 16 steps: a(k, row), b(k, column)
+template <class FA, class FB>
+__device__ __forceinline__ v4d product16(FA&& a, FB&& b) {
+    const int l = threadIdx.x & 63, o = l & 15, q = l >> 4;
+    v4d acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 16; k += 4) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a(k + q, o), b(k + q, o), acc, 0, 0, 0);
+    return acc;
+}
+
+// L L^T of the tile t (its lower triangle, t[column][row]) and X = L^-1 (w, the same layout)
+// written to rows and columns d0.. of a, mirrored: the elimination of the whole matrix again
+// on 16 x 16 blocks, a wavefront per block product.  A 64-step elimination by all threads with
+// a barrier per step made the launch of one tile 41 us against this one's 24.
+__device__ __forceinline__ void diag_factor(SpdTile& t, SpdTile& w, double (*colb)[16], double (*rowb)[16], double* a,
+                                            int n, int d0, int* info) {
+    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, lo = l & 15, lq = l >> 4;
+    for (int i = threadIdx.x; i < kSB * kSB; i += 256) w[i / kSB][i % kSB] = 0.0;
     __syncthreads();
+#pragma unroll 1
+    for (int jb = 0; jb < 4; ++jb) {
+        const int o = 16 * jb;
+        if (wave == 0) factor16(t, w, o, colb, rowb, info);
+        __syncthreads();
+        // the panel L_i = A_io X_o^T (i > jb) and the finished rows X_oj = X_o W_oj (j < jb)
+        if (wave < 3) {
+            const int i = wave < jb ? wave : wave + 1;
+            v4d p;
+            if (i > jb)
+                p = product16([&](int k, int r) { return t[o + k][16 * i + r]; },
+                              [&](int k, int c) { return w[o + k][o + c]; });
+            else
+                p = product16([&](int k, int r) { return w[o + k][o + r]; },
+                              [&](int k, int c) { return w[16 * i + c][o + k]; });
+            wave_sync();
+            SpdTile& out = i > jb ? t : w;
+            const int c0 = i > jb ? o : 16 * i, r0 = i > jb ? 16 * i : o;
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const int r = ty + 16 * u, c = tx + 16 * w;
-            if (r >= c) { t[c][r] = X[u][w]; t[r][c] = X[u][w]; }
+            for (int v = 0; v < 4; ++v) out[c0 + lo][r0 + 4 * v + lq] = p[v];
         }
-    __syncthreads();
+        __syncthreads();
+        // blocks (i, j <= i), i > jb: A_ij -= L_i L_j^T (j > jb), W_ij -= L_i X_oj (j <= jb)
+        int task = 0;
+        for (int i = jb + 1; i < 4; ++i)
+            for (int j = 0; j <= i; ++j, ++task) {
+                if ((task & 3) != wave) continue;
+                SpdTile& out = j > jb ? t : w;
+                const v4d p = product16([&](int k, int r) { return t[o + k][16 * i + r]; },
+                                        [&](int k, int c) { return j > jb ? t[o + k][16 * j + c] : w[16 * j + c][o + k]; });
+#pragma unroll
+                for (int v = 0; v < 4; ++v) out[16 * j + lo][16 * i + 4 * v + lq] -= p[v];
+            }
+        __syncthreads();
+    }
     for (int i = threadIdx.x; i < kSB * kSB; i += 256) {
         const int r = i % kSB, c = i / kSB;
-        if (d0 + r < n && d0 + c < n) a[(size_t)(d0 + r) + (size_t)(d0 + c) * n] = t[c][r];
+        if (d0 + r < n && d0 + c < n) a[(size_t)(d0 + r) + (size_t)(d0 + c) * n] = r >= c ? w[c][r] : w[r][c];
     }
 }
 
 __global__ void __launch_bounds__(256, 2) k_spd_first(int n, double* __restrict__ A, size_t strideA,
                                                    int* __restrict__ info) {
-    __shared__ SpdTile t;
-    __shared__ double colb[2][kSB], rowb[2][kSB];
+    __shared__ SpdTile t, w;
+    __shared__ double colb[2][16], rowb[2][16];
     double* a = A + blockIdx.y * strideA;
     tile_load(t, a, n, n, 0, 0, n, true);
     __syncthreads();
-    diag_factor(t, colb, rowb, a, n, 0, info);
+    diag_factor(t, w, colb, rowb, a, n, 0, info);
 }
 
 // blocks b < k: X_kb = X_kk W_kb (lower tile and its mirror); blocks b >= k: the panel
@@ -178,26 +231,33 @@ __global__ void __launch_bounds__(256, 2) k_spd_panel(int n, double* __restrict_
     v4d acc[2][2];
     tile_zero(acc);
     // X_kk as [column][row], lower triangle (the upper one holds the mirror)
-    for (int i = threadIdx.x; i < kSB * kSB; i += 256) {
-        const int r = i % kSB, c = i / kSB;
-        double v = r == c ? 1.0 : 0.0;
-        if (d0 + r < n && d0 + c < n) v = r >= c ? a[(size_t)(d0 + r) + (size_t)(d0 + c) * n] : 0.0;
-        tb[c][r] = v;
+    {
+        SpdElems e;
+        e.load([&](int r, int c) { return a + (size_t)min(d0 + r, n - 1) + (size_t)min(d0 + c, n - 1) * n; });
+#pragma unroll
+        for (int u = 0; u < kSB * kSB / 256; ++u) {
+            const int r = e.place(u) % kSB, c = e.place(u) / kSB;
+            tb[c][r] = d0 + r < n && d0 + c < n ? (r >= c ? e.v[u] : 0.0) : (r == c ? 1.0 : 0.0);
+        }
     }
     if (b < k) {
         // out[r][c] = sum_t X_kk[r][t] W_kb[t][c]: operand a[t][r] = tb, b[t][c] transposed
         const int c0 = b * kSB;
-        for (int i = threadIdx.x; i < kSB * kSB; i += 256) {
-            const int t = i % kSB, c = i / kSB;
-            ta[t][c] = d0 + t < n ? a[(size_t)(d0 + t) + (size_t)(c0 + c) * n] : 0.0;
+        SpdElems e;
+        e.load([&](int t, int c) { return a + (size_t)min(d0 + t, n - 1) + (size_t)(c0 + c) * n; });
+#pragma unroll
+        for (int u = 0; u < kSB * kSB / 256; ++u) {
+            const int t = e.place(u) % kSB, c = e.place(u) / kSB;
+            ta[t][c] = d0 + t < n ? e.v[u] : 0.0;
         }
         __syncthreads();
         tile_product(tb, ta, acc);
         __syncthreads();
         tile_put(ta, acc);
         __syncthreads();
-        for (int i = threadIdx.x; i < kSB * kSB; i += 256) {
-            const int r = i % kSB, c = i / kSB;
+#pragma unroll
+        for (int i0 = 0; i0 < kSB * kSB; i0 += 256) {
+            const int i = i0 + threadIdx.x, r = i % kSB, c = i / kSB;
             if (d0 + r < n) a[(size_t)(d0 + r) + (size_t)(c0 + c) * n] = ta[c][r];
             if (d0 + c < n) a[(size_t)(c0 + r) + (size_t)(d0 + c) * n] = ta[r][c];
         }
@@ -210,8 +270,9 @@ __global__ void __launch_bounds__(256, 2) k_spd_panel(int n, double* __restrict_
         __syncthreads();
         tile_put(ta, acc);
         __syncthreads();
-        for (int i = threadIdx.x; i < kSB * kSB; i += 256) {
-            const int r = i % kSB, c = i / kSB;
+#pragma unroll
+        for (int i0 = 0; i0 < kSB * kSB; i0 += 256) {
+            const int i = i0 + threadIdx.x, r = i % kSB, c = i / kSB;
             if (r0 + r < n) p[(size_t)(r0 + r) + (size_t)c * n] = ta[c][r];
         }
     }
@@ -223,7 +284,7 @@ __global__ void __launch_bounds__(256, 2) k_spd_update(int n, double* __restrict
                                                     const double* __restrict__ P, size_t strideP, int k,
                                                     int* __restrict__ info) {
     __shared__ SpdTile ta, tb;
-    __shared__ double colb[2][kSB], rowb[2][kSB];
+    __shared__ double colb[2][16], rowb[2][16];
     double* a = A + blockIdx.y * strideA;
     const double* p = P + blockIdx.y * strideP;
     // row k + 1 has k + 2 tiles, its last one (the diagonal) taken by block 0
@@ -247,11 +308,12 @@ __global__ void __launch_bounds__(256, 2) k_spd_update(int n, double* __restrict
     } else {
         // X_k,j as [t][column]: row block k of X from its mirror; the diagonal tile's mirror is
         // its upper triangle
-        for (int e = threadIdx.x; e < kSB * kSB; e += 256) {
-            const int c = e % kSB, t = e / kSB;
-            double v = 0.0;
-            if (d0 + t < n && (j < k || c <= t)) v = a[(size_t)(c0 + c) + (size_t)(d0 + t) * n];
-            tb[t][c] = v;
+        SpdElems e;
+        e.load([&](int c, int t) { return a + (size_t)(c0 + c) + (size_t)min(d0 + t, n - 1) * n; });
+#pragma unroll
+        for (int u = 0; u < kSB * kSB / 256; ++u) {
+            const int c = e.place(u) % kSB, t = e.place(u) / kSB;
+            tb[t][c] = d0 + t < n && (j < k || c <= t) ? e.v[u] : 0.0;
         }
     }
     __syncthreads();
@@ -260,25 +322,24 @@ __global__ void __launch_bounds__(256, 2) k_spd_update(int n, double* __restrict
     __syncthreads();
     tile_put(ta, acc);
     __syncthreads();
+    SpdElems e;
+    if (j != k) e.load([&](int r, int c) { return a + (size_t)min(r0 + r, n - 1) + (size_t)min(c0 + c, n - 1) * n; });
     if (i == k + 1 && j == k + 1) {
         // the next diagonal tile: updated in LDS, factored here
-        for (int e = threadIdx.x; e < kSB * kSB; e += 256) {
-            const int r = e % kSB, c = e / kSB;
-            double v = r == c ? 1.0 : 0.0;
-            if (r0 + r < n && c0 + c < n) v = a[(size_t)(r0 + r) + (size_t)(c0 + c) * n] - ta[c][r];
-            ta[c][r] = v;
+#pragma unroll
+        for (int u = 0; u < kSB * kSB / 256; ++u) {
+            const int r = e.place(u) % kSB, c = e.place(u) / kSB;
+            ta[c][r] = r0 + r < n && c0 + c < n ? e.v[u] - ta[c][r] : (r == c ? 1.0 : 0.0);
         }
         __syncthreads();
-        diag_factor(ta, colb, rowb, a, n, r0, info);
+        diag_factor(ta, tb, colb, rowb, a, n, r0, info);
         return;
     }
-#pragma unroll 4
-    for (int e = threadIdx.x; e < kSB * kSB; e += 256) {
-        const int r = e % kSB, c = e / kSB;
-        if (r0 + r < n && c0 + c < n) {
-            double* o = a + (size_t)(r0 + r) + (size_t)(c0 + c) * n;
-            *o = (j == k ? 0.0 : *o) - ta[c][r];
-        }
+#pragma unroll
+    for (int u = 0; u < kSB * kSB / 256; ++u) {
+        const int r = e.place(u) % kSB, c = e.place(u) / kSB;
+        if (r0 + r < n && c0 + c < n)
+            a[(size_t)(r0 + r) + (size_t)(c0 + c) * n] = (j == k ? 0.0 : e.v[u]) - ta[c][r];
     }
 }
 
