@@ -19,6 +19,8 @@
 
 namespace mpf {
 
+static constexpr int kXcds = 8;
+
 struct ComplexModel::Impl {
     mpf_ctx* ctx = nullptr;
     MeshSetup S;
@@ -41,8 +43,22 @@ struct ComplexModel::Impl {
     DBuf<zd> U64, G, y, rgn, vE;
     DBuf<int2> pairs;
     DBuf<int> info;
+    // on-chip solves (chip_complex.hip)
+    bool chip_tried = false, chip_ok = false;
+    ChipShape shape;
+    DBuf<uint8_t> gw, tpos, octs;
+    DBuf<uint16_t> crow, cpos;
+    DBuf<uint4> cid;
+    DBuf<float4> cval;
+    DBuf<int4> chip_items;
+    DBuf<int2> gst[2];               // (steps, flags) of every lane group, before and after a phase
+    int2* h_gst = nullptr;
+
+    bool ensure_chip();
+    void run_chip();
 
     ~Impl() {
+        if (h_gst) (void)hipHostFree(h_gst);
         if (h_live) (void)hipHostFree(h_live);
         if (h_st) (void)hipHostFree(h_st);
     }
@@ -60,6 +76,88 @@ struct ComplexModel::Impl {
         info.alloc(1);
     }
 };
+
+// Tables of the on-chip solver, once per model; false where the mesh does not fit or there is no
+// room for them: the solves are streamed then
+bool ComplexModel::Impl::ensure_chip() {
+    if (chip_tried) return chip_ok;
+    chip_tried = true;
+    const int np = S.np, W = S.wpad;
+    if (np > kCChipMaxRows || W > kChipMaxWidth) return false;
+    hipStream_t st0 = ctx->stream;
+    shape = c_chip_shape(np, (long long)frames * S.C * S.Ru);
+    const int groups = Rq / shape.G, total = njs * groups;
+    try {
+        gw.alloc(S.group_width.size()); gw.upload(S.group_width.data(), S.group_width.size(), st0);
+        tpos.alloc(np); tpos.upload(S.tile_pos.data(), np, st0);
+        crow.alloc(np);
+        cpos.alloc(np);
+        octs.alloc(np / 64);
+        cid.alloc((size_t)W / 8 * np);
+        const size_t nval = (size_t)S.C * (W / 2) * np;
+        cval.alloc(nval * frames);
+        // the longest pairs (low harmonics) first; the groups of a pair on one XCD (block b runs on
+        // XCD b % 8), which then reads the pair's matrix into its L2 once
+        std::vector<int4> on[kXcds], items;
+        int pair = 0;
+        for (int k = 0; k < S.C; ++k)
+            for (int f = 0; f < frames; ++f, ++pair)
+                for (int g = 0; g < groups; ++g)
+                    on[pair % kXcds].push_back(make_int4(f, k, g, (f * S.C + k) * groups));
+        for (size_t i = 0; i < on[0].size(); ++i)        // the longest list
+            for (const auto& x : on)
+                if (i < x.size()) items.push_back(x[i]);
+        MPF_REQUIRE((int)items.size() == total, "complex conductivity: on-chip work list incomplete");
+        chip_items.alloc(total); chip_items.upload(items.data(), total, st0);
+        for (auto& g : gst) {
+            g.alloc(total);
+            MPF_HIP(hipMemsetAsync(g.p, 0, g.bytes(), st0));
+        }
+        MPF_HIP(hipHostMalloc((void**)&h_gst, sizeof(int2) * total, hipHostMallocDefault));
+        launch_chip_order(np, tpos.p, crow.p, cpos.p, st0);
+        launch_chip_ids(np, W, ids.p, gw.p, crow.p, cpos.p, cid.p, octs.p, st0);
+        MPF_HIP(hipStreamSynchronize(st0));
+        for (int f = 0; f < frames; ++f) {
+            CJob& J = hjobs[f];
+            J.crow = crow.p; J.cid = cid.p; J.cocts = octs.p;
+            J.cval = cval.p + nval * f;
+        }
+    } catch (const Error& e) {
+        if (e.code != MPF_ENOMEM) throw;
+        cval.release();
+        return false;
+    }
+    return chip_ok = true;
+}
+
+// One solve: phase 0, then phase 1 until the lane groups of every pair have taken the same number
+// of steps, as KrylovDriver::run_chip.  Step counts and flags go to h_st.
+void ComplexModel::Impl::run_chip() {
+    hipStream_t st0 = ctx->stream;
+    const int groups = Rq / shape.G, total = njs * groups;
+    launch_c_chip_pack(jobs.p, js.p, njs, S.np, st0);
+    launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, gst[1].p, gst[0].p, 0, st0);
+    int in = 0;
+    for (bool open = true; open;) {
+        launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, gst[in].p, gst[in ^ 1].p, 1, st0);
+        in ^= 1;
+        MPF_HIP(hipMemcpyAsync(h_gst, gst[in].p, sizeof(int2) * total, hipMemcpyDeviceToHost, st0));
+        MPF_HIP(hipStreamSynchronize(st0));
+        open = false;
+        for (int i = 0; i < njs; ++i) {
+            const int2* g = h_gst + (size_t)i * groups;
+            int steps = 0, flags = 0;
+            for (int k = 0; k < groups; ++k) {
+                steps = std::max(steps, g[k].x);
+                flags |= g[k].y & (kChipCapped | kChipNan);
+            }
+            for (int k = 0; k < groups; ++k)
+                if (!g[k].y && g[k].x != steps) open = true;
+            int* sp = h_st + ((size_t)(i / S.C) * kMaxSlices + i % S.C) * 4;
+            sp[0] = 0; sp[1] = steps; sp[2] = flags ? 1 : 0;
+        }
+    }
+}
 
 ComplexModel::ComplexModel(mpf_ctx* c, const mpf_model_desc& d) : impl(new Impl) {
     Impl& M = *impl;
@@ -173,6 +271,8 @@ int ComplexModel::forward(const mpf_solve_opts& o, const float2* d_gamma, float2
     MPF_REQUIRE(o.stop_rule == MPF_STOP_REFERENCE || o.stop_rule == MPF_STOP_TOLERANCE, "solve: unknown stop rule");
     MPF_HIP(hipMemcpyAsync(M.gamma.p, d_gamma, sizeof(float2) * (size_t)S.E * M.frames, hipMemcpyDeviceToDevice,
                            st0));
+    // small meshes run on chip; profiled contexts stream, as the real model's do
+    const bool chip = !M.ctx->prof && M.ensure_chip();
     for (auto& J : M.hjobs) {
         J.herm = o.complex_hermitian ? 1 : 0;
         J.rule = o.stop_rule;
@@ -182,21 +282,25 @@ int ComplexModel::forward(const mpf_solve_opts& o, const float2* d_gamma, float2
     M.jobs.upload(M.hjobs.data(), M.frames, st0);
     launch_c_assemble(M.jobs.p, M.asm_items.p, M.nasm, st0);
     launch_c_dinv(M.jobs.p, M.tiles.p, M.ntiles, st0);
-    launch_c_init(M.jobs.p, M.tiles.p, M.ntiles, M.js.p, M.njs, st0);
-    *M.h_live = M.njs;
-    MPF_HIP(hipMemcpyAsync(M.live.p, M.h_live, sizeof(int), hipMemcpyHostToDevice, st0));
-    const int every = o.check_every > 0 ? o.check_every : 16;
-    const int maxit = M.hjobs[0].maxit;
-    int it = 0;
-    while (true) {
-        for (int i = 0; i < every; ++i) launch_c_iter(M.jobs.p, M.tiles.p, M.ntiles, M.js.p, M.njs, M.live.p, st0);
-        it += every;
-        MPF_HIP(hipMemcpyAsync(M.h_live, M.live.p, sizeof(int), hipMemcpyDeviceToHost, st0));
+    if (chip) {
+        M.run_chip();
+    } else {
+        launch_c_init(M.jobs.p, M.tiles.p, M.ntiles, M.js.p, M.njs, st0);
+        *M.h_live = M.njs;
+        MPF_HIP(hipMemcpyAsync(M.live.p, M.h_live, sizeof(int), hipMemcpyHostToDevice, st0));
+        const int every = o.check_every > 0 ? o.check_every : 16;
+        const int maxit = M.hjobs[0].maxit;
+        int it = 0;
+        while (true) {
+            for (int i = 0; i < every; ++i) launch_c_iter(M.jobs.p, M.tiles.p, M.ntiles, M.js.p, M.njs, M.live.p, st0);
+            it += every;
+            MPF_HIP(hipMemcpyAsync(M.h_live, M.live.p, sizeof(int), hipMemcpyDeviceToHost, st0));
+            MPF_HIP(hipStreamSynchronize(st0));
+            if (*M.h_live <= 0 || it >= maxit + every) break;
+        }
+        MPF_HIP(hipMemcpyAsync(M.h_st, M.st.p, M.st.bytes(), hipMemcpyDeviceToHost, st0));
         MPF_HIP(hipStreamSynchronize(st0));
-        if (*M.h_live <= 0 || it >= maxit + every) break;
     }
-    MPF_HIP(hipMemcpyAsync(M.h_st, M.st.p, M.st.bytes(), hipMemcpyDeviceToHost, st0));
-    MPF_HIP(hipStreamSynchronize(st0));
     bool capped = false;
     for (int f = 0; f < M.frames; ++f)
         for (int k = 0; k < S.C; ++k) {

@@ -5,6 +5,7 @@
 
 #include <memory>
 
+#include "chip.h"
 #include "cplx.h"
 #include "dense.h"
 
@@ -39,6 +40,9 @@ struct CJob {
     int* st;                     // [C][4]: live, steps, capped, -
     const float2* gamma;         // [E]
     const int32_t* ctb_off; const int32_t* ctb_elem; const double* ctb_k; const double* ctb_m;
+    // on-chip solves (chip_complex.hip): chip order, 16-bit column positions, 8-slot groups in
+    // use per 64 positions (as jobs.h) and the values S + alpha_c R, [C][width / 8][4][np]
+    const uint16_t* crow; const uint4* cid; const uint8_t* cocts; float4* cval;
 };
 
 struct CMeasDev {
@@ -62,6 +66,16 @@ void launch_c_init(const CJob* d_jobs, const int4* d_tiles, int ntiles, const in
 // one CG iteration over the listed tiles of live (frame, slice) pairs
 void launch_c_iter(const CJob* d_jobs, const int4* d_tiles, int ntiles, const int2* d_js, int njs, int* d_live,
                    hipStream_t st);
+// whole solves on chip: the meshes whose p and inverse diagonal fit one CU's LDS
+constexpr int kCChipMaxRows = 8192;
+// G complex lanes per workgroup, K rows per thread, for np padded rows when a solve has `lanes`
+// (frame, harmonic, column) triples
+ChipShape c_chip_shape(int np, long long lanes);
+void launch_c_chip_pack(const CJob* d_jobs, const int2* d_js, int njs, int np, hipStream_t st);
+// one phase over `n` items (frame, slice, lane group, index of the pair's first group state), as
+// launch_chip
+void launch_c_chip(const CJob* d_jobs, const int4* d_items, int n, const ChipShape& c, int width, const int2* gin,
+                   int2* gout, int phase, hipStream_t st);
 void launch_c_voltages(const CJob* d_jobs, int njobs, const CMeasDev& md, float2* U32, zd* U64, hipStream_t st);
 void launch_c_jacobian(const CJob* d_jobs, int njobs, const CJacDev& jd, float2* J, hipStream_t st);
 // G_b = J_b J_b^T + shift I (complex symmetric, FP64 sums of the FP32 J, both triangles);

@@ -1,0 +1,67 @@
+"""The on-chip complex conjugate gradients (whole solves in one workgroup per lane group) against
+the streamed iteration of the same solve -- a profiled context streams every mesh -- at the edges
+of its shapes: one row per thread, a partial last tile, both lane-group sizes, rows wider than
+8 entries, the largest mesh it takes and the first one it does not."""
+import numpy as np
+import pytest
+
+from tests.problems import make_problem
+
+pytestmark = pytest.mark.gpu
+
+# rings, electrodes, harmonics, P2, frames
+SHAPES = [
+    (5, 8, 1, False, 1),        # 91 nodes: one tile, 256 threads
+    (16, 16, 2, False, 1),      # 817 nodes: one row per thread
+    (18, 20, 3, False, 1),      # 1027 nodes: one row past 1024, 12 empty lanes
+    (14, 16, 2, True, 1),       # P2: rows of 9 and 19 entries
+    (20, 16, 3, False, 8),      # two lanes, 1261 nodes
+    (36, 16, 1, False, 20),     # two lanes, 3997 nodes
+    (51, 16, 1, False, 1),      # 7957 nodes: the largest
+    (52, 16, 1, False, 1),      # 8269 nodes: streamed
+]
+
+
+def _solve(eit, g, ctx, streamed, **kw):
+    from mpflow_amd import capi
+    from mpflow_amd.eit import SolveOptions
+    capi.check(capi.lib().mpf_ctx_profile(ctx.h, int(streamed)))
+    try:
+        eit.solve(g, SolveOptions(**kw))
+    finally:
+        capi.check(capi.lib().mpf_ctx_profile(ctx.h, 0))
+    return eit.voltages(eit.result64).cpu().numpy().copy(), eit.last_stats
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "-".join(map(str, s)))
+def test_on_chip_complex_matches_streamed(gpu_ctx, shape):
+    import torch
+    from mpflow_amd import capi
+    from mpflow_amd.eit import EIT
+    rings, L, C, p2, frames = shape
+    p = make_problem(rings, L, 1.6 / L, C=C, height=1.0 if C == 1 else 0.4, port_height=1.0 if C == 1 else 0.1, p2=p2)
+    eit = EIT(p["nodes"], p["elements"], p["boundary"], p["ports"], p["drive"], p["meas"], p["current"], 1.0,
+              C, p["height"], p["port_height"], frames=frames, ctx=gpu_ctx, complex_gamma=True)
+    rng = np.random.default_rng(7)
+    n = (frames, p["elements"].shape[0])
+    g = torch.tensor(rng.uniform(0.5, 2.0, n) + 0.3j * rng.uniform(-1.0, 1.0, n), dtype=torch.complex64)
+    for herm in (0, 1):
+        print("case: on-chip complex %s hermitian %d" % (shape, herm), flush=True)
+        # the iteration cap: every pair ends there and says so.  Unconverged voltages are not
+        # compared: on the dcFree harmonic the constant mode grows back from rounding after
+        # four or five steps, in any summation order
+        kw = dict(stop_rule=capi.MPF_STOP_TOLERANCE, tol=1e-12, max_iter=8, complex_hermitian=herm)
+        for streamed in (False, True):
+            _, st = _solve(eit, g, gpu_ctx, streamed, **kw)
+            assert st.max_steps == 8 and st.steps == 8 * C * frames and st.not_converged == C * frames
+    # both stop rules to convergence: tol = 1e-6 leaves the FP32 iteration's own error, as the
+    # oracle comparison of the same solve allows (2e-5)
+    for kw in (dict(stop_rule=capi.MPF_STOP_TOLERANCE, tol=1e-6, max_iter=4000), dict(max_iter=4000)):
+        print("case: on-chip complex %s %s" % (shape, kw), flush=True)
+        a, sa = _solve(eit, g, gpu_ctx, False, **kw)
+        b, sb = _solve(eit, g, gpu_ctx, True, **kw)
+        err = np.max(np.abs(a - b)) / np.max(np.abs(b))
+        print("steps %d / %d, difference %.2e" % (sa.steps, sb.steps, err))
+        assert sa.not_converged == sb.not_converged
+        assert err < 4e-5
+        assert abs(sa.steps - sb.steps) <= 0.1 * sb.steps + 4
