@@ -29,13 +29,16 @@ void launch_chip_order(int np, const uint8_t* tpos, uint16_t* rowof, uint16_t* p
 // 8-slot groups in use per 64 positions
 void launch_chip_ids(int np, int width, const int32_t* ids, const uint8_t* gw, const uint16_t* rowof,
                      const uint16_t* posof, uint4* cid, uint8_t* octs, hipStream_t st);
-// values S + alpha_c R of every (job, slice) pair of the list: J.cval [C][width / 8][2][np] float4
-void launch_chip_pack(const JobDev* d_jobs, const int2* d_js, int njs, int max_np, hipStream_t st);
+// progress[0, nprogress) = 0, and the values S + alpha_c R of every (job, slice) pair of the
+// list: J.cval [C][width / 8][2][np] float4
+void launch_chip_pack(const JobDev* d_jobs, const int2* d_js, int njs, int max_np, int* progress, int nprogress,
+                      hipStream_t st);
 // one phase over `n` items (job, slice, lane group, index of the pair's first group state):
-// phase 0 runs every lane group from its start to its own stop test; phase 1 takes the
-// groups behind their pair's largest step count (gin) on to it.  gout receives every group's
-// (steps, flags).
+// phase 0 runs every lane group from its start to its own stop test -- under the reference rule
+// to the step its pair's deciding group stops at, which that group publishes in progress (zeroed
+// by launch_chip_pack; at the pair's first index) -- and phase 1 takes the groups behind their
+// pair's largest step count (gin) on to it.  gout receives every group's (steps, flags).
 void launch_chip(const JobDev* d_jobs, const int4* d_items, int n, const ChipShape& c, const int2* gin, int2* gout,
-                 int phase, hipStream_t st);
+                 int* progress, int phase, hipStream_t st);
 
 }  // namespace mpf

@@ -13,9 +13,10 @@
 // first coarse entries are loaded before the barrier that the sums wait for, and 512 threads
 // with 256 VGPRs beat 1024 with 128 where there are lanes enough for every CU.
 //
-// Measured (MI355X, whole calls): one 2D forward solve of 817 nodes, 168 steps, 4.60 -> 1.05
-// ms; 64 frames x 5 harmonics of 4921 nodes to 1e-6 18.1 -> 5.5 ms (1024 threads 7.2 ms); a
-// caller's 4921-row matrix with 32 columns 2.02 -> 0.88 ms.
+// Measured (MI355X, whole calls): one 2D forward solve of 817 nodes, 168 steps, 4.60 -> 0.58
+// ms (1.02 ms with the deciding group of the reference rule run before the others); 64 frames x 5
+// harmonics of 4921 nodes to 1e-6 18.1 -> 5.5 ms (1024 threads 7.2 ms); a caller's 4921-row
+// matrix with 32 columns 2.02 -> 0.63 ms.
 //
 // The recurrences, the FP64 scalars, the stop rules and the breakdown rules are those of the
 // streaming kernels (sparse.hip); sums run in a fixed order.
@@ -66,7 +67,10 @@ __global__ void __launch_bounds__(64) k_chip_ids(int np, int width, const int32_
 }
 
 // the values of one (job, slice) pair: S + alpha_c R in FP32, as the SpMV stages them
-__global__ void __launch_bounds__(256) k_chip_pack(const JobDev* __restrict__ jobs, const int2* __restrict__ js) {
+__global__ void __launch_bounds__(256) k_chip_pack(const JobDev* __restrict__ jobs, const int2* __restrict__ js,
+                                                   int* __restrict__ progress, int nprogress) {
+    const int at = (blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
+    if (at < nprogress) progress[at] = 0;
     const int2 pr = js[blockIdx.y];
     const JobDev& J = jobs[pr.x];
     const int s = pr.y, np = J.np, pos = blockIdx.x * 256 + threadIdx.x;
@@ -101,7 +105,7 @@ constexpr bool chip_dinv_in_lds() { return (size_t)NP * 4 * (G + 1) <= 140 * 102
 template <int G, int K, int NT>
 __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restrict__ jobs, const int4* __restrict__ items,
                                                     const int2* __restrict__ gin, int2* __restrict__ gout,
-                                                    int phase) {
+                                                    int* progress, int phase) {
     typedef typename ChipVec<G>::type VecG;
     constexpr int NP = K * NT, NA = NP / kAggRows;
     constexpr bool DLDS = chip_dinv_in_lds<G, NP>();
@@ -111,6 +115,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
     __shared__ VecG cys[NA];                       // coarse correction
     __shared__ float cs[NA];                       // c_a
     __shared__ double red1[NT / 64][2 * G], red2[NT / 64][2 * G];
+    __shared__ int told;                           // the leader's word
     const int4 it = items[blockIdx.x];
     const JobDev& J = jobs[it.x];
     const int s = it.y, lane0 = it.z * G, me = it.w + it.z;
@@ -135,10 +140,6 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
             if (tid == 0) gout[me] = make_int2(0, kChipEmpty);
             return;
         }
-        if (reference && it.z != lead) {
-            if (tid == 0) gout[me] = make_int2(-1, 0);
-            return;
-        }
     } else {
         const int2 own = gin[me];
         if (reference) target = gin[it.w + lead].x;
@@ -151,8 +152,10 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
             return;
         }
         target = min(target, J.maxit);             // every loop below ends by the iteration cap
-        steps = max(own.x, 0);
+        steps = own.x;
     }
+    const bool decides = phase == 0 && reference && it.z == lead, follows = phase == 0 && reference && !decides;
+    int* const word = progress + it.w;
     const bool coarse = J.cinv != nullptr, dc = s == J.dc;
     const int na = np / kAggRows, noct = J.width / 8;
     int npu = np;
@@ -342,10 +345,13 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
 
     // ---- iterations ------------------------------------------------------------
     int flags = 0;
+    bool late = false;
     while (true) {
         // opaque per iteration: the offsets and tests derived from these are formed where they
         // are used instead of being kept in (spilled) registers across the loop
         asm volatile("" : "+s"(npu), "+s"(wave), "+v"(real));
+        int seen = 0;
+        if (follows && tid == 0) seen = lead_seen(word);
         double pq[G];
 #pragma unroll
         for (int c = 0; c < G; ++c) pq[c] = 0.0;
@@ -442,6 +448,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
         precondition();
         double vz[G], vr[G], rz, rr;
         dots(vz, vr);
+        if (follows && tid == 0) told = lead_word(word, steps + 1, seen);
         block_sum(red2, vz, vr, true, rz, rr);
         // beta = rho' / rho (rho == 0 zeroes p)
         const float be = rho != 0.0 ? (float)(rz / rho) : 0.0f;
@@ -457,12 +464,17 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
         const bool live = __ballot(open) != 0;
         const bool nan = __ballot(lane < J.R && bb > 0.0 && rr != rr) != 0;
         bool stop;
-        if (reference && it.z != lead) stop = steps >= target;
+        if (follows) {
+            const int v = told;
+            late = v < 0;
+            stop = late || v == 2 * steps + 1;
+        } else if (reference && it.z != lead) stop = steps >= target;
         else {
             stop = (!live && (phase == 0 || steps >= target)) || steps >= J.maxit;
             if (live && steps >= J.maxit) flags = kChipCapped;
         }
         if (nan) { stop = true; flags = kChipNan; }
+        if (decides && tid == 0) lead_tell(word, 2 * steps + stop);
         // x += alpha p, p = z + beta p
         float b[G];
 #pragma unroll
@@ -495,7 +507,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
     }
 
     // ---- result, and the state from which a later phase goes on -----------------
-    const bool keep = !reference;
+    const bool keep = !reference || late;
     each_row<K>([&](auto kc) __attribute__((always_inline)) {
         constexpr int k = decltype(kc)::value;
         if (has(k)) {
@@ -551,18 +563,20 @@ void launch_chip_ids(int np, int width, const int32_t* ids, const uint8_t* gw, c
     check_launch();
 }
 
-void launch_chip_pack(const JobDev* d_jobs, const int2* d_js, int njs, int max_np, hipStream_t st) {
-    k_chip_pack<<<dim3(max_np / 256, njs), 256, 0, st>>>(d_jobs, d_js);
+void launch_chip_pack(const JobDev* d_jobs, const int2* d_js, int njs, int max_np, int* progress, int nprogress,
+                      hipStream_t st) {
+    MPF_REQUIRE(nprogress <= njs * max_np, "on-chip solver: more lane groups than threads");
+    k_chip_pack<<<dim3(max_np / 256, njs), 256, 0, st>>>(d_jobs, d_js, progress, nprogress);
     check_launch();
 }
 
 template <int G, int NT, int MAXK>
 static void chip_dispatch(const JobDev* d_jobs, const int4* d_items, int n, const ChipShape& c, const int2* gin,
-                          int2* gout, int phase, hipStream_t st) {
+                          int2* gout, int* progress, int phase, hipStream_t st) {
 #define MPF_CHIP(k)                                                                                      \
     case k:                                                                                              \
         if constexpr (k <= MAXK) {                                                             \
-            k_pcg_chip<G, k, NT><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, phase);            \
+            k_pcg_chip<G, k, NT><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, phase);            \
             return;                                                                                      \
         }                                                                                                \
         break;
@@ -576,12 +590,12 @@ static void chip_dispatch(const JobDev* d_jobs, const int4* d_items, int n, cons
 }
 
 void launch_chip(const JobDev* d_jobs, const int4* d_items, int n, const ChipShape& c, const int2* gin, int2* gout,
-                 int phase, hipStream_t st) {
+                 int* progress, int phase, hipStream_t st) {
     if (!n) return;
-    if (c.G == 4) chip_dispatch<4, 512, 10>(d_jobs, d_items, n, c, gin, gout, phase, st);
-    else if (c.G == 2 && c.threads <= 512) chip_dispatch<2, 512, 20>(d_jobs, d_items, n, c, gin, gout, phase, st);
-    else if (c.G == 2) chip_dispatch<2, 1024, 8>(d_jobs, d_items, n, c, gin, gout, phase, st);
-    else chip_dispatch<1, 1024, 20>(d_jobs, d_items, n, c, gin, gout, phase, st);
+    if (c.G == 4) chip_dispatch<4, 512, 10>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
+    else if (c.G == 2 && c.threads <= 512) chip_dispatch<2, 512, 20>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
+    else if (c.G == 2) chip_dispatch<2, 1024, 8>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
+    else chip_dispatch<1, 1024, 20>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
     check_launch();
 }
 

@@ -6,7 +6,7 @@
 //
 // Bound by the chain of an iteration (two block sums with their barriers, two complex divisions,
 // the gathers), not by any pipe.  Measured (MI355X): two frames x 3 harmonics of 1261 nodes, 16
-// patterns, 216 steps of the reference rule: 10.8 -> 1.6 ms per forward solve (before: six launches
+// patterns, 216 steps of the reference rule: 10.8 -> 0.88 ms per forward solve (before: six launches
 // per iteration).
 #include <climits>
 
@@ -16,7 +16,10 @@
 namespace mpf {
 
 // values S + alpha_c R of every (job, slice): cval [C][width / 8][4][np] float4 (two entries each)
-__global__ void __launch_bounds__(256) k_c_chip_pack(const CJob* __restrict__ jobs, const int2* __restrict__ js) {
+__global__ void __launch_bounds__(256) k_c_chip_pack(const CJob* __restrict__ jobs, const int2* __restrict__ js,
+                                                     int* __restrict__ progress, int nprogress) {
+    const int at = (blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
+    if (at < nprogress) progress[at] = 0;
     const int2 pr = js[blockIdx.y];
     const CJob& J = jobs[pr.x];
     const int s = pr.y, np = J.np, pos = blockIdx.x * 256 + threadIdx.x;
@@ -69,12 +72,13 @@ struct ZDiv {
 template <int G, int K, int NT, bool HOLD>
 __global__ void __launch_bounds__(NT, NT / 256) k_c_chip(const CJob* __restrict__ jobs, const int4* __restrict__ items,
                                                          const int2* __restrict__ gin, int2* __restrict__ gout,
-                                                         int phase) {
+                                                         int* progress, int phase) {
     constexpr int NP = K * NT, W = 2 * G;
     typedef typename ChipVec<W>::type VecW;        // G complex columns
     __shared__ VecW ps[NP];
     __shared__ float2 ds[NP];
     __shared__ double red1[NT / 64][2 * W], red2[NT / 64][W + G];
+    __shared__ int told;                           // the leader's word
     const int4 it = items[blockIdx.x];
     const CJob& J = jobs[it.x];
     const int s = it.y, lane0 = it.z * G, me = it.w + it.z;
@@ -95,10 +99,6 @@ __global__ void __launch_bounds__(NT, NT / 256) k_c_chip(const CJob* __restrict_
             if (tid == 0) gout[me] = make_int2(0, kChipEmpty);
             return;
         }
-        if (reference && it.z != lead) {
-            if (tid == 0) gout[me] = make_int2(-1, 0);
-            return;
-        }
     } else {
         const int2 own = gin[me];
         if (reference) target = gin[it.w + lead].x;
@@ -111,8 +111,10 @@ __global__ void __launch_bounds__(NT, NT / 256) k_c_chip(const CJob* __restrict_
             return;
         }
         target = min(target, J.maxit);
-        steps = max(own.x, 0);
+        steps = own.x;
     }
+    const bool decides = phase == 0 && reference && it.z == lead, follows = phase == 0 && reference && !decides;
+    int* const word = progress + it.w;
     const int noct = J.width / 8;
     int npu = np;
     const __amdgpu_buffer_rsrc_t ids = uniform_rsrc(J.cid, (size_t)noct * np * 16);
@@ -215,8 +217,11 @@ __global__ void __launch_bounds__(NT, NT / 256) k_c_chip(const CJob* __restrict_
 
     // ---- iterations ------------------------------------------------------------
     int flags = 0;
+    bool late = false;
     while (true) {
         asm volatile("" : "+s"(npu), "+s"(wave), "+v"(real));   // as in chip.hip
+        int seen = 0;
+        if (follows && tid == 0) seen = lead_seen(word);
         double pq[W], pu[W];
 #pragma unroll
         for (int c = 0; c < W; ++c) { pq[c] = 0.0; pu[c] = 0.0; }
@@ -331,6 +336,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_c_chip(const CJob* __restrict_
         double vz[W], vr[G], rr;
         precondition(vz, vr);
         zd rz;
+        if (follows && tid == 0) told = lead_word(word, steps + 1, seen);
         sum_zr(vz, vr, rz, rr);
         const bool rz0 = zzero(rho);
         const zd be = rz0 ? zmake(0.0) : by_rho.of(rz);
@@ -345,13 +351,18 @@ __global__ void __launch_bounds__(NT, NT / 256) k_c_chip(const CJob* __restrict_
         const bool live = __ballot(open) != 0;
         const bool bad = __ballot(mine && !(isfinite(rr) && isfinite(rz.x) && isfinite(rz.y))) != 0;
         bool stop;
-        if (reference && it.z != lead) stop = steps >= target;
+        if (follows) {
+            const int v = told;
+            late = v < 0;
+            stop = late || v == 2 * steps + 1;
+        } else if (reference && it.z != lead) stop = steps >= target;
         else {
             stop = (!live && (phase == 0 || steps >= target)) || steps >= J.maxit;
             // the iteration cap reports, converged in its last step or not
             if (steps >= J.maxit) flags = kChipCapped;
         }
         if (bad) { stop = true; flags = kChipNan; }
+        if (decides && tid == 0) lead_tell(word, 2 * steps + stop);
         zd b[G];
 #pragma unroll
         for (int g = 0; g < G; ++g)
@@ -374,7 +385,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_c_chip(const CJob* __restrict_
     }
 
     // ---- result and state ------------------------------------------------------
-    const bool keep = !reference;
+    const bool keep = !reference || late;
     each_row<K>([&](auto kc) __attribute__((always_inline)) {
         constexpr int k = decltype(kc)::value;
         if (has(k)) {
@@ -415,25 +426,27 @@ ChipShape c_chip_shape(int np, long long lanes) {
     return c;
 }
 
-void launch_c_chip_pack(const CJob* d_jobs, const int2* d_js, int njs, int np, hipStream_t st) {
-    k_c_chip_pack<<<dim3(np / 256, njs), 256, 0, st>>>(d_jobs, d_js);
+void launch_c_chip_pack(const CJob* d_jobs, const int2* d_js, int njs, int np, int* progress, int nprogress,
+                        hipStream_t st) {
+    MPF_REQUIRE(nprogress <= njs * np, "on-chip solver: more lane groups than threads");
+    k_c_chip_pack<<<dim3(np / 256, njs), 256, 0, st>>>(d_jobs, d_js, progress, nprogress);
     check_launch();
 }
 
 template <int G, int NT>
 static void c_chip_dispatch(const CJob* d_jobs, const int4* d_items, int n, const ChipShape& c, bool one_oct,
-                            const int2* gin, int2* gout, int phase, hipStream_t st) {
+                            const int2* gin, int2* gout, int* progress, int phase, hipStream_t st) {
     // (1024 threads take more than 4096 rows.)  Rows of one 8-slot group: the matrix stays in registers where they have room for it (20 per
     // row; 1280 rows 1.85 -> 1.54 ms per call)
 #define MPF_CHIP(k)                                                                                \
     case k:                                                                                        \
         if constexpr (G == 1 && NT == 512 && k <= 5)                                               \
             if (one_oct) {                                                                         \
-                k_c_chip<G, k, NT, true><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, phase); \
+                k_c_chip<G, k, NT, true><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, phase); \
                 return;                                                                            \
             }                                                                                      \
         if constexpr (NT == 512 || k > 4) {                                                        \
-            k_c_chip<G, k, NT, false><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, phase); \
+            k_c_chip<G, k, NT, false><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, phase); \
             return;                                                                                \
         }                                                                                          \
         break;
@@ -446,11 +459,11 @@ static void c_chip_dispatch(const CJob* d_jobs, const int4* d_items, int n, cons
 }
 
 void launch_c_chip(const CJob* d_jobs, const int4* d_items, int n, const ChipShape& c, int width, const int2* gin,
-                   int2* gout, int phase, hipStream_t st) {
+                   int2* gout, int* progress, int phase, hipStream_t st) {
     const bool one_oct = width == 8;
-    if (c.G == 2) c_chip_dispatch<2, 512>(d_jobs, d_items, n, c, one_oct, gin, gout, phase, st);
-    else if (c.threads <= 512) c_chip_dispatch<1, 512>(d_jobs, d_items, n, c, one_oct, gin, gout, phase, st);
-    else c_chip_dispatch<1, 1024>(d_jobs, d_items, n, c, one_oct, gin, gout, phase, st);
+    if (c.G == 2) c_chip_dispatch<2, 512>(d_jobs, d_items, n, c, one_oct, gin, gout, progress, phase, st);
+    else if (c.threads <= 512) c_chip_dispatch<1, 512>(d_jobs, d_items, n, c, one_oct, gin, gout, progress, phase, st);
+    else c_chip_dispatch<1, 1024>(d_jobs, d_items, n, c, one_oct, gin, gout, progress, phase, st);
     check_launch();
 }
 

@@ -52,6 +52,7 @@ struct ComplexModel::Impl {
     DBuf<float4> cval;
     DBuf<int4> chip_items;
     DBuf<int2> gst[2];               // (steps, flags) of every lane group, before and after a phase
+    DBuf<int> progress;              // the deciding group's steps, at its pair's first group index
     int2* h_gst = nullptr;
 
     bool ensure_chip();
@@ -113,6 +114,7 @@ bool ComplexModel::Impl::ensure_chip() {
             g.alloc(total);
             MPF_HIP(hipMemsetAsync(g.p, 0, g.bytes(), st0));
         }
+        progress.alloc(total);
         MPF_HIP(hipHostMalloc((void**)&h_gst, sizeof(int2) * total, hipHostMallocDefault));
         launch_chip_order(np, tpos.p, crow.p, cpos.p, st0);
         launch_chip_ids(np, W, ids.p, gw.p, crow.p, cpos.p, cid.p, octs.p, st0);
@@ -135,11 +137,12 @@ bool ComplexModel::Impl::ensure_chip() {
 void ComplexModel::Impl::run_chip() {
     hipStream_t st0 = ctx->stream;
     const int groups = Rq / shape.G, total = njs * groups;
-    launch_c_chip_pack(jobs.p, js.p, njs, S.np, st0);
-    launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, gst[1].p, gst[0].p, 0, st0);
+    launch_c_chip_pack(jobs.p, js.p, njs, S.np, progress.p, total, st0);
+    launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, gst[1].p, gst[0].p, progress.p, 0, st0);
     int in = 0;
     for (bool open = true; open;) {
-        launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, gst[in].p, gst[in ^ 1].p, 1, st0);
+        launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, gst[in].p, gst[in ^ 1].p, progress.p, 1,
+                      st0);
         in ^= 1;
         MPF_HIP(hipMemcpyAsync(h_gst, gst[in].p, sizeof(int2) * total, hipMemcpyDeviceToHost, st0));
         MPF_HIP(hipStreamSynchronize(st0));

@@ -259,6 +259,7 @@ bool KrylovDriver::ensure_chip() {
         chip_js.upload(h_chip_js.data(), h_chip_js.size(), s0);
         gst[0].alloc(total);
         gst[1].alloc(total);
+        progress.alloc(total);
         MPF_HIP(hipMemsetAsync(gst[0].p, 0, gst[0].bytes(), s0));
         MPF_HIP(hipMemsetAsync(gst[1].p, 0, gst[1].bytes(), s0));
         MPF_HIP(hipHostMalloc((void**)&h_gst, sizeof(int2) * total, hipHostMallocDefault));
@@ -279,14 +280,15 @@ bool KrylovDriver::ensure_chip() {
 // which the pair's slowest group stopped).  Step counts and flags go to h_st.
 void KrylovDriver::run_chip() {
     hipStream_t s0 = ctx->stream;
-    launch_chip_pack(jobs.p, chip_js.p, (int)h_chip_js.size(), chip_max_np, s0);
     const int total = chip_first.back();
+    launch_chip_pack(jobs.p, chip_js.p, (int)h_chip_js.size(), chip_max_np, progress.p, total, s0);
     auto phase = [&](int ph, int in) {
         if (chips.size() > 1) MPF_HIP(hipEventRecord(chip_fork, s0));
         for (auto& c : chips) {
             hipStream_t s = c.stream ? c.stream : s0;
             if (c.stream) MPF_HIP(hipStreamWaitEvent(s, chip_fork, 0));
-            launch_chip(jobs.p, c.items.p, (int)c.h_items.size(), c.shape, gst[in].p, gst[in ^ 1].p, ph, s);
+            launch_chip(jobs.p, c.items.p, (int)c.h_items.size(), c.shape, gst[in].p, gst[in ^ 1].p, progress.p, ph,
+                        s);
             if (c.stream) {
                 MPF_HIP(hipEventRecord(c.done, s));
                 MPF_HIP(hipStreamWaitEvent(s0, c.done, 0));

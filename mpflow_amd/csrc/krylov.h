@@ -96,6 +96,7 @@ class KrylovDriver {
     std::vector<int2> h_chip_js;      // the on-chip (job, slice) pairs
     std::vector<int> chip_first;      // first group index of each pair; then the total
     DBuf<int2> chip_js, gst[2];
+    DBuf<int> progress;               // the deciding group's steps, at its pair's first group index
     DBuf<float4> cval;
     std::vector<size_t> cval_off;     // per job
     int chip_max_np = 0;
