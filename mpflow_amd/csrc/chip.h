@@ -13,11 +13,12 @@ constexpr int kChipCus = 256;         // one workgroup each
 
 struct ChipShape {
     int G = 0, K = 0, threads = 0;
+    bool hold = false;                // the matrix in registers (padded ELL width 8)
 };
-// The shape for np padded rows when a solve has `lanes` (job, harmonic, lane) triples in
-// all.  Enough lanes to fill the chip: the largest group, 512 threads; fewer: the smallest
-// group that keeps every workgroup on a CU of its own, 1024 threads.
-ChipShape chip_shape(int np, long long lanes);
+// The shape for np padded rows of `width` slots when a solve has `lanes` (job, harmonic, lane)
+// triples in all.  Enough lanes to fill the chip: the largest group; fewer: the smallest group
+// that keeps every workgroup on a CU of its own.
+ChipShape chip_shape(int np, int width, long long lanes);
 
 // gst flags of a lane group
 constexpr int kChipCapped = 1, kChipNan = 2, kChipEmpty = 4;

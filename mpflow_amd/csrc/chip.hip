@@ -13,10 +13,10 @@
 // first coarse entries are loaded before the barrier that the sums wait for, and 512 threads
 // with 256 VGPRs beat 1024 with 128 where there are lanes enough for every CU.
 //
-// Measured (MI355X, whole calls): one 2D forward solve of 817 nodes, 168 steps, 4.60 -> 0.58
+// Measured (MI355X, whole calls): one 2D forward solve of 817 nodes, 168 steps, 4.60 -> 0.42
 // ms (1.02 ms with the deciding group of the reference rule run before the others); 64 frames x 5
 // harmonics of 4921 nodes to 1e-6 18.1 -> 5.5 ms (1024 threads 7.2 ms); a caller's 4921-row
-// matrix with 32 columns 2.02 -> 0.63 ms.
+// matrix with 32 columns 2.02 -> 0.54 ms.
 //
 // The recurrences, the FP64 scalars, the stop rules and the breakdown rules are those of the
 // streaming kernels (sparse.hip); sums run in a fixed order.
@@ -101,8 +101,9 @@ template <int G, int NP>
 constexpr bool chip_dinv_in_lds() { return (size_t)NP * 4 * (G + 1) <= 140 * 1024; }
 
 // NT = 512: two wavefronts per SIMD with 256 VGPRs each, the most right-hand sides per
-// iteration; NT = 1024: four per SIMD with 128 VGPRs, the shortest iteration of few lanes.
-template <int G, int K, int NT>
+// iteration; NT = 1024: four per SIMD with 128 VGPRs, the shortest iteration of two lanes.
+// HOLD: one 8-slot group per row, kept in registers over the iterations.
+template <int G, int K, int NT, bool HOLD>
 __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restrict__ jobs, const int4* __restrict__ items,
                                                     const int2* __restrict__ gin, int2* __restrict__ gout,
                                                     int* progress, int phase) {
@@ -170,6 +171,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
     auto has = [&](int k) { return (wave + k * nw) * kAggRows < npu; };
     float r[K][G], x[K][G], q[K][G];               // q: A p, then z
     float di[DLDS ? 1 : K];
+    v4u hid[HOLD ? K : 1], hva[HOLD ? K : 1], hvb[HOLD ? K : 1];
     uint64_t more = 0;                             // 2 bits per k: 8-slot groups after the first
     uint32_t real = 0;                             // bit k: a row of the matrix, not padding
     auto dinv = [&](int k) {
@@ -301,6 +303,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
             if (has(k)) {
                 const int row = rowof[pos];
                 const size_t o = (size_t)row * Rp;
+                if constexpr (HOLD) { hid[k] = load(ids, k * nt); hva[k] = load(val, k * nt); hvb[k] = load(val, np + k * nt); }
                 if (noct > 1)
                     more |= (uint64_t)(__builtin_amdgcn_readfirstlane((int)gp(J.cocts)[wave + k * nw]) - 1) << (2 * k);
                 if (row < n) {
@@ -356,12 +359,15 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
 #pragma unroll
         for (int c = 0; c < G; ++c) pq[c] = 0.0;
         // the next positions' first 8 slots are loaded while the current ones are gathered
-        v4u idn = load(ids, 0), van = load(val, 0), vbn = load(val, npu);
+        v4u idn, van, vbn;
+        if constexpr (!HOLD) { idn = load(ids, 0); van = load(val, 0); vbn = load(val, npu); }
         each_row<K>([&](auto kc) __attribute__((always_inline)) {
             constexpr int k = decltype(kc)::value;
-            __builtin_amdgcn_sched_barrier(0);
-            v4u id = idn, va = van, vb = vbn;
-            if (k + 1 < K) {
+            if constexpr (!HOLD) __builtin_amdgcn_sched_barrier(0);
+            v4u id, va, vb;
+            if constexpr (HOLD) { id = hid[k]; va = hva[k]; vb = hvb[k]; }
+            else { id = idn; va = van; vb = vbn; }
+            if (!HOLD && k + 1 < K) {
                 // past the last position the loads are out of range or another row's: unused
                 idn = load(ids, (k + 1) * nt);
                 van = load(val, (k + 1) * nt);
@@ -375,7 +381,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
                         // four gathers in flight (registers)
-                        __builtin_amdgcn_sched_barrier(0);
+                        if constexpr (!HOLD) __builtin_amdgcn_sched_barrier(0);
                         const v4u w = h ? vb : va;
                         float g[4][G];
 #pragma unroll
@@ -386,7 +392,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
 #pragma unroll
                             for (int c = 0; c < G; ++c) acc[c] = fmaf(__uint_as_float(w[u]), g[u][c], acc[c]);
                     }
-                    if (o++ >= (int)((more >> (2 * k)) & 3)) break;
+                    if (HOLD || o++ >= (int)((more >> (2 * k)) & 3)) break;
                     id = load(ids, o * npu + k * nt);
                     va = load(val, 2 * o * npu + k * nt);
                     vb = load(val, (2 * o + 1) * npu + k * nt);
@@ -536,15 +542,21 @@ static inline void check_launch() {
     if (e != hipSuccess) throw Error(MPF_EHIP, std::string("kernel launch: ") + hipGetErrorString(e));
 }
 
-ChipShape chip_shape(int np, long long lanes) {
+ChipShape chip_shape(int np, int width, long long lanes) {
     // the largest lane group whose rows fit the registers
     const int fit = np <= 512 * 10 ? 4 : (np <= 512 * 20 ? 2 : 1);
     ChipShape c;
     c.threads = fit == 1 ? 1024 : 512;
     c.G = fit;
     while (c.G > 1 && lanes <= (c.G / 2) * kChipCus) c.G /= 2;
-    // few lanes: 1024 threads where 128 VGPRs hold the rows without spills
-    if (c.G == 1 || (c.G == 2 && lanes <= 2 * kChipCus && np <= 1024 * 8)) c.threads = 1024;
+    // few lanes: 1024 threads where 128 VGPRs hold the rows without spills, but one lane of a
+    // small mesh takes 512 -- half the wavefronts repeat the scalars, and 256 VGPRs hold the matrix
+    // of rows of one 8-slot group.  817 rows: 0.58 ms per call at 1024 threads, 0.49 at 512, 0.42
+    // with the matrix held; a 4921-row matrix with 32 columns 0.62, 0.58, 0.54 ms; one
+    // Gauss-Newton step of 4921 nodes 3.77, 3.87, 3.72 ms, hence half the rows without it.
+    c.hold = c.G == 1 && width == 8 && np <= 512 * 10;
+    if (c.G == 1) c.threads = c.hold || np <= 512 * 5 ? 512 : 1024;
+    if (c.G == 2 && lanes <= 2 * kChipCus && np <= 1024 * 8) c.threads = 1024;
     const int k = (np + c.threads - 1) / c.threads;
     for (int q : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20})
         if (k <= q) { c.K = q; break; }
@@ -570,15 +582,21 @@ void launch_chip_pack(const JobDev* d_jobs, const int2* d_js, int njs, int max_n
     check_launch();
 }
 
-template <int G, int NT, int MAXK>
+// kernels for MINK..MAXK rows per thread; up to MAXH the matrix may stay in registers
+template <int G, int NT, int MINK, int MAXK, int MAXH>
 static void chip_dispatch(const JobDev* d_jobs, const int4* d_items, int n, const ChipShape& c, const int2* gin,
                           int2* gout, int* progress, int phase, hipStream_t st) {
-#define MPF_CHIP(k)                                                                                      \
-    case k:                                                                                              \
-        if constexpr (k <= MAXK) {                                                             \
-            k_pcg_chip<G, k, NT><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, phase);            \
-            return;                                                                                      \
-        }                                                                                                \
+#define MPF_CHIP(k)                                                                                           \
+    case k:                                                                                                   \
+        if constexpr (k <= MAXH)                                                                              \
+            if (c.hold) {                                                                                     \
+                k_pcg_chip<G, k, NT, true><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, phase); \
+                return;                                                                                       \
+            }                                                                                                 \
+        if constexpr (k >= MINK && k <= MAXK) {                                                               \
+            k_pcg_chip<G, k, NT, false><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, phase); \
+            return;                                                                                           \
+        }                                                                                                     \
         break;
     switch (c.K) {
         MPF_CHIP(1) MPF_CHIP(2) MPF_CHIP(3) MPF_CHIP(4) MPF_CHIP(5) MPF_CHIP(6) MPF_CHIP(8) MPF_CHIP(10)
@@ -592,10 +610,13 @@ static void chip_dispatch(const JobDev* d_jobs, const int4* d_items, int n, cons
 void launch_chip(const JobDev* d_jobs, const int4* d_items, int n, const ChipShape& c, const int2* gin, int2* gout,
                  int* progress, int phase, hipStream_t st) {
     if (!n) return;
-    if (c.G == 4) chip_dispatch<4, 512, 10>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
-    else if (c.G == 2 && c.threads <= 512) chip_dispatch<2, 512, 20>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
-    else if (c.G == 2) chip_dispatch<2, 1024, 8>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
-    else chip_dispatch<1, 1024, 20>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
+    if (c.G == 4) chip_dispatch<4, 512, 1, 10, 0>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
+    else if (c.G == 2 && c.threads <= 512)
+        chip_dispatch<2, 512, 1, 20, 0>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
+    else if (c.G == 2) chip_dispatch<2, 1024, 1, 8, 0>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
+    else if (c.threads <= 512)
+        chip_dispatch<1, 512, 1, 5, 10>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
+    else chip_dispatch<1, 1024, 3, 20, 0>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
     check_launch();
 }
 

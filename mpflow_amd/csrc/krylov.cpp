@@ -209,10 +209,12 @@ bool KrylovDriver::ensure_chip() {
             for (int j : jobs_on) {
                 const JobDev& J = h[j];
                 if (c >= J.C) continue;
-                const ChipShape sh = chip_shape(J.np, lanes);
+                const ChipShape sh = chip_shape(J.np, J.width, lanes);
                 ChipClass* cl = nullptr;
                 for (auto& q : chips)
-                    if (q.shape.G == sh.G && q.shape.K == sh.K && q.shape.threads == sh.threads) cl = &q;
+                    if (q.shape.G == sh.G && q.shape.K == sh.K && q.shape.threads == sh.threads &&
+                        q.shape.hold == sh.hold)
+                        cl = &q;
                 if (!cl) {
                     chips.emplace_back();
                     cl = &chips.back();
