@@ -15,6 +15,7 @@ struct Mlp {
     std::vector<DBuf<float>> Z, H;  // pre-activations / activations of the last forward
     DBuf<float> dA, dB;             // backward work (batch x widest layer)
     DBuf<double> part, loss;
+    DBuf<float> work;               // partial sums of split products
     int cap = 0, batch = 0;
     const float* x_in = nullptr;    // input of the last forward (caller-owned)
     int64_t t = 0;                  // Adam steps taken

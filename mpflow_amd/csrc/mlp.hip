@@ -3,12 +3,10 @@
 //
 // Every GEMM runs on MFMA (v_mfma_f32_32x32x16_bf16): FP32 operands in HBM are rounded to
 // BF16 (nearest even) while staged in LDS, products accumulate in FP32.  One kernel covers
-// the three products of a layer through element strides:
+// the three products of a layer:
 //   forward   Z = H W (+ b)        A = H  (batch x in),  B = W   (in x out)
 //   backward  dW = H^T dZ          A = H^T,              B = dZ
 //             dH = dZ W^T          A = dZ,               B = W^T
-// Tiles of 64 x 64 outputs per 256-thread block (4 wavefronts x 32 x 32), K staged 32 at a
-// time; the staging loop walks the unit-stride dimension so loads coalesce.
 #include <cmath>
 
 #include "mlp.h"
@@ -18,181 +16,202 @@ namespace mpf {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-constexpr int kMT = 64;       // output tile
-constexpr int kMK = 32;       // K step
-constexpr int kMLds = kMK + 8;
-
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 __device__ __forceinline__ float gelu_grad(float x) {
     return 0.5f * (1.0f + erff(x * 0.70710678118654752f)) + x * 0.39894228040143268f * expf(-0.5f * x * x);
 }
 
-// C[m][n] = sum_k A(m, k) B(k, n) with A(m, k) = A[m*sam + k*sak], B(k, n) = B[k*sbk + n*sbn].
-// epi 0: C = acc;  1: Z = acc + bias[n] (stored in C) and H = GELU(Z);  2: C = acc + bias[n]
-__global__ void __launch_bounds__(256) k_mlp_gemm(int M, int N, int K, const float* __restrict__ A, long sam,
-                                                  long sak, const float* __restrict__ B, long sbk, long sbn,
-                                                  float* __restrict__ C, int ldc, int epi,
-                                                  const float* __restrict__ bias, float* __restrict__ H) {
-    __shared__ __attribute__((aligned(16))) __bf16 sa[kMT][kMLds];   // [m][k]
-    __shared__ __attribute__((aligned(16))) __bf16 sb[kMT][kMLds];   // [n][k]
-    const int m0 = blockIdx.y * kMT, n0 = blockIdx.x * kMT;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    f32x16_t acc;
+// C[m][n] = sum_k A(m, k) B(k, n) with A(m, k) = A[m*pa + k] (AK) or A[k*pa + m], B(k, n) =
+// B[n*pb + k] (BK) or B[k*pb + n], at any pitch: the 128-bit loads are aligned to 4 bytes.  epi 0: C = acc;  1: Z = acc + bias[n] (stored in C) and H =
+// GELU(Z);  2: C = acc + bias[n].  With gridDim.z > 1 slice z sums the K steps [z per, (z + 1) per)
+// alone and stores its sum in part[z][m][n] (k_mlp_split_sum adds them).
+//
+// T x T outputs per workgroup, wavefronts of T/2 x T/2.  Each tile pair is staged 64 K at a time,
+// converted to BF16 and written to one of two LDS buffers while the MFMAs consume the other.
+// Rows and columns past M and N read a neighbour's values instead of being tested for (their
+// outputs are not stored); only K is padded with zeros.
+//
+// Bound by the FP32 operands' L2 and HBM reads: 128 x 128 where that fills the chip halves them,
+// and a product with few tiles splits K until it has enough workgroups.  Measured (MI355X) on
+// 1024 -> 2048 x 3 -> 9600: one forward pass of 64 rows 35 -> 11 + 5 us per layer (unsplit, the
+// weights came at 0.9 TB/s; now 3), forward and backward of 4096 rows 234 -> 353 TFLOP/s.
+constexpr int kGK = 64;                // K step
+constexpr int kGL = kGK + 8;           // LDS row: 72 BF16 (144 bytes, 16-byte aligned)
+typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+
+// one operand's T x 64 tile: rows r0.. (of `rows`), steps k0.. (of K)
+template <bool ALONG_K, int T>
+struct GemmTile {
+    static constexpr int kVec = T / 16;          // float4 per thread
+    float4 v[kVec];
+    __device__ __forceinline__ void load(const float* __restrict__ P, long pitch, int r0, int rows, int k0, int K) {
+        const int tid = threadIdx.x;
+        if (ALONG_K) {
+            // float4 u of thread t: row (t + 256 u) / 16, k from 4 ((t + 256 u) % 16)
+            if (k0 + kGK <= K) {
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
-    for (int k0 = 0; k0 < K; k0 += kMK) {
-        for (int i = tid; i < kMT * kMK; i += 256) {
-            int m, k;
-            if (sak == 1) { m = i / kMK; k = i % kMK; } else { m = i % kMT; k = i / kMT; }
-            const int gm = m0 + m, gk = k0 + k;
-            sa[m][k] = (__bf16)((gm < M && gk < K) ? A[gm * sam + gk * sak] : 0.0f);
-            int n, kb;
-            if (sbn == 1) { n = i % kMT; kb = i / kMT; } else { n = i / kMK; kb = i % kMK; }
-            const int gn = n0 + n, gkb = k0 + kb;
-            sb[n][kb] = (__bf16)((gn < N && gkb < K) ? B[gkb * sbk + gn * sbn] : 0.0f);
+                for (int u = 0; u < kVec; ++u) {
+                    const int f = tid + 256 * u, r = min(r0 + (f >> 4), rows - 1), c = k0 + 4 * (f & 15);
+                    const f32x4u_t w = *(const f32x4u_t*)(P + (size_t)r * pitch + c);
+                    v[u] = make_float4(w.x, w.y, w.z, w.w);
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < kVec; ++u) {
+                    const int f = tid + 256 * u, r = min(r0 + (f >> 4), rows - 1), c = k0 + 4 * (f & 15);
+                    float e[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) e[i] = P[(size_t)r * pitch + min(c + i, K - 1)];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) e[i] = c + i < K ? e[i] : 0.0f;
+                    v[u] = make_float4(e[0], e[1], e[2], e[3]);
+                }
+            }
+        } else {
+            // 4 x 4 blocks: float4 4 h + u of thread t is step 4 (b / (T / 4)) + u of the four rows
+            // from 4 (b % (T / 4)), b = t + 256 h
+            const bool whole = r0 + T <= rows;
+#pragma unroll
+            for (int h = 0; h < kVec / 4; ++h)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int b = tid + 256 * h, k = k0 + 4 * (b / (T / 4)) + u, c = r0 + 4 * (b % (T / 4));
+                    const float* row = P + (size_t)min(k, K - 1) * pitch;
+                    float4 e;
+                    if (whole) {
+                        const f32x4u_t w = *(const f32x4u_t*)(row + c);
+                        e = make_float4(w.x, w.y, w.z, w.w);
+                    } else {
+                        e = make_float4(row[min(c, rows - 1)], row[min(c + 1, rows - 1)], row[min(c + 2, rows - 1)],
+                                        row[min(c + 3, rows - 1)]);
+                    }
+                    v[4 * h + u] = e;
+                }
+            if (k0 + kGK > K) {
+#pragma unroll
+                for (int h = 0; h < kVec / 4; ++h)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (k0 + 4 * ((tid + 256 * h) / (T / 4)) + u >= K) v[4 * h + u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
         }
-        __syncthreads();
+    }
+    __device__ __forceinline__ void store(__bf16 (*s)[kGL]) const {
+        const int tid = threadIdx.x;
+        if (ALONG_K) {
 #pragma unroll
-        for (int ks = 0; ks < kMK; ks += 16) {
+            for (int u = 0; u < kVec; ++u) {
+                const int f = tid + 256 * u;
+                *reinterpret_cast<bf16x4_t*>(&s[f >> 4][4 * (f & 15)]) =
+                    bf16x4_t{(__bf16)v[u].x, (__bf16)v[u].y, (__bf16)v[u].z, (__bf16)v[u].w};
+            }
+        } else {
+#pragma unroll
+            for (int h = 0; h < kVec / 4; ++h) {
+                const int b = tid + 256 * h, kq = 4 * (b / (T / 4)), c = 4 * (b % (T / 4));
+                const float4 *q = v + 4 * h;
+                *reinterpret_cast<bf16x4_t*>(&s[c][kq]) =
+                    bf16x4_t{(__bf16)q[0].x, (__bf16)q[1].x, (__bf16)q[2].x, (__bf16)q[3].x};
+                *reinterpret_cast<bf16x4_t*>(&s[c + 1][kq]) =
+                    bf16x4_t{(__bf16)q[0].y, (__bf16)q[1].y, (__bf16)q[2].y, (__bf16)q[3].y};
+                *reinterpret_cast<bf16x4_t*>(&s[c + 2][kq]) =
+                    bf16x4_t{(__bf16)q[0].z, (__bf16)q[1].z, (__bf16)q[2].z, (__bf16)q[3].z};
+                *reinterpret_cast<bf16x4_t*>(&s[c + 3][kq]) =
+                    bf16x4_t{(__bf16)q[0].w, (__bf16)q[1].w, (__bf16)q[2].w, (__bf16)q[3].w};
+            }
+        }
+    }
+};
+
+template <bool AK, bool BK, int T>
+__global__ void __launch_bounds__(256, 2) k_mlp_gemm(int M, int N, int K, const float* __restrict__ A, long pa,
+                                                     const float* __restrict__ B, long pb, float* __restrict__ C,
+                                                     int ldc, int epi, const float* __restrict__ bias,
+                                                     float* __restrict__ H, float* __restrict__ part, int per) {
+    constexpr int W = T / 64;                                        // 32 x 32 MFMA tiles per wavefront side
+    __shared__ __attribute__((aligned(16))) __bf16 sa[2][T][kGL];    // [m][k]
+    __shared__ __attribute__((aligned(16))) __bf16 sb[2][T][kGL];    // [n][k]
+    const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
+    GemmTile<AK, T> ta;
+    GemmTile<BK, T> tb;
+    f32x16_t acc[W][W];
+#pragma unroll
+    for (int i = 0; i < W; ++i)
+#pragma unroll
+        for (int j = 0; j < W; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+    const int kt0 = blockIdx.z * per, kt1 = min((K + kGK - 1) / kGK, kt0 + per);
+    ta.load(A, pa, m0, M, kt0 * kGK, K);
+    tb.load(B, pb, n0, N, kt0 * kGK, K);
+    ta.store(sa[0]);
+    tb.store(sb[0]);
+    __syncthreads();
+    for (int kt = kt0; kt < kt1; ++kt) {
+        const int buf = (kt - kt0) & 1;
+        if (kt + 1 < kt1) {
+            ta.load(A, pa, m0, M, (kt + 1) * kGK, K);
+            tb.load(B, pb, n0, N, (kt + 1) * kGK, K);
+        }
+#pragma unroll
+        for (int ks = 0; ks < kGK; ks += 16) {
             const int kq = ks + (lane >> 5) * 8;
-            const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(&sa[wm + (lane & 31)][kq]);
-            const bf16x8_t b = *reinterpret_cast<const bf16x8_t*>(&sb[wn + (lane & 31)][kq]);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+            bf16x8_t a[W], b[W];
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                a[i] = *reinterpret_cast<const bf16x8_t*>(&sa[buf][wm + 32 * i + (lane & 31)][kq]);
+                b[i] = *reinterpret_cast<const bf16x8_t*>(&sb[buf][wn + 32 * i + (lane & 31)][kq]);
+            }
+#pragma unroll
+            for (int i = 0; i < W; ++i)
+#pragma unroll
+                for (int j = 0; j < W; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        if (kt + 1 < kt1) {
+            ta.store(sa[buf ^ 1]);
+            tb.store(sb[buf ^ 1]);
         }
         __syncthreads();
     }
     // accumulator layout: lane -> column (lane & 31) of the 32 x 32 sub-tile (stores
     // coalesce along rows of C), register v -> row 8*(v/4) + 4*(lane/32) + v%4
+    const bool split = gridDim.z > 1;
+    float* out = split ? part + (size_t)blockIdx.z * M * N : C;
+    const int ld = split ? N : ldc;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int row = m0 + wm + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        const int col = n0 + wn + (lane & 31);
-        if (row < M && col < N) {
-            float z = acc[v];
-            if (epi >= 1) z += bias[col];
-            C[(size_t)row * ldc + col] = z;
-            if (epi == 1) H[(size_t)row * ldc + col] = gelu(z);
-        }
-    }
+    for (int i = 0; i < W; ++i)
+#pragma unroll
+        for (int j = 0; j < W; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int row = m0 + wm + 32 * i + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                const int col = n0 + wn + 32 * j + (lane & 31);
+                if (row < M && col < N) {
+                    float z = acc[i][j][v];
+                    if (!split && epi >= 1) z += bias[col];
+                    out[(size_t)row * ld + col] = z;
+                    if (!split && epi == 1) H[(size_t)row * ldc + col] = gelu(z);
+                }
+            }
 }
 
-// The same product for operands whose unit-stride dimensions, sizes and pitches are
-// multiples of 4 floats: each 64 x 64 tile pair is staged 64 K at a time with 128-bit
-// loads along each operand's unit-stride dimension (AK: A(m, k) contiguous in k, else in
-// m; BK: B(k, n) contiguous in k, else in n), converted to BF16 and written to one of two
-// LDS buffers while the MFMAs consume the other.  The MFMA sequence per output (k chunks
-// of 16 in order) is the one k_mlp_gemm runs, so both give the same sums.
-constexpr int kGK = 64;                // K step of the staged kernel
-constexpr int kGL = kGK + 8;           // LDS row: 72 BF16 (144 bytes, 16-byte aligned)
-template <bool AK, bool BK>
-__global__ void __launch_bounds__(256) k_mlp_gemm4(int M, int N, int K, const float* __restrict__ A, long sam,
-                                                   long sak, const float* __restrict__ B, long sbk, long sbn,
-                                                   float* __restrict__ C, int ldc, int epi,
-                                                   const float* __restrict__ bias, float* __restrict__ H) {
-    __shared__ __attribute__((aligned(16))) __bf16 sa[2][kMT][kGL];   // [m][k]
-    __shared__ __attribute__((aligned(16))) __bf16 sb[2][kMT][kGL];   // [n][k]
-    const int m0 = blockIdx.y * kMT, n0 = blockIdx.x * kMT;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    // a tile is 64 x 64 floats = 1024 float4: four per thread.  Contiguous in k: float4 u
-    // of thread t covers row (t + 256 u) / 16 and k from 4 ((t + 256 u) % 16).  Contiguous
-    // in m (or n): thread t loads rows k = 4 (t / 16) + u, u = 0..3, of the four columns
-    // from 4 (t % 16), a 4 x 4 block it writes to LDS transposed, four k per 8-byte store.
-    float4 ra[4], rb[4];
-    auto load = [&](int k0) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (AK) {
-                const int f = tid + 256 * u, r = f >> 4, c = 4 * (f & 15);   // r = m, c = k
-                if (m0 + r < M && k0 + c < K) v = *(const float4*)(A + (size_t)(m0 + r) * sam + (k0 + c));
-            } else {
-                const int k = 4 * (tid >> 4) + u, c = 4 * (tid & 15);        // c = m
-                if (k0 + k < K && m0 + c < M) v = *(const float4*)(A + (size_t)(k0 + k) * sak + (m0 + c));
-            }
-            ra[u] = v;
-            float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (BK) {
-                const int f = tid + 256 * u, r = f >> 4, c = 4 * (f & 15);   // r = n, c = k
-                if (n0 + r < N && k0 + c < K) w = *(const float4*)(B + (size_t)(n0 + r) * sbn + (k0 + c));
-            } else {
-                const int k = 4 * (tid >> 4) + u, c = 4 * (tid & 15);        // c = n
-                if (k0 + k < K && n0 + c < N) w = *(const float4*)(B + (size_t)(k0 + k) * sbk + (n0 + c));
-            }
-            rb[u] = w;
-        }
-    };
-    typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-    auto store = [&](int buf) {
-        if (AK) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int f = tid + 256 * u, r = f >> 4, c = 4 * (f & 15);
-                *reinterpret_cast<bf16x4_t*>(&sa[buf][r][c]) =
-                    bf16x4_t{(__bf16)ra[u].x, (__bf16)ra[u].y, (__bf16)ra[u].z, (__bf16)ra[u].w};
-            }
-        } else {
-            const int kq = 4 * (tid >> 4), c = 4 * (tid & 15);
-            *reinterpret_cast<bf16x4_t*>(&sa[buf][c][kq]) =
-                bf16x4_t{(__bf16)ra[0].x, (__bf16)ra[1].x, (__bf16)ra[2].x, (__bf16)ra[3].x};
-            *reinterpret_cast<bf16x4_t*>(&sa[buf][c + 1][kq]) =
-                bf16x4_t{(__bf16)ra[0].y, (__bf16)ra[1].y, (__bf16)ra[2].y, (__bf16)ra[3].y};
-            *reinterpret_cast<bf16x4_t*>(&sa[buf][c + 2][kq]) =
-                bf16x4_t{(__bf16)ra[0].z, (__bf16)ra[1].z, (__bf16)ra[2].z, (__bf16)ra[3].z};
-            *reinterpret_cast<bf16x4_t*>(&sa[buf][c + 3][kq]) =
-                bf16x4_t{(__bf16)ra[0].w, (__bf16)ra[1].w, (__bf16)ra[2].w, (__bf16)ra[3].w};
-        }
-        if (BK) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int f = tid + 256 * u, r = f >> 4, c = 4 * (f & 15);
-                *reinterpret_cast<bf16x4_t*>(&sb[buf][r][c]) =
-                    bf16x4_t{(__bf16)rb[u].x, (__bf16)rb[u].y, (__bf16)rb[u].z, (__bf16)rb[u].w};
-            }
-        } else {
-            const int kq = 4 * (tid >> 4), c = 4 * (tid & 15);
-            *reinterpret_cast<bf16x4_t*>(&sb[buf][c][kq]) =
-                bf16x4_t{(__bf16)rb[0].x, (__bf16)rb[1].x, (__bf16)rb[2].x, (__bf16)rb[3].x};
-            *reinterpret_cast<bf16x4_t*>(&sb[buf][c + 1][kq]) =
-                bf16x4_t{(__bf16)rb[0].y, (__bf16)rb[1].y, (__bf16)rb[2].y, (__bf16)rb[3].y};
-            *reinterpret_cast<bf16x4_t*>(&sb[buf][c + 2][kq]) =
-                bf16x4_t{(__bf16)rb[0].z, (__bf16)rb[1].z, (__bf16)rb[2].z, (__bf16)rb[3].z};
-            *reinterpret_cast<bf16x4_t*>(&sb[buf][c + 3][kq]) =
-                bf16x4_t{(__bf16)rb[0].w, (__bf16)rb[1].w, (__bf16)rb[2].w, (__bf16)rb[3].w};
-        }
-    };
-    f32x16_t acc;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
-    const int nk = (K + kGK - 1) / kGK;
-    load(0);
-    store(0);
-    __syncthreads();
-    for (int kt = 0; kt < nk; ++kt) {
-        const int buf = kt & 1;
-        if (kt + 1 < nk) load((kt + 1) * kGK);
-#pragma unroll
-        for (int ks = 0; ks < kGK; ks += 16) {
-            const int kq = ks + (lane >> 5) * 8;
-            const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(&sa[buf][wm + (lane & 31)][kq]);
-            const bf16x8_t b = *reinterpret_cast<const bf16x8_t*>(&sb[buf][wn + (lane & 31)][kq]);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-        }
-        if (kt + 1 < nk) store(buf ^ 1);
-        __syncthreads();
-    }
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int row = m0 + wm + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        const int col = n0 + wn + (lane & 31);
-        if (row < M && col < N) {
-            float z = acc[v];
-            if (epi >= 1) z += bias[col];
-            C[(size_t)row * ldc + col] = z;
-            if (epi == 1) H[(size_t)row * ldc + col] = gelu(z);
-        }
-    }
+// the slices' sums added in order, then the epilogue of k_mlp_gemm
+__global__ void __launch_bounds__(256) k_mlp_split_sum(int M, int N, int slices, const float* __restrict__ part,
+                                                       float* __restrict__ C, int ldc, int epi,
+                                                       const float* __restrict__ bias, float* __restrict__ H) {
+    const int col = blockIdx.x * 256 + threadIdx.x, row = blockIdx.y;
+    if (col >= N) return;
+    const size_t o = (size_t)row * N + col, step = (size_t)M * N;
+    float z = 0.0f;
+#pragma unroll 8
+    for (int q = 0; q < slices; ++q) z += part[q * step + o];
+    if (epi >= 1) z += bias[col];
+    C[(size_t)row * ldc + col] = z;
+    if (epi == 1) H[(size_t)row * ldc + col] = gelu(z);
 }
 
 // dZ = dH * GELU'(Z) elementwise (in place on dH)
@@ -268,25 +287,33 @@ __global__ void k_mlp_adam(size_t n, float* __restrict__ w, const float* __restr
 // --------------------------------------------------------------------------------
 // host
 // --------------------------------------------------------------------------------
-static void gemm(int M, int N, int K, const float* A, long sam, long sak, const float* B, long sbk, long sbn,
-                 float* C, int ldc, int epi, const float* bias, float* H, hipStream_t st) {
-    dim3 grid((N + kMT - 1) / kMT, (M + kMT - 1) / kMT);
-    // the staged kernel needs each operand contiguous along k or along its other index,
-    // with sizes and the other stride multiples of 4 floats and 16-byte aligned bases
-    const bool ak = sak == 1, bk = sbk == 1;
-    const long pa = ak ? sam : sak, pb = bk ? sbn : sbk;
-    const bool vec = (ak || sam == 1) && (bk || sbn == 1) && M % 4 == 0 && N % 4 == 0 && K % 4 == 0 &&
-                     pa % 4 == 0 && pb % 4 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0;
-    if (!vec)
-        k_mlp_gemm<<<grid, 256, 0, st>>>(M, N, K, A, sam, sak, B, sbk, sbn, C, ldc, epi, bias, H);
-    else if (ak && bk)
-        k_mlp_gemm4<true, true><<<grid, 256, 0, st>>>(M, N, K, A, sam, sak, B, sbk, sbn, C, ldc, epi, bias, H);
-    else if (ak)
-        k_mlp_gemm4<true, false><<<grid, 256, 0, st>>>(M, N, K, A, sam, sak, B, sbk, sbn, C, ldc, epi, bias, H);
-    else if (bk)
-        k_mlp_gemm4<false, true><<<grid, 256, 0, st>>>(M, N, K, A, sam, sak, B, sbk, sbn, C, ldc, epi, bias, H);
+static int div_up(int a, int b) { return (a + b - 1) / b; }
+
+// slices of K: products of few tiles split it until the chip has two workgroups per CU, as long as
+// a slice keeps two K steps and the partial sums' traffic (8 bytes per slice and output) stays
+// below the weights' (4 K bytes per column).  slices * M * N never exceeds kSplitWork floats.
+constexpr size_t kSplitWork = 512 * 64 * 64;
+static int gemm_slices(int M, int N, int K) {
+    const int tiles = div_up(M, 64) * div_up(N, 64);
+    if (tiles > 256) return 1;
+    return std::max(1, std::min({512 / tiles, K / (2 * kGK), K / (2 * M)}));
+}
+
+template <bool AK, bool BK>
+static void gemm(int M, int N, int K, const float* A, long pa, const float* B, long pb, float* C, int ldc, int epi,
+                 const float* bias, float* H, float* work, hipStream_t st) {
+    // 128 x 128 tiles where they fill the chip (4096 rows: 267 -> 170 us per forward product)
+    const bool large = (long long)div_up(M, 128) * div_up(N, 128) >= 256;
+    const int nk = div_up(K, kGK), want = large || !work ? 1 : gemm_slices(M, N, K);
+    const int per = div_up(nk, want), slices = div_up(nk, per);
+    if (large)
+        k_mlp_gemm<AK, BK, 128><<<dim3(div_up(N, 128), div_up(M, 128)), 256, 0, st>>>(M, N, K, A, pa, B, pb, C, ldc,
+                                                                                     epi, bias, H, nullptr, per);
     else
-        k_mlp_gemm4<false, false><<<grid, 256, 0, st>>>(M, N, K, A, sam, sak, B, sbk, sbn, C, ldc, epi, bias, H);
+        k_mlp_gemm<AK, BK, 64><<<dim3(div_up(N, 64), div_up(M, 64), slices), 256, 0, st>>>(
+            M, N, K, A, pa, B, pb, C, ldc, epi, bias, H, work, per);
+    if (slices > 1)
+        k_mlp_split_sum<<<dim3(div_up(N, 256), M), 256, 0, st>>>(M, N, slices, work, C, ldc, epi, bias, H);
     MPF_HIP(hipGetLastError());
 }
 
@@ -337,6 +364,14 @@ void Mlp::ensure_batch(int B) {
     dA.alloc((size_t)B * wmax);
     dB.alloc((size_t)B * wmax);
     part.alloc(1024);
+    if (!work.p) {
+        try {
+            work.alloc(kSplitWork);
+        } catch (const Error& e) {
+            if (e.code != MPF_ENOMEM) throw;   // no room: no product is split
+            (void)hipGetLastError();
+        }
+    }
 }
 
 void Mlp::forward(int B, const float* X, float* Y) {
@@ -346,7 +381,7 @@ void Mlp::forward(int B, const float* X, float* Y) {
     for (int l = 0; l < L; ++l) {
         const int ni = dims[l], no = dims[l + 1];
         const bool last = l == L - 1;
-        gemm(B, no, ni, in, ni, 1, W[l].p, no, 1, Z[l].p, no, last ? 2 : 1, b[l].p, H[l].p, st);
+        gemm<true, false>(B, no, ni, in, ni, W[l].p, no, Z[l].p, no, last ? 2 : 1, b[l].p, H[l].p, work.p, st);
         in = H[l].p;
     }
     x_in = X;
@@ -368,11 +403,11 @@ double Mlp::backward(const float* T) {
         const int ni = dims[l], no = dims[l + 1];
         const float* hin = l == 0 ? x_in : H[l - 1].p;
         // dW = H_in^T dZ ; db = column sums of dZ
-        gemm(ni, no, B, hin, 1, ni, dz, no, 1, gW[l].p, no, 0, nullptr, nullptr, st);
+        gemm<false, false>(ni, no, B, hin, ni, dz, no, gW[l].p, no, 0, nullptr, nullptr, work.p, st);
         k_mlp_colsum<<<(no + 63) / 64, 256, 0, st>>>(B, no, dz, gb[l].p);
         if (l > 0) {
             // dH_in = dZ W^T, then dZ_in = dH_in * GELU'(Z_in)
-            gemm(B, ni, no, dz, no, 1, W[l].p, 1, no, dh, ni, 0, nullptr, nullptr, st);
+            gemm<true, true>(B, ni, no, dz, no, W[l].p, no, dh, ni, 0, nullptr, nullptr, work.p, st);
             const size_t n = (size_t)B * ni;
             k_mlp_gelu_back<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(n, Z[l - 1].p, dh);
             std::swap(dz, dh);
