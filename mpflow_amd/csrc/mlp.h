@@ -21,6 +21,7 @@ struct Mlp {
     int64_t t = 0;                  // Adam steps taken
 
     Mlp(hipStream_t s, const std::vector<int>& d, uint64_t seed);
+    ~Mlp();
     void ensure_batch(int B);
     // Y (nullable) = network(X); X (B x in) stays caller-owned until backward
     void forward(int B, const float* X, float* Y);
@@ -29,6 +30,18 @@ struct Mlp {
     void adam(float lr, float b1, float b2, float eps);
     int64_t count() const;
     void params(int which, bool set, float* host);
+
+private:
+    struct Span {
+        char* dst;
+        const char* src;
+        size_t bytes;
+    };
+    static constexpr int kReadThreads = 8;
+    static constexpr size_t kReadMin = (size_t)48 << 20;
+    bool read(const std::vector<Span>& spans);   // false: too little, or no pinned memory
+    char* pinned = nullptr;         // a chunk per reading thread, from the first large read on
+    hipEvent_t copied[kReadThreads] = {};
 };
 
 }  // namespace mpf

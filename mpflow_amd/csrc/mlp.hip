@@ -7,7 +7,11 @@
 //   forward   Z = H W (+ b)        A = H  (batch x in),  B = W   (in x out)
 //   backward  dW = H^T dZ          A = H^T,              B = dZ
 //             dH = dZ W^T          A = dZ,               B = W^T
+#include <atomic>
 #include <cmath>
+#include <cstring>
+#include <system_error>
+#include <thread>
 
 #include "mlp.h"
 
@@ -438,11 +442,70 @@ int64_t Mlp::count() const {
     return n;
 }
 
+// Copies of device memory to pageable host memory by kReadThreads threads, a chunk at a time: each
+// enqueues its copy into a pinned buffer of its own, waits for it and moves it on.  Bound by the
+// first touch of the caller's memory, which the runtime's own copy does on one thread.  Measured
+// into new arrays: 120 MB 12.0 -> 3.5 ms (first read, with the pinned buffers made, 12.6 -> 4.7), 25
+// MB 1.5 -> 0.8 ms (2.4 -> 3.6), hence kReadMin: above it the first read is not slower either.
+bool Mlp::read(const std::vector<Span>& spans) {
+    constexpr size_t kChunk = (size_t)1 << 21;
+    std::vector<Span> chunks;
+    size_t total = 0;
+    for (const Span& s : spans)
+        for (size_t o = 0; o < s.bytes; o += kChunk) {
+            chunks.push_back(Span{s.dst + o, s.src + o, std::min(kChunk, s.bytes - o)});
+            total += chunks.back().bytes;
+        }
+    if (total < kReadMin) return false;
+    if (!pinned && hipHostMalloc((void**)&pinned, kReadThreads * kChunk, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        pinned = nullptr;
+        return false;
+    }
+    for (auto& e : copied)
+        if (!e) MPF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    int device = 0;
+    MPF_HIP(hipGetDevice(&device));
+    std::atomic<size_t> next{0};
+    std::atomic<int> failed{(int)hipSuccess};
+    auto work = [&](int t) {
+        char* buf = pinned + t * kChunk;
+        hipError_t e = hipSetDevice(device);
+        while (e == hipSuccess) {
+            const size_t c = next.fetch_add(1);
+            if (c >= chunks.size()) return;
+            e = hipMemcpyAsync(buf, chunks[c].src, chunks[c].bytes, hipMemcpyDeviceToHost, st);
+            if (e == hipSuccess) e = hipEventRecord(copied[t], st);
+            if (e == hipSuccess) e = hipEventSynchronize(copied[t]);
+            if (e == hipSuccess) std::memcpy(chunks[c].dst, buf, chunks[c].bytes);
+        }
+        failed = (int)e;
+    };
+    std::vector<std::thread> threads;
+    threads.reserve(kReadThreads);
+    try {
+        for (int t = 1; t < kReadThreads; ++t) threads.emplace_back(work, t);
+    } catch (const std::system_error&) {
+        // the threads there are share the chunks
+    }
+    work(0);
+    for (auto& t : threads) t.join();
+    MPF_HIP((hipError_t)failed.load());
+    return true;
+}
+
+Mlp::~Mlp() {
+    for (auto& e : copied)
+        if (e) (void)hipEventDestroy(e);
+    if (pinned) (void)hipHostFree(pinned);
+}
+
 // flat order: W_0, b_0, W_1, b_1, ... (W row-major in x out)
 void Mlp::params(int which, bool set, float* host) {
     MPF_REQUIRE(which == 0 || which == 1, "mlp: which must be 0 (parameters) or 1 (gradients)");
     MPF_REQUIRE(!(set && which == 1), "mlp: gradients are read-only");
     size_t off = 0;
+    std::vector<Span> spans;
     for (int l = 0; l < L; ++l) {
         const size_t nw = (size_t)dims[l] * dims[l + 1];
         DBuf<float>& w = which == 0 ? W[l] : gW[l];
@@ -451,11 +514,13 @@ void Mlp::params(int which, bool set, float* host) {
             w.upload(host + off, nw, st);
             bb.upload(host + off + nw, dims[l + 1], st);
         } else {
-            MPF_HIP(hipMemcpyAsync(host + off, w.p, nw * sizeof(float), hipMemcpyDeviceToHost, st));
-            MPF_HIP(hipMemcpyAsync(host + off + nw, bb.p, dims[l + 1] * sizeof(float), hipMemcpyDeviceToHost, st));
+            spans.push_back(Span{(char*)(host + off), (const char*)w.p, nw * sizeof(float)});
+            spans.push_back(Span{(char*)(host + off + nw), (const char*)bb.p, dims[l + 1] * sizeof(float)});
         }
         off += nw + dims[l + 1];
     }
+    if (!set && read(spans)) return;
+    for (const Span& s : spans) MPF_HIP(hipMemcpyAsync(s.dst, s.src, s.bytes, hipMemcpyDeviceToHost, st));
     MPF_HIP(hipStreamSynchronize(st));
 }
 

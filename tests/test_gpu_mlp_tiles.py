@@ -39,3 +39,15 @@ def test_mlp_products_at_tile_edges(gpu_ctx, dims, batch):
     assert ey < 2e-3
     assert abs(loss - lo) < 1e-3 * lo
     assert eg < 3e-3
+
+
+@pytest.mark.parametrize("dims", [[3001, 4099, 33], [33, 4099, 3001], [700, 900, 9]])
+def test_mlp_parameters_read_back_as_set(gpu_ctx, dims):
+    """Above and below the size that is read by several threads, with ragged last chunks."""
+    from mpflow_amd.learned import Mlp
+    print("case: mlp read back", dims, flush=True)
+    net = Mlp(dims, seed=1, ctx=gpu_ctx)
+    w = np.random.default_rng(3).standard_normal(net.n_params).astype(np.float32)
+    net.set_params(w)
+    for _ in range(2):
+        np.testing.assert_array_equal(net.params(), w)
