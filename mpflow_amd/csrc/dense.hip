@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "chip_dev.h"
 #include "dense.h"
 
 namespace mpf {
@@ -554,52 +555,84 @@ __global__ void __launch_bounds__(256) k_gemv_t4(int rows, int cols, const float
 // partial[slab][r] = sum_{c in slab} A[r + c*lda] x[c]
 constexpr int kNSlab = 256;
 
-// partial[slab][r] = sum_{c in slab} A[r + c*lda] (sum_r' A[r' + c*lda] x[r']): A (A^T x)
-// in one pass over A (rows <= 1024, rows, lda and strideA multiples of 4).  A block owns
-// the sw columns of its slab, kTnCols at a time: thread t loads rows 4t..4t+3 of each
-// column (128-bit), the block reduces the column dots in FP64, and the same registers
-// then give the rows' partial sums, so every element of A is read once.
-constexpr int kTnCols = 8;
-__global__ void __launch_bounds__(256) k_gemv_tn_part(int rows, int cols, const float* __restrict__ A, int lda,
-                                                      size_t strideA, const double* __restrict__ x,
-                                                      size_t stridex, double* __restrict__ part, int sw) {
-    const int slab = blockIdx.x, b = blockIdx.y;
+// TN: out[b][slab][r] = sum_{c in slab} A[r + c*lda] (sum_r' A[r' + c*lda] x_b[r']): A (A^T x) in
+// one pass over A; else out[b * strideout + c] = sum_r A[r + c*lda] x_b[r] (rows <= 1024, rows, lda
+// and strideA multiples of 4).  A block owns the sw columns of its slab, kTnCols at a time:
+// thread t loads rows 4t..4t+3 of each column (128-bit), the block reduces the column dots in
+// FP64, and the same registers then give the rows' partial sums, so every element of A is
+// read once for the block's F frames.
+//
+// F = 1: one A per frame, bound by reading it.  F = 4: one A for all frames (strideA 0), which is
+// then read and converted once per four frames; bound by the FP64 products and the dots' sums,
+// which stay on the VALU.  Measured (MI355X), 64 frames, one 1024 x 9600 A: A A^T x 463 -> 109 us,
+// A^T x 293 -> 85 us; one A per frame 639 -> 447 us (5.6 TB/s).
+constexpr int kTnCols = 8, kTnFrames = 4;
+template <int F, bool TN>
+__global__ void __launch_bounds__(256, 2) k_gemv_tn_part(int rows, int cols, const float* __restrict__ A, int lda,
+                                                         size_t strideA, const double* __restrict__ x, size_t stridex,
+                                                         double* __restrict__ out, size_t strideout, int sw, int batch) {
+    const int slab = blockIdx.x, b0 = blockIdx.y * F;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int r0 = 4 * threadIdx.x;
+    const int r0 = 4 * threadIdx.x, ra = min(r0, rows - 4);
     const bool act = r0 < rows;
-    const float* a = A + b * strideA;
-    double xv[4] = {0.0, 0.0, 0.0, 0.0};
-    if (act)
-        for (int i = 0; i < 4; ++i) xv[i] = x[b * stridex + r0 + i];
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    __shared__ double red[4][kTnCols];
+    const float* a = A + (F == 1 ? b0 * strideA : 0) + ra;
+    double xv[F][4], acc[F][4];
+#pragma unroll
+    for (int f = 0; f < F; ++f)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const double v = x[(size_t)min(b0 + f, batch - 1) * stridex + ra + i];
+            xv[f][i] = act ? v : 0.0;
+            acc[f][i] = 0.0;
+        }
+    __shared__ double red[F][4][kTnCols];
+    __shared__ double tot[F][kTnCols];
     const int c0 = slab * sw, c1 = min(cols, c0 + sw);
     for (int cb = c0; cb < c1; cb += kTnCols) {
         float4 p[kTnCols];
 #pragma unroll
+        for (int j = 0; j < kTnCols; ++j) p[j] = *(const float4*)(a + (size_t)min(cb + j, cols - 1) * lda);
+#pragma unroll
         for (int j = 0; j < kTnCols; ++j)
-            p[j] = (act && cb + j < c1) ? *(const float4*)(a + (size_t)(cb + j) * lda + r0)
-                                        : make_float4(0.f, 0.f, 0.f, 0.f);
-        double d[kTnCols];
+            if (!act || cb + j >= c1) p[j] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-        for (int j = 0; j < kTnCols; ++j) {
-            d[j] = (double)p[j].x * xv[0] + (double)p[j].y * xv[1] + (double)p[j].z * xv[2] + (double)p[j].w * xv[3];
-            for (int off = 32; off > 0; off >>= 1) d[j] += __shfl_xor(d[j], off, 64);
-        }
-        if (lane == 0)
+        for (int f = 0; f < F; ++f)
 #pragma unroll
-            for (int j = 0; j < kTnCols; ++j) red[wave][j] = d[j];
+            for (int h = 0; h < 2; ++h) {
+                double d[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float4 q = p[4 * h + j];
+                    d[j] = (double)q.x * xv[f][0] + (double)q.y * xv[f][1] + (double)q.z * xv[f][2] + (double)q.w * xv[f][3];
+                }
+                const double s = wave_sum<4>(d, lane);
+                if (lane < 4) red[f][wave][4 * h + col_of<4>(lane)] = s;
+            }
         __syncthreads();
-#pragma unroll
-        for (int j = 0; j < kTnCols; ++j) {
-            const double v = (red[0][j] + red[1][j]) + (red[2][j] + red[3][j]);
-            acc[0] += (double)p[j].x * v; acc[1] += (double)p[j].y * v;
-            acc[2] += (double)p[j].z * v; acc[3] += (double)p[j].w * v;
+        if ((int)threadIdx.x < F * kTnCols) {
+            const int f = threadIdx.x / kTnCols, j = threadIdx.x % kTnCols;
+            const double v = (red[f][0][j] + red[f][1][j]) + (red[f][2][j] + red[f][3][j]);
+            if constexpr (TN) tot[f][j] = v;
+            else if (b0 + f < batch && cb + j < c1) out[(size_t)(b0 + f) * strideout + cb + j] = v;
         }
-        __syncthreads();   // red is rewritten by the next group of columns
+        __syncthreads();       // red is rewritten by the next columns; tot after their first barrier
+        if constexpr (TN)
+#pragma unroll
+            for (int f = 0; f < F; ++f)
+#pragma unroll
+                for (int j = 0; j < kTnCols; ++j) {
+                    const double v = tot[f][j];
+                    acc[f][0] += (double)p[j].x * v; acc[f][1] += (double)p[j].y * v;
+                    acc[f][2] += (double)p[j].z * v; acc[f][3] += (double)p[j].w * v;
+                }
     }
-    if (act)
-        for (int i = 0; i < 4; ++i) part[((size_t)b * gridDim.x + slab) * rows + r0 + i] = acc[i];
+    if (TN && act)
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+            if (b0 + f < batch)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    out[((size_t)(b0 + f) * gridDim.x + slab) * rows + r0 + i] = acc[f][i];
 }
 __global__ void __launch_bounds__(256) k_gemv_n_part(int rows, int cols, const float* __restrict__ A, int lda,
                                                      size_t strideA, const double* __restrict__ x, size_t stridex,
@@ -1119,8 +1152,30 @@ void launch_gram(const float* A, int trans, int n, int nk, int lda, float* G, vo
     check_launch();
 }
 
+bool gemv_tn_applies(int rows, int lda, size_t strideA, const float* A) {
+    return rows > 0 && rows <= 1024 && rows % 4 == 0 && lda % 4 == 0 && strideA % 4 == 0 && ((uintptr_t)A & 15) == 0;
+}
+
+// columns per block: kNSlab (512 with four frames per block), fewer where that leaves the chip
+// idle (below 512 blocks; one frame of 9600 columns: 38 blocks and 126 us before, 400 and 17 us now)
+static int gemv_tn_slab(int cols, int groups, int frames) {
+    const int want = (512 + groups - 1) / groups;
+    const int sw = round_up((cols + want - 1) / want, kTnCols);
+    return std::min(frames > 1 ? 2 * kNSlab : kNSlab, sw);
+}
+// frames per block: four where they share A
+static int gemv_tn_frames(size_t strideA, int batch) { return strideA == 0 && batch >= kTnFrames ? kTnFrames : 1; }
+
 void launch_gemv_t(int rows, int cols, const float* A, int lda, size_t strideA, const double* x,
                    size_t stridex, double* y, size_t stridey, int batch, hipStream_t st) {
+    const int frames = gemv_tn_frames(strideA, batch), groups = (batch + frames - 1) / frames;
+    if (frames > 1 && gemv_tn_applies(rows, lda, strideA, A)) {
+        const int sw = gemv_tn_slab(cols, groups, frames);
+        k_gemv_tn_part<kTnFrames, false><<<dim3((cols + sw - 1) / sw, groups), 256, 0, st>>>(
+            rows, cols, A, lda, strideA, x, stridex, y, stridey, sw, batch);
+        check_launch();
+        return;
+    }
     dim3 grid((cols + 3) / 4, batch);
     if (rows % 4 == 0 && lda % 4 == 0 && strideA % 4 == 0 && ((uintptr_t)A & 15) == 0)
         k_gemv_t4<<<grid, 256, 0, st>>>(rows, cols, A, lda, strideA, x, stridex, y, stridey);
@@ -1129,29 +1184,28 @@ void launch_gemv_t(int rows, int cols, const float* A, int lda, size_t strideA, 
     check_launch();
 }
 
-bool gemv_tn_applies(int rows, int lda, size_t strideA, const float* A) {
-    return rows > 0 && rows <= 1024 && rows % 4 == 0 && lda % 4 == 0 && strideA % 4 == 0 && ((uintptr_t)A & 15) == 0;
-}
-
-// columns per block: kNSlab, fewer where that leaves the chip idle (below 512 blocks; one frame of
-// 9600 columns: 38 blocks and 126 us before, 400 and 17 us now)
-static int gemv_tn_slab(int cols, int batch) {
-    const int want = (512 + batch - 1) / batch;
-    const int sw = round_up((cols + want - 1) / want, kTnCols);
-    return std::min(kNSlab, sw);
-}
-
 size_t gemv_tn_workspace(int rows, int cols, int batch) {
-    const int sw = gemv_tn_slab(cols, batch);
-    return (size_t)batch * ((cols + sw - 1) / sw) * rows * sizeof(double);
+    size_t slabs = 0;              // of all frames, the most that any number up to batch takes
+    for (int n = 1; n <= batch; ++n)
+        for (int f : {1, kTnFrames}) {
+            const int sw = gemv_tn_slab(cols, (n + f - 1) / f, f);
+            slabs = std::max(slabs, (size_t)n * ((cols + sw - 1) / sw));
+        }
+    return slabs * rows * sizeof(double);
 }
 
 void launch_gemv_tn(int rows, int cols, const float* A, int lda, size_t strideA, const double* x,
                     size_t stridex, double shift, const double* rhs, size_t striderhs, double* out,
                     size_t strideout, int batch, double* work, hipStream_t st) {
     MPF_REQUIRE(gemv_tn_applies(rows, lda, strideA, A), "gemv_tn: rows <= 1024, multiples of 4, aligned A");
-    const int sw = gemv_tn_slab(cols, batch), nslab = (cols + sw - 1) / sw;
-    k_gemv_tn_part<<<dim3(nslab, batch), 256, 0, st>>>(rows, cols, A, lda, strideA, x, stridex, work, sw);
+    const int frames = gemv_tn_frames(strideA, batch), groups = (batch + frames - 1) / frames;
+    const int sw = gemv_tn_slab(cols, groups, frames), nslab = (cols + sw - 1) / sw;
+    if (frames > 1)
+        k_gemv_tn_part<kTnFrames, true><<<dim3(nslab, groups), 256, 0, st>>>(rows, cols, A, lda, strideA, x, stridex,
+                                                                            work, 0, sw, batch);
+    else
+        k_gemv_tn_part<1, true><<<dim3(nslab, groups), 256, 0, st>>>(rows, cols, A, lda, strideA, x, stridex, work, 0,
+                                                                    sw, batch);
     dim3 g2((rows + 15) / 16, batch);
     k_gemv_n_reduce<<<g2, 256, 0, st>>>(rows, nslab, work, shift, x, stridex, rhs, striderhs, out, strideout);
     check_launch();
