@@ -16,7 +16,7 @@
 // Measured (MI355X, whole calls): one 2D forward solve of 817 nodes, 168 steps, 4.60 -> 0.42
 // ms (1.02 ms with the deciding group of the reference rule run before the others); 64 frames x 5
 // harmonics of 4921 nodes to 1e-6 18.1 -> 5.5 ms (1024 threads 7.2 ms); a caller's 4921-row
-// matrix with 32 columns 2.02 -> 0.54 ms.
+// matrix with 32 columns 2.02 -> 0.56 ms.
 //
 // The recurrences, the FP64 scalars, the stop rules and the breakdown rules are those of the
 // streaming kernels (sparse.hip); sums run in a fixed order.

@@ -57,7 +57,8 @@ void launch_gram(const float* A, int trans, int n, int nk, int lda, float* G, vo
 void launch_gemv_t(int rows, int cols, const float* A, int lda, size_t strideA, const double* x,
                    size_t stridex, double* y, size_t stridey, int batch, hipStream_t st);
 size_t gemv_n_workspace(int rows, int cols, int batch);
-// out = rhs - (A A^T x + shift x) in one pass over A (work: gemv_tn_workspace bytes);
+// out = rhs - (A A^T x + shift x) in one pass over A (work: gemv_tn_workspace bytes, which
+// serve any number of frames up to batch);
 // applies for rows <= 1024 with rows, lda, strideA multiples of 4 and A 16-byte aligned
 size_t gemv_tn_workspace(int rows, int cols, int batch);
 bool gemv_tn_applies(int rows, int lda, size_t strideA, const float* A);
