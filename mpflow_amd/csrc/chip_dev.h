@@ -42,6 +42,20 @@ __device__ __forceinline__ double add_halves(double v) {
     const v2u lo = swap_halves<HALF>((uint32_t)b), hi = swap_halves<HALF>((uint32_t)(b >> 32));
     return __longlong_as_double(((uint64_t)hi[0] << 32) | lo[0]) + __longlong_as_double(((uint64_t)hi[1] << 32) | lo[1]);
 }
+// both of them, apart: the lower half's value first
+template <int HALF>
+__device__ __forceinline__ void both_halves(double v, double (&o)[2]) {
+    const uint64_t b = __double_as_longlong(v);
+    const v2u lo = swap_halves<HALF>((uint32_t)b), hi = swap_halves<HALF>((uint32_t)(b >> 32));
+    o[0] = __longlong_as_double(((uint64_t)hi[0] << 32) | lo[0]);
+    o[1] = __longlong_as_double(((uint64_t)hi[1] << 32) | lo[1]);
+}
+// LDS accesses of one wavefront made visible to its own lanes
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 // sum over the lanes that agree in l mod 4
 template <class T>
 __device__ __forceinline__ T add_quads(T v) {

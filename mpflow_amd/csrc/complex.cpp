@@ -46,8 +46,7 @@ struct ComplexModel::Impl {
     // on-chip solves (chip_complex.hip)
     bool chip_tried = false, chip_ok = false;
     ChipShape shape;
-    DBuf<uint8_t> gw, tpos, octs;
-    DBuf<uint16_t> crow, cpos;
+    DBuf<uint8_t> octs;
     DBuf<uint4> cid;
     DBuf<float4> cval;
     DBuf<int4> chip_items;
@@ -84,15 +83,14 @@ bool ComplexModel::Impl::ensure_chip() {
     if (chip_tried) return chip_ok;
     chip_tried = true;
     const int np = S.np, W = S.wpad;
-    if (np > kCChipMaxRows || W > kChipMaxWidth) return false;
+    if (np > kCChipMaxRows || W > kChipMaxWidth || Rq < kCChipMinLanes) return false;
     hipStream_t st0 = ctx->stream;
     shape = c_chip_shape(np, (long long)frames * S.C * S.Ru);
     const int groups = Rq / shape.G, total = njs * groups;
     try {
-        gw.alloc(S.group_width.size()); gw.upload(S.group_width.data(), S.group_width.size(), st0);
-        tpos.alloc(np); tpos.upload(S.tile_pos.data(), np, st0);
-        crow.alloc(np);
-        cpos.alloc(np);
+        DBuf<uint8_t> gw(S.group_width.size());
+        DBuf<uint16_t> crow(np), cpos(np);          // row order: the identity
+        gw.upload(S.group_width.data(), S.group_width.size(), st0);
         octs.alloc(np / 64);
         cid.alloc((size_t)W / 8 * np);
         const size_t nval = (size_t)S.C * (W / 2) * np;
@@ -116,12 +114,12 @@ bool ComplexModel::Impl::ensure_chip() {
         }
         progress.alloc(total);
         MPF_HIP(hipHostMalloc((void**)&h_gst, sizeof(int2) * total, hipHostMallocDefault));
-        launch_chip_order(np, tpos.p, crow.p, cpos.p, st0);
+        launch_chip_order(np, nullptr, crow.p, cpos.p, st0);
         launch_chip_ids(np, W, ids.p, gw.p, crow.p, cpos.p, cid.p, octs.p, st0);
         MPF_HIP(hipStreamSynchronize(st0));
         for (int f = 0; f < frames; ++f) {
             CJob& J = hjobs[f];
-            J.crow = crow.p; J.cid = cid.p; J.cocts = octs.p;
+            J.cid = cid.p; J.cocts = octs.p;
             J.cval = cval.p + nval * f;
         }
     } catch (const Error& e) {
@@ -138,10 +136,10 @@ void ComplexModel::Impl::run_chip() {
     hipStream_t st0 = ctx->stream;
     const int groups = Rq / shape.G, total = njs * groups;
     launch_c_chip_pack(jobs.p, js.p, njs, S.np, progress.p, total, st0);
-    launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, gst[1].p, gst[0].p, progress.p, 0, st0);
+    launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, Rq, gst[1].p, gst[0].p, progress.p, 0, st0);
     int in = 0;
     for (bool open = true; open;) {
-        launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, gst[in].p, gst[in ^ 1].p, progress.p, 1,
+        launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, Rq, gst[in].p, gst[in ^ 1].p, progress.p, 1,
                       st0);
         in ^= 1;
         MPF_HIP(hipMemcpyAsync(h_gst, gst[in].p, sizeof(int2) * total, hipMemcpyDeviceToHost, st0));

@@ -40,9 +40,9 @@ struct CJob {
     int* st;                     // [C][4]: live, steps, capped, -
     const float2* gamma;         // [E]
     const int32_t* ctb_off; const int32_t* ctb_elem; const double* ctb_k; const double* ctb_m;
-    // on-chip solves (chip_complex.hip): chip order, 16-bit column positions, 8-slot groups in
-    // use per 64 positions (as jobs.h) and the values S + alpha_c R, [C][width / 8][4][np]
-    const uint16_t* crow; const uint4* cid; const uint8_t* cocts; float4* cval;
+    // on-chip solves (chip_complex.hip): 16-bit column ids, 8-slot groups in use per 64 rows (as
+    // jobs.h, in row order) and the values S + alpha_c R, [C][width / 8][4][np]
+    const uint4* cid; const uint8_t* cocts; float4* cval;
 };
 
 struct CMeasDev {
@@ -60,14 +60,29 @@ struct CJacDev {
     float weight[kMaxSlices];
 };
 
+// The products of the conjugate gradients, with the rounded and the fused half of each part spelled out: the
+// streamed and the on-chip solver take the same steps to the same bits whatever the compiler would
+// fuse.  a b, |a|^2, and one ELL entry a x added to a row (the imaginary part's fused half differs
+// between even and odd lanes)
+__device__ __forceinline__ zd zprod(zd a, zd b) { return zd{fma(a.x, b.x, -(a.y * b.y)), fma(a.y, b.x, a.x * b.y)}; }
+__device__ __forceinline__ double znorm2(zd a) { return fma(a.x, a.x, a.y * a.y); }
+__device__ __forceinline__ void add_entry(bool odd, float& re, float& im, float ar, float ai, float xr, float xi) {
+    re += fmaf(ar, xr, -(ai * xi));
+    im += odd ? fmaf(ai, xr, ar * xi) : fmaf(ar, xi, ai * xr);
+}
+// one term a . b of a Krylov dot product: a conj(b) (the reference's) or a b (COCG)
+__device__ __forceinline__ zd zdot(bool herm, zd a, zd b) { return zprod(a, herm ? zconj(b) : b); }
+
 void launch_c_assemble(const CJob* d_jobs, const int4* d_items, int nitems, hipStream_t st);
 void launch_c_dinv(const CJob* d_jobs, const int4* d_tiles, int ntiles, hipStream_t st);
 void launch_c_init(const CJob* d_jobs, const int4* d_tiles, int ntiles, const int2* d_js, int njs, hipStream_t st);
 // one CG iteration over the listed tiles of live (frame, slice) pairs
 void launch_c_iter(const CJob* d_jobs, const int4* d_tiles, int ntiles, const int2* d_js, int njs, int* d_live,
                    hipStream_t st);
-// whole solves on chip: the meshes whose p and inverse diagonal fit one CU's LDS
-constexpr int kCChipMaxRows = 8192;
+// whole solves on chip: the meshes whose p and inverse diagonal fit one CU's LDS.  Lane strides
+// below 8 (at most four right-hand sides) are streamed: the tile sums that the streamed kernels add in
+// one thread would be chains of 128 and 256
+constexpr int kCChipMaxRows = 8192, kCChipMinLanes = 8;
 // G complex lanes per workgroup, K rows per thread, for np padded rows when a solve has `lanes`
 // (frame, harmonic, column) triples
 ChipShape c_chip_shape(int np, long long lanes);
@@ -75,8 +90,8 @@ void launch_c_chip_pack(const CJob* d_jobs, const int2* d_js, int njs, int np, i
                         hipStream_t st);
 // one phase over `n` items (frame, slice, lane group, index of the pair's first group state), as
 // launch_chip
-void launch_c_chip(const CJob* d_jobs, const int4* d_items, int n, const ChipShape& c, int width, const int2* gin,
-                   int2* gout, int* progress, int phase, hipStream_t st);
+void launch_c_chip(const CJob* d_jobs, const int4* d_items, int n, const ChipShape& c, int width, int Rq,
+                   const int2* gin, int2* gout, int* progress, int phase, hipStream_t st);
 void launch_c_voltages(const CJob* d_jobs, int njobs, const CMeasDev& md, float2* U32, zd* U64, hipStream_t st);
 void launch_c_jacobian(const CJob* d_jobs, int njobs, const CJacDev& jd, float2* J, hipStream_t st);
 // G_b = J_b J_b^T + shift I (complex symmetric, FP64 sums of the FP32 J, both triangles);

@@ -17,8 +17,7 @@ constexpr int kCBlock = 256;   // threads per block of the tile kernels (one 256
 constexpr double kLn10 = 2.302585092994046;
 
 __device__ __forceinline__ bool c_live(const CJob& J, int s) { return J.st[s * 4] != 0; }
-// one term a . b of a Krylov dot product: a conj(b) (reference) or a b (COCG)
-__device__ __forceinline__ zd c_dot(const CJob& J, zd a, zd b) { return J.herm ? a * zconj(b) : a * b; }
+__device__ __forceinline__ zd c_dot(const CJob& J, zd a, zd b) { return zdot(J.herm != 0, a, b); }
 __device__ __forceinline__ size_t c_idx(const CJob& J, int s, int row, int lane) {
     return ((size_t)s * J.np + row) * J.Rq + lane;
 }
@@ -107,7 +106,7 @@ __global__ void __launch_bounds__(kCBlock) k_c_init(const CJob* __restrict__ job
         for (int h = 0; h < 2; ++h) {
             const int lane = 2 * ly.l2 + h;
             const double b = lane < J.Ru ? (double)J.beta[s] * J.F[(size_t)row * J.Fp + lane] : 0.0;
-            const zd z = d * zmake(b);
+            const zd z = zprod(d, zmake(b));
             xs[h] = make_float2(0.0f, 0.0f);
             rs[h] = make_float2((float)b, 0.0f);
             zs[h] = fz(z);
@@ -145,8 +144,8 @@ __global__ void __launch_bounds__(kCBlock) k_c_spmv(const CJob* __restrict__ job
             const float2 sv = J.sv[e], rv = J.rv[e];
             const float ar = sv.x + al * rv.x, ai = sv.y + al * rv.y;
             const float4 x = *reinterpret_cast<const float4*>(P + (size_t)id * J.Rq + 2 * ly.l2);
-            a0r += ar * x.x - ai * x.y; a0i += ar * x.y + ai * x.x;
-            a1r += ar * x.z - ai * x.w; a1i += ar * x.w + ai * x.z;
+            add_entry(false, a0r, a0i, ar, ai, x.x, x.y);
+            add_entry(true, a1r, a1i, ar, ai, x.z, x.w);
         }
         const size_t i = c_idx(J, s, row, 2 * ly.l2);
         *reinterpret_cast<float4*>(J.q + i) = make_float4(a0r, a0i, a1r, a1i);
@@ -202,13 +201,13 @@ __global__ void __launch_bounds__(kCBlock) k_c_update(const CJob* __restrict__ j
                 xo[h] = make_float2(0.0f, 0.0f);
             } else {
                 const zd qf = (dc && row < J.n) ? qv[h] + ps[h] : qv[h];
-                ro[h] = fz(rv[h] - al[h] * qf);
-                xo[h] = fz(xv[h] + al[h] * pv[h]);
+                ro[h] = fz(rv[h] - zprod(qf, al[h]));
+                xo[h] = fz(xv[h] + zprod(al[h], pv[h]));
             }
             const zd rn = zf(ro[h]);
-            const zd z = zf(fz(d * rn));
+            const zd z = zf(fz(zprod(d, rn)));
             v[0][h] += c_dot(J, rn, z);
-            v[1][h] += zmake(zabs2(rn));
+            v[1][h] += zmake(znorm2(rn));
         }
         *reinterpret_cast<float4*>(J.r + i) = make_float4(ro[0].x, ro[0].y, ro[1].x, ro[1].y);
         *reinterpret_cast<float4*>(J.x + i) = make_float4(xo[0].x, xo[0].y, xo[1].x, xo[1].y);
@@ -267,7 +266,7 @@ __global__ void __launch_bounds__(64) k_c_state(const CJob* __restrict__ jobs, c
         if (J.rule == MPF_STOP_REFERENCE) {
             const zd rho = c_sc(J, ZF_RHON, s)[J.col0];
             const double bb = c_sc(J, ZF_BB, s)[J.col0].x;
-            const double crit = sqrt(sqrt(zabs2(rho)) / bb);
+            const double crit = sqrt(sqrt(znorm2(rho)) / bb);
             stop = !(crit >= 1.1920928955078125e-07);
         } else {
             stop = !unconv;
@@ -309,8 +308,8 @@ __global__ void __launch_bounds__(kCBlock) k_c_pupdate(const CJob* __restrict__ 
         float2 po[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const zd z = zf(fz(d * rv[h]));
-            po[h] = zero[h] ? make_float2(0.0f, 0.0f) : fz(z + be[h] * pv[h]);
+            const zd z = zf(fz(zprod(d, rv[h])));
+            po[h] = zero[h] ? make_float2(0.0f, 0.0f) : fz(z + zprod(be[h], pv[h]));
         }
         *reinterpret_cast<float4*>(J.p + i) = make_float4(po[0].x, po[0].y, po[1].x, po[1].y);
     }

@@ -51,13 +51,6 @@ __global__ void __launch_bounds__(256) k_voltages(const JobDev* __restrict__ job
 constexpr int kJacMaxRows = 4096;   // Dp * Mp <= 64 * 64
 constexpr int kJacWaves = 4;        // elements per 256-thread block
 
-// LDS writes of a wavefront made visible to its own lanes
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // PER: column rows per lane (mrows <= 64 PER); FIXEDM: Mp divides 64, so a lane's
 // measurement column is the same for all of its rows; K: nodes per element (3 or 6), a
 // compile-time constant so that the per-node loops unroll and the lane's column of T

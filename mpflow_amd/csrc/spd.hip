@@ -20,6 +20,7 @@
 // first form (whole-tile eliminations, operands loaded one by one), which matched the former
 // factorisation; one solve 1140 -> 16 us, 64 solves 1610 -> 153 us (3.5 TB/s), 64 against one
 // factor 1120 -> 100 us.
+#include "chip_dev.h"
 #include "dense.h"
 
 namespace mpf {
@@ -103,13 +104,6 @@ __device__ __forceinline__ void tile_put(SpdTile& t, const v4d (&acc)[2][2]) {
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) t[wj + 16 * j + o][wi + 16 * i + 4 * v + q] = acc[i][j][v];
-}
-
-// LDS accesses of one wavefront made visible to its own lanes
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // L L^T of the 16 x 16 diagonal block of t at o and its inverse into w's, by one wavefront: lane

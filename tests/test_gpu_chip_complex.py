@@ -65,3 +65,55 @@ def test_on_chip_complex_matches_streamed(gpu_ctx, shape):
         assert sa.not_converged == sb.not_converged
         assert err < 4e-5
         assert abs(sa.steps - sb.steps) <= 0.1 * sb.steps + 4
+
+
+# the same and each lane stride of the sums (rows per pass of the streamed kernels: 64, 32, 16, 8):
+# rings, electrodes, harmonics, P2, frames, measurement pattern apart from the drive
+ORDER = [
+    (5, 8, 1, False, 1, False),       # stride 8: one tile
+    (22, 8, 2, False, 3, False),      # stride 8
+    (16, 16, 2, False, 3, False),     # stride 16: four tiles
+    (20, 16, 3, False, 40, False),    # stride 16, more groups than CUs
+    (14, 16, 2, True, 2, False),      # stride 16, rows of 9 and 19 entries
+    (18, 20, 3, False, 2, False),     # stride 32, empty lanes
+    (30, 32, 1, False, 20, False),    # stride 32, two lanes, two tiles per wavefront
+    (29, 16, 1, False, 1, False),     # 11 tiles: the last five wavefronts have one
+    (20, 32, 2, False, 2, True),      # stride 64
+    (25, 32, 1, True, 2, True),       # stride 64, P2, 30 tiles: 1024 threads
+    (30, 32, 1, False, 6, True),      # stride 64, two lanes
+    (30, 8, 2, False, 20, False),     # stride 8, two lanes
+    (51, 16, 1, False, 2, False),     # 32 tiles: 1024 threads
+    (45, 12, 1, False, 1, False),     # 25 tiles: some wavefronts with one tile
+]
+
+
+@pytest.mark.parametrize("shape", ORDER, ids=lambda s: "-".join(map(str, s)))
+def test_on_chip_complex_takes_the_streamed_steps(gpu_ctx, shape):
+    """The sums run in the streamed kernels' order: the same steps and the same bits, converged or
+    not, and so the streamed solver's error on every input."""
+    import torch
+    from mpflow_amd import capi
+    from mpflow_amd.eit import EIT
+    from oracle.eit_oracle import ComplexEITOracle
+    rings, L, C, p2, frames, apart = shape
+    p = make_problem(rings, L, 1.6 / L, C=C, height=1.0 if C == 1 else 0.4, port_height=1.0 if C == 1 else 0.1, p2=p2)
+    if apart:
+        p["meas"] = np.eye(L) - np.roll(np.eye(L), 3, axis=0)
+    args = (p["nodes"], p["elements"], p["boundary"], p["ports"], p["drive"], p["meas"], p["current"], 1.0, C,
+            p["height"], p["port_height"])
+    eit = EIT(*args, frames=frames, ctx=gpu_ctx, complex_gamma=True)
+    rng = np.random.default_rng(19)
+    n = (frames, p["elements"].shape[0])
+    for imag in (0.1, 1.0):
+        g = torch.tensor(rng.uniform(0.3, 3.0, n) + 1j * imag * rng.uniform(-1.0, 1.0, n), dtype=torch.complex64)
+        for kw in (dict(), dict(complex_hermitian=1, max_iter=300), dict(max_iter=9),
+                   dict(stop_rule=capi.MPF_STOP_TOLERANCE, tol=1e-6, max_iter=4000)):
+            print("case: on-chip complex bits %s imag %g %s" % (shape, imag, kw), flush=True)
+            a, sa = _solve(eit, g, gpu_ctx, False, **kw)
+            b, sb = _solve(eit, g, gpu_ctx, True, **kw)
+            assert (sa.steps, sa.max_steps, sa.not_converged) == (sb.steps, sb.max_steps, sb.not_converged)
+            assert np.isfinite(b).all() and np.array_equal(a, b)
+    # the last solve (tolerance 1e-6) against the FP64 oracle, with the bound of its own comparison
+    if eit.N < 3000:
+        u = ComplexEITOracle(*args).solve(g[0].numpy().astype(np.complex128))[0]
+        assert np.abs(a[0] - u).max() / np.abs(u).max() < 2e-5
