@@ -239,8 +239,10 @@ typedef struct mpf_solve_opts {
                                      frame's conductivity; several times fewer iterations on
                                      large meshes.  Above 20480 unknowns D^-1 is replaced by
                                      D^-1/2 B D^-1/2 with B the inverses of the 32-node diagonal
-                                     blocks of the unit-diagonal matrix at sigma = 1.  Models
-                                     above 512 tiles (131072 unknowns) fall back to Jacobi. */
+                                     blocks of the unit-diagonal matrix at sigma = 1, except
+                                     for frames with a negative diagonal entry.
+                                     Models above 512 tiles (131072 unknowns) fall back to
+                                     Jacobi. */
     int32_t complex_hermitian;    /* complex-conductivity models only.  0 (default): conjugate
                                      orthogonal CG (dot products r^T z, p^T q without
                                      conjugation), the Krylov method for complex symmetric

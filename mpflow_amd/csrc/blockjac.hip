@@ -7,7 +7,9 @@
 // block of D1^-1/2 A(1) D1^-1/2, the unit-diagonal matrix at sigma = 1 -- one set of blocks per
 // mesh and harmonic, shared by all frames, no factorisation per frame.  The blocks follow
 // the frame's conductivity through D; exact blocks of the frame's matrix need as many
-// iterations (measured on an ellipse phantom with contrasts 0.2 to 5).
+// iterations (measured on an ellipse phantom with contrasts 0.2 to 5).  Conductivities are not
+// constrained to be positive: a frame with a negative diagonal entry has no D^-1/2 and takes the
+// signed diagonal, by the kernels of the jobs without blocks (the model leaves its bloc null).
 //
 // Iterations of the coupled electrode model on the 81181-node mesh to 1e-4, harmonics 0-4:
 // diagonal 68 / 53 / 44 / 37 / 31, blocks of 16 rows 51 / 35 / 28 / 24 / 20, of 32 48 / 31 / 25 /
@@ -208,6 +210,7 @@ __global__ void __launch_bounds__(256, 4) k_block_init(const JobDev* __restrict_
     constexpr int Rp = 1 << LG, LPR = Rp / 4, ROWS = 256 / LPR, PER = kTileRows / ROWS, CT = BT::CT;
     const int4 t = tiles[blockIdx.x];
     const JobDev& J = jobs[t.x];
+    if (!J.bloc) return;  // k_pcg_init
     const int s = t.y, tile0 = t.z * kTileRows;
     __shared__ typename BT::Rows rs;
     __shared__ float sd[kTileRows];
@@ -265,6 +268,7 @@ __global__ void __launch_bounds__(256, 4) k_block_update(const JobDev* __restric
     const int par = iter & 1, k4 = iter & (kRing - 1);
     const int4 t = tiles[blockIdx.x];
     const JobDev& J = jobs[t.x];
+    if (!J.bloc) return;  // k_pcg_update4
     const int s = t.y, tile0 = t.z * kTileRows;
     const bool live = slice_active(J, s);
     if (t.z == 0 && threadIdx.x == 0) J.st[s * kStInts + 3] = live ? 1 : 0;

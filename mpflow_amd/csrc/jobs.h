@@ -80,6 +80,7 @@ struct JobDev {
     // the unit-diagonal matrix at sigma = 1
     const uint8_t* tpos;         // [np] place of each row in its tile
     const float* bloc;           // [C][np / 32][4][64][4] operand order of the FP32 MFMA
+    int* dneg;                   // set with dinv: an entry of some harmonic is negative (no D^-1/2)
     // on-chip PCG (chip.hip; set by the Krylov driver for jobs that fit): the matrix in chip
     // order, positions of 16 bits
     const uint16_t* crow;        // [np] device row of each position
@@ -123,15 +124,16 @@ void launch_bicg_iter(const JobDev* d_jobs, const int4* d_tiles, int ntiles, int
 // (0: 128-bit gathers, width-binned, for padded widths <= 24; 1: 32-bit gathers; 2: as 0
 // with all harmonics of a (job, tile) in one block, over the (job, -, tile) list d_ftiles).
 constexpr int kSpmvVariants = 3;
+// which of the list's jobs have inverse diagonal blocks: none, all, or some (a launch for either kind)
+enum UpdateKind { kUpdDiagonal, kUpdBlocks, kUpdBoth };
 // d_js lists the group's (job, slice) pairs and `nchunk` the largest job's 32-tile
 // chunks: after the SpMV a small launch sums p.q and 1^T p per chunk, and between update
 // and pupdate one launch applies the two-level coarse correction (jobs that have one) and
-// sums r.z and r.r per chunk, so update and pupdate reduce chunk partials only.  blocks: every
-// job has inverse diagonal blocks.
+// sums r.z and r.r per chunk, so update and pupdate reduce chunk partials only.
 void launch_pcg_iter(const JobDev* d_jobs, const int4* d_tiles, int ntiles, int* d_active, int iter,
                      int lg, int wpad, int variant, hipStream_t st, hipEvent_t ev0 = nullptr,
                      hipEvent_t ev1 = nullptr, const int2* d_js = nullptr, int njs = 0, int nchunk = 0,
-                     const int4* d_ftiles = nullptr, int nftiles = 0, bool blocks = false);
+                     const int4* d_ftiles = nullptr, int nftiles = 0, UpdateKind upd = kUpdDiagonal);
 // per-tile conductivity scale of the two-level preconditioner (after assembly); d1: the
 // model's per-tile sigma = 1 diagonal sums; work items with slice != 0 are skipped
 void launch_coarse_scale(const JobDev* d_jobs, const int4* d_tiles, int ntiles, const double* d1,

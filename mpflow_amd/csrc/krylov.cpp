@@ -337,7 +337,7 @@ void KrylovDriver::launch_group_iter(Group& g, int iter, bool bicg, hipStream_t 
         launch_bicg_iter(jobs.p, g.cur, g.ncur, active.p, iter, g.lg, g.wpad, s, e0, e1);
     else
         launch_pcg_iter(jobs.p, g.cur, g.ncur, active.p, iter, g.lg, g.wpad, g.variant, s, e0, e1, g.js.p, g.njs,
-                        g.nchunk, g.fcur, g.nfcur, g.blocks);
+                        g.nchunk, g.fcur, g.nfcur, g.upd);
 }
 
 // Time each SpMV candidate that supports the group's width on the live job data (the
@@ -423,17 +423,16 @@ bool KrylovDriver::run(const mpf_solve_opts& o, int rule, double tol, bool use_r
         }
     }
     for (auto& g : groups) {
-        g.blocks = !(chip && g.chip);
-        for (int j : g.jobs) g.blocks = g.blocks && h[j].bloc;
-        if (!g.blocks)
-            for (int j : g.jobs) h[j].bloc = nullptr;
+        size_t with = 0;
+        for (int j : g.jobs) with += h[j].bloc != nullptr;
+        g.upd = with == 0 ? kUpdDiagonal : (with == g.jobs.size() ? kUpdBlocks : kUpdBoth);
     }
     jobs.upload(h.data(), h.size(), s0);
     MPF_HIP(hipMemsetAsync(active.p, 0, sizeof(int), s0));
     // the start: jobs with inverse blocks by their own kernel, the others by k_pcg_init
     auto start = [&](const int4* lt, int nt, const int2* lj, int nj2) {
         for (auto& g : groups)
-            if (g.blocks) launch_block_init(jobs.p, g.tiles_o[0].p, g.nall, g.lg, s0);
+            if (g.upd != kUpdDiagonal) launch_block_init(jobs.p, g.tiles_o[0].p, g.nall, g.lg, s0);
         launch_pcg_init(jobs.p, lt, nt, lj, nj2, active.p, s0, coarse ? init_nchunk : 0);
     };
     const int4* itiles = chip ? stream_tiles.p : init_tiles.p;

@@ -65,7 +65,7 @@ class KrylovDriver {
         int nall = 0, ncur = 0;
         const int4* cur = nullptr;
         size_t hoff = 0;              // the group's region of the pinned staging buffer
-        bool blocks = false;          // this run's update applies inverse diagonal blocks
+        UpdateKind upd = kUpdDiagonal;   // this run's jobs with inverse diagonal blocks
         // (job, 0, tile) items of the harmonic-fused SpMV (variant 2)
         std::vector<int4> fbase, fall;   // in (job, tile) order; XCD-ordered
         DBuf<int4> ftiles, fact;

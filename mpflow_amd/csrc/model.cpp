@@ -221,6 +221,7 @@ Model::Model(mpf_ctx* c, const mpf_model_desc& d) : ctx(c) {
 }
 
 Model::~Model() {
+    if (h_dneg) (void)hipHostFree(h_dneg);
 }
 
 void Model::upload_jobs() {
@@ -251,9 +252,17 @@ void Model::prepare(const mpf_solve_opts& o) {
     if (two_level) ensure_blocks();
     upload_jobs();
     launch_assemble(jobs.p, asm_items.p, nasm, st0);
+    const bool blocks = two_level && bloc.p;
+    if (blocks) MPF_HIP(hipMemsetAsync(dneg.p, 0, dneg.bytes(), st0));
     launch_dinv(jobs.p, tiles.p, ntiles, st0);
+    if (blocks) MPF_HIP(hipMemcpyAsync(h_dneg, dneg.p, dneg.bytes(), hipMemcpyDeviceToHost, st0));
     if (S.fixed) launch_fixed_rhs(jobs.p, frames, fixdev(), st0);
     if (two_level) launch_coarse_scale(jobs.p, tiles.p, ntiles, cd1.p, st0);
+    if (blocks) {
+        // the blocks need D^-1/2: frames with a negative diagonal entry take the diagonal
+        MPF_HIP(hipStreamSynchronize(st0));
+        for (int f = 0; f < frames; ++f) hjobs[f].bloc = h_dneg[f] ? nullptr : bloc.p;
+    }
 }
 
 // The inverse diagonal blocks of a mesh that the streaming PCG solves (the on-chip one keeps
@@ -265,10 +274,13 @@ void Model::ensure_blocks() {
     hipStream_t st0 = ctx->stream;
     try {
         bloc.alloc(block_inverse_floats(S.C, S.np));
+        dneg.alloc(frames);
     } catch (const Error& e) {
         if (e.code != MPF_ENOMEM) throw;
+        bloc.release();
         return;
     }
+    MPF_HIP(hipHostMalloc((void**)&h_dneg, dneg.bytes(), hipHostMallocDefault));
     DBuf<int> bad(1);
     int hbad = 0;
     bad.upload(&hbad, 1, st0);
@@ -280,7 +292,7 @@ void Model::ensure_blocks() {
         bloc.release();
         return;
     }
-    for (auto& J : hjobs) J.bloc = bloc.p;
+    for (int f = 0; f < frames; ++f) hjobs[f].dneg = dneg.p + f;
 }
 
 // FP64 refinement report, voltages and (optionally) the Jacobian after the solves.

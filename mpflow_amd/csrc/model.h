@@ -43,6 +43,8 @@ struct Model {
     DBuf<float> cinv, csc, cy, cg;          // two-level preconditioner (allocated if the mesh has one)
     DBuf<double> cd1;
     DBuf<float> bloc;                       // inverse diagonal blocks (first two-level solve of a large mesh)
+    DBuf<int> dneg;                         // per frame: a negative diagonal entry
+    int* h_dneg = nullptr;                  // pinned
     bool bloc_tried = false;
     void ensure_blocks();
     DBuf<float> ek, em;

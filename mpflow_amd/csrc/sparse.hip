@@ -63,6 +63,7 @@ __global__ void __launch_bounds__(kBlock) k_dinv(const JobDev* __restrict__ jobs
         v = a != 0.0f ? 1.0f / a : 0.0f;
     }
     J.dinv[(size_t)s * J.np + row] = v;
+    if (v < 0.0f && J.dneg) *J.dneg = 1;
 }
 
 // --------------------------------------------------------------------------------
@@ -375,6 +376,7 @@ __global__ void __launch_bounds__(kUpdBlock, 6) k_pcg_update4(const JobDev* __re
     const int par = iter & 1, k4 = iter & (kRing - 1);
     const int4 t = tiles[blockIdx.x];
     const JobDev& J = jobs[t.x];
+    if (J.bloc) return;   // k_block_update
     const int s = t.y;
     const bool live = slice_active(J, s);
     if (t.z == 0 && threadIdx.x == 0) J.st[s * kStInts + 3] = live ? 1 : 0;
@@ -1172,7 +1174,7 @@ void launch_pcg_spmv(const JobDev* d_jobs, const int4* d_tiles, int ntiles, int 
 
 void launch_pcg_iter(const JobDev* d_jobs, const int4* d_tiles, int ntiles, int* d_active, int iter,
                      int lg, int wpad, int variant, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1,
-                     const int2* d_js, int njs, int nchunk, const int4* d_ftiles, int nftiles, bool blocks) {
+                     const int2* d_js, int njs, int nchunk, const int4* d_ftiles, int nftiles, UpdateKind upd) {
     if (ev0) MPF_HIP(hipEventRecord(ev0, st));
     if (variant == 2) {
         MPF_REQUIRE(d_ftiles, "pcg iteration: the harmonic-fused SpMV needs a (job, tile) list");
@@ -1185,10 +1187,12 @@ void launch_pcg_iter(const JobDev* d_jobs, const int4* d_tiles, int ntiles, int*
     if (lg == 6) chunks_launch<6>(d_jobs, d_js, njs, nchunk, st);
     else if (lg == 5) chunks_launch<5>(d_jobs, d_js, njs, nchunk, st);
     else chunks_launch<4>(d_jobs, d_js, njs, nchunk, st);
-    if (blocks) launch_block_update(d_jobs, d_tiles, ntiles, iter, lg, st);
-    else if (lg == 6) k_pcg_update4<6><<<ntiles, kUpdBlock, 0, st>>>(d_jobs, d_tiles, iter);
-    else if (lg == 5) k_pcg_update4<5><<<ntiles, kUpdBlock, 0, st>>>(d_jobs, d_tiles, iter);
-    else k_pcg_update4<4><<<ntiles, kUpdBlock, 0, st>>>(d_jobs, d_tiles, iter);
+    if (upd != kUpdDiagonal) launch_block_update(d_jobs, d_tiles, ntiles, iter, lg, st);
+    if (upd != kUpdBlocks) {
+        if (lg == 6) k_pcg_update4<6><<<ntiles, kUpdBlock, 0, st>>>(d_jobs, d_tiles, iter);
+        else if (lg == 5) k_pcg_update4<5><<<ntiles, kUpdBlock, 0, st>>>(d_jobs, d_tiles, iter);
+        else k_pcg_update4<4><<<ntiles, kUpdBlock, 0, st>>>(d_jobs, d_tiles, iter);
+    }
     // coarse correction where the job has one; chunk sums of r.z and r.r for every job
     launch_coarse_all(d_jobs, d_js, njs, nchunk, lg, 2, 3, st);
     // the last iteration of each direction-ring cycle also moves x
