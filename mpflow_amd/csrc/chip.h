@@ -20,6 +20,15 @@ struct ChipShape {
 // that keeps every workgroup on a CU of its own.
 ChipShape chip_shape(int np, int width, long long lanes);
 
+// Step k of a workgroup of nw wavefronts: the offset of its positions from those of step 0, 64 per
+// wavefront.  K is rounded up to an instantiated kernel, so a wavefront's last steps may lie past the
+// np rows; their loads, issued ahead of the gather's test, go to step 0's positions.  (As the scalar
+// offset of a raw buffer load it is not part of the offset that the bounds check sees: a step past
+// the table would read past it.)
+__host__ __device__ constexpr int chip_step(int k, int wave, int nw, int np) {
+    return (wave + k * nw) * 64 < np ? k * nw * 64 : 0;
+}
+
 // gst flags of a lane group
 constexpr int kChipCapped = 1, kChipNan = 2, kChipEmpty = 4;
 

@@ -368,10 +368,10 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
             if constexpr (HOLD) { id = hid[k]; va = hva[k]; vb = hvb[k]; }
             else { id = idn; va = van; vb = vbn; }
             if (!HOLD && k + 1 < K) {
-                // past the last position the loads are out of range or another row's: unused
-                idn = load(ids, (k + 1) * nt);
-                van = load(val, (k + 1) * nt);
-                vbn = load(val, npu + (k + 1) * nt);
+                const int next = chip_step(k + 1, wave, nw, npu);   // past the rows: another row's, unused
+                idn = load(ids, next);
+                van = load(val, next);
+                vbn = load(val, npu + next);
             }
             if (has(k)) {
                 float acc[G];
