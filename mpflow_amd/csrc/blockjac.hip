@@ -105,8 +105,8 @@ __global__ void __launch_bounds__(256) k_block_inverse(const JobDev* __restrict_
 // --------------------------------------------------------------------------------
 // one tile's z = D^-1/2 B D^-1/2 r
 // --------------------------------------------------------------------------------
-// rs: r of the tile as [place][column], replaced by z; sd: D^-1/2 per place.  Adds r.z, r.r (FP64)
-// and W^T r (FP32) of the lane's entries: columns 16 ct + l % 16 of the wavefront's aggregate.
+// rs: r of the tile as [place][column], replaced by z; sd: D^-1/2 per place.  Adds r.z, r.r and W^T r
+// (FP64) of the lane's entries: columns 16 ct + l % 16 of the wavefront's aggregate.
 template <int LG>
 struct BlockTile {
     static constexpr int Rp = 1 << LG, CT = Rp / 16, LD = Rp + 4;
@@ -120,7 +120,7 @@ struct BlockTile {
         for (int f = 0; f < 8; ++f) a[f] = b[64 * f];
     }
     static __device__ __forceinline__ void apply(Rows& rs, const float* sd, const float4 (&a)[8], double (&rz)[CT],
-                                                 double (&rr)[CT], float (&g)[CT]) {
+                                                 double (&rr)[CT], double (&g)[CT]) {
         const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, o = l & 15, q4 = 4 * (l >> 4);
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
@@ -166,7 +166,7 @@ struct BlockTile {
                         const float r = rv[ib][v][ct], z = sv[ib][v] * acc[ib][ct][v];
                         rz[ct] += (double)r * (double)z;
                         rr[ct] += (double)r * (double)r;
-                        g[ct] += r;
+                        g[ct] += (double)r;
                         rs[p0 + 16 * ib + q4 + v][16 * ct + o] = z;
                     }
         }
@@ -174,7 +174,7 @@ struct BlockTile {
     // the wavefronts' sums: rz and rr as the tile's partials of channels c0 and c0 + 1, W^T r of
     // aggregate w in its channel and, scaled, for the coarse kernel
     static __device__ __forceinline__ void sums(const JobDev& J, int s, int tile, int c0, double (&rz)[CT],
-                                                double (&rr)[CT], float (&g)[CT], double (*red)[4][Rp]) {
+                                                double (&rr)[CT], double (&g)[CT], double (*red)[4][Rp]) {
         const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, o = l & 15;
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
@@ -188,8 +188,8 @@ struct BlockTile {
                 const int col = 16 * ct + o, a = kAggPerTile * tile + wave;
                 red[0][wave][col] = rz[ct];
                 red[1][wave][col] = rr[ct];
-                part_ptr(J, agg_channel(wave), s, tile)[col] = (double)g[ct];
-                gp(J.cg)[((size_t)s * kAggPerTile * J.ntiles + a) * Rp + col] = J.csc[a] * g[ct];
+                part_ptr(J, agg_channel(wave), s, tile)[col] = g[ct];
+                gp(J.cg)[((size_t)s * kAggPerTile * J.ntiles + a) * Rp + col] = (float)((double)J.csc[a] * g[ct]);
             }
         }
         __syncthreads();
@@ -244,10 +244,9 @@ __global__ void __launch_bounds__(256, 4) k_block_init(const JobDev* __restrict_
         *(float4*)&rs[J.tpos[row]][4 * c4] = make_float4(b[0], b[1], b[2], b[3]);
     }
     __syncthreads();
-    double rz[CT], rr[CT];
-    float g[CT];
+    double rz[CT], rr[CT], g[CT];
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) { rz[ct] = 0.0; rr[ct] = 0.0; g[ct] = 0.0f; }
+    for (int ct = 0; ct < CT; ++ct) { rz[ct] = 0.0; rr[ct] = 0.0; g[ct] = 0.0; }
     BT::apply(rs, sd, a, rz, rr, g);
     BT::sums(J, s, t.z, 0, rz, rr, g, red);
 #pragma unroll
@@ -348,10 +347,9 @@ __global__ void __launch_bounds__(256, 4) k_block_update(const JobDev* __restric
     float4 a[8];
     BT::load(J, s, t.z, a);
     __syncthreads();
-    double rz[CT], rr[CT];
-    float g[CT];
+    double rz[CT], rr[CT], g[CT];
 #pragma unroll
-    for (int ct = 0; ct < CT; ++ct) { rz[ct] = 0.0; rr[ct] = 0.0; g[ct] = 0.0f; }
+    for (int ct = 0; ct < CT; ++ct) { rz[ct] = 0.0; rr[ct] = 0.0; g[ct] = 0.0; }
     BT::apply(rs, sd, a, rz, rr, g);
     BT::sums(J, s, t.z, 2, rz, rr, g, red);
 #pragma unroll

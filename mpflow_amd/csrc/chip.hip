@@ -15,7 +15,7 @@
 //
 // Measured (MI355X, whole calls): one 2D forward solve of 817 nodes, 168 steps, 4.60 -> 0.42
 // ms (1.02 ms with the deciding group of the reference rule run before the others); 64 frames x 5
-// harmonics of 4921 nodes to 1e-6 18.1 -> 5.5 ms (1024 threads 7.2 ms); a caller's 4921-row
+// harmonics of 4921 nodes to 1e-6 18.1 -> 5.75 ms (1024 threads 7.2 ms against 5.5 at the time); a caller's 4921-row
 // matrix with 32 columns 2.02 -> 0.56 ms.
 //
 // The recurrences, the FP64 scalars, the stop rules and the breakdown rules are those of the
@@ -112,6 +112,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
     constexpr bool DLDS = chip_dinv_in_lds<G, NP>();
     __shared__ VecG ps[NP];                        // p (0 past the rows)
     __shared__ float ds[DLDS ? NP : 1];            // Jacobi inverse
+    __shared__ double gs[NA * G];                  // (W^T r)_a
     __shared__ VecG cgs[NA];                       // c_a (W^T r)_a
     __shared__ VecG cys[NA];                       // coarse correction
     __shared__ float cs[NA];                       // c_a
@@ -180,10 +181,13 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
     };
     const __amdgpu_buffer_rsrc_t cinv =
         uniform_rsrc(coarse ? J.cinv + (size_t)s * na * J.cld : nullptr, coarse ? (size_t)na * J.cld * 4 : 0);
-    // z = D^-1 r + W C cinv C W^T r into q (two barriers with a coarse level).  The coarse
-    // product runs in items of 4 coarse rows (16 lanes each) x 64 columns per wavefront,
-    // four of them loaded ahead: the first four before the barrier that the sums wait for.
-    auto precondition = [&]() {
+    // z = D^-1 r + W C cinv C W^T r into q (two barriers with a coarse level) and, added to vz, r.z as
+    // r.D^-1 r over the rows and W^T r . y over the aggregates, in FP64.  W^T r is as wide as the
+    // streamed kernels': FP64 at the start, in the iteration FP32 sums of 16 rows added in FP64 (FP64
+    // throughout: 4% more per forward solve of 64 frames x 5 harmonics of 4921 nodes).  The coarse
+    // product runs in items of 4 coarse rows (16 lanes each) x 64 columns per wavefront, four of
+    // them loaded ahead: the first four before the barrier that the sums wait for.
+    auto precondition = [&](double (&vz)[G], auto at_start) __attribute__((always_inline)) {
         if (coarse) {
             constexpr int PF = 4;
             int lo = l;
@@ -202,9 +206,20 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
             fetch(0);
             each_row<K>([&](auto kc) __attribute__((always_inline)) {
                 constexpr int k = decltype(kc)::value;
-                const float t = wave_sum<G>(r[k], l);
+                double t;
+                if constexpr (decltype(at_start)::value) {
+                    double rd[G];
+#pragma unroll
+                    for (int c = 0; c < G; ++c) rd[c] = (double)r[k][c];
+                    t = wave_sum<G>(rd, l);
+                } else {
+                    t = wave_sum_wide<G>(r[k], l);
+                }
                 const int a = wave + k * nw;
-                if (l < G) reinterpret_cast<float*>(cgs)[a * G + col] = cs[a] * t;
+                if (l < G) {
+                    gs[a * G + col] = t;
+                    reinterpret_cast<float*>(cgs)[a * G + col] = (float)((double)cs[a] * t);
+                }
             });
             __syncthreads();
             float y[G];
@@ -242,6 +257,12 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
                 if (i0 + PF < nitem) fetch(i0 + PF);
             }
             __syncthreads();
+            if (tid < na) {
+                float y[G];
+                unpack<G>(cys[tid], y);
+#pragma unroll
+                for (int c = 0; c < G; ++c) vz[c] += gs[tid * G + c] * (double)y[c];
+            }
         }
         each_row<K>([&](auto kc) __attribute__((always_inline)) {
             constexpr int k = decltype(kc)::value;
@@ -256,7 +277,10 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
                     for (int c = 0; c < G; ++c) y[c] = 0.0f;
             }
 #pragma unroll
-            for (int c = 0; c < G; ++c) q[k][c] = fmaf(d, r[k][c], y[c]);
+            for (int c = 0; c < G; ++c) {
+                vz[c] += (double)r[k][c] * (double)(d * r[k][c]);
+                q[k][c] = fmaf(d, r[k][c], y[c]);
+            }
         });
     };
     // per-lane column totals of two quantities over the block (one barrier)
@@ -272,17 +296,11 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
         a = across_waves<G>(&red[0][0], 2 * G, nw, l);
         b = second ? across_waves<G>(&red[0][G], 2 * G, nw, l) : 0.0;
     };
-    // r.z and r.r
-    auto dots = [&](double (&vz)[G], double (&vr)[G]) {
-#pragma unroll
-        for (int c = 0; c < G; ++c) { vz[c] = 0.0; vr[c] = 0.0; }
+    auto norms = [&](double (&vr)[G]) {
         each_row<K>([&](auto kc) __attribute__((always_inline)) {
             constexpr int k = decltype(kc)::value;
 #pragma unroll
-            for (int c = 0; c < G; ++c) {
-                vz[c] += (double)r[k][c] * (double)q[k][c];
-                vr[c] += (double)r[k][c] * (double)r[k][c];
-            }
+            for (int c = 0; c < G; ++c) vr[c] += (double)r[k][c] * (double)r[k][c];
         });
     };
 
@@ -331,9 +349,11 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
             bb = sc_ptr(J, SC_BB, s)[lane];
         } else {
             __syncthreads();                       // cs
-            precondition();
             double vb[G], vz[G];
-            dots(vz, vb);
+#pragma unroll
+            for (int c = 0; c < G; ++c) { vb[c] = 0.0; vz[c] = 0.0; }
+            precondition(vz, std::true_type());
+            norms(vb);
             each_row<K>([&](auto kc) __attribute__((always_inline)) {
                 constexpr int k = decltype(kc)::value;
                 ps[tid + k * nt] = pack<G>(q[k]);
@@ -451,9 +471,11 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
                 for (int c = 0; c < G; ++c)
                     if ((zeros >> lane_of<G>(c)) & 1) r[k][c] = 0.0f;
             });
-        precondition();
         double vz[G], vr[G], rz, rr;
-        dots(vz, vr);
+#pragma unroll
+        for (int c = 0; c < G; ++c) { vz[c] = 0.0; vr[c] = 0.0; }
+        precondition(vz, std::false_type());
+        norms(vr);
         if (follows && tid == 0) told = lead_word(word, steps + 1, seen);
         block_sum(red2, vz, vr, true, rz, rr);
         // beta = rho' / rho (rho == 0 zeroes p)

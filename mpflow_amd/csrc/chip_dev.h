@@ -73,10 +73,10 @@ __device__ __forceinline__ int col_of(int l) {
 template <int G>
 constexpr int lane_of(int c) { return G == 4 ? ((c >> 1) & 1) | ((c & 1) << 1) : c; }
 
-// per-lane values of G columns summed over the wavefront: lane l returns column col_of(l).
-// The first steps halve the columns (each lane keeps one half and sends the other).
+// per-lane values of G columns summed over quads: lane l returns column col_of(l).  The steps halve
+// the columns (each lane keeps one half and sends the other).
 template <int G, class T>
-__device__ __forceinline__ T wave_sum(const T (&v)[G], int l) {
+__device__ __forceinline__ T quad_sum(const T (&v)[G], int l) {
     T a;
     if constexpr (G == 4) {
         const bool hi = l & 1;
@@ -96,7 +96,20 @@ __device__ __forceinline__ T wave_sum(const T (&v)[G], int l) {
         a += dpp<kXor1>(a);
         a += dpp<kXor2>(a);
     }
-    return add_quads(a);
+    return a;
+}
+// the same over the wavefront
+template <int G, class T>
+__device__ __forceinline__ T wave_sum(const T (&v)[G], int l) {
+    return add_quads(quad_sum<G>(v, l));
+}
+// FP32 values: 16 lanes in FP32, their sums in FP64
+template <int G>
+__device__ __forceinline__ double wave_sum_wide(const float (&v)[G], int l) {
+    float a = quad_sum<G>(v, l);
+    a += dpp<kRor4>(a);
+    a += dpp<kRor8>(a);
+    return add_halves<32>(add_halves<16>((double)a));
 }
 
 // the wavefronts' wave_sum results (red[wave][column]) summed in a fixed tree: every lane
