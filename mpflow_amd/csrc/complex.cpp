@@ -113,7 +113,7 @@ bool ComplexModel::Impl::ensure_chip() {
             MPF_HIP(hipMemsetAsync(g.p, 0, g.bytes(), st0));
         }
         progress.alloc(total);
-        MPF_HIP(hipHostMalloc((void**)&h_gst, sizeof(int2) * total, hipHostMallocDefault));
+        h_gst = pinned_alloc<int2>(total);
         launch_chip_order(np, nullptr, crow.p, cpos.p, st0);
         launch_chip_ids(np, W, ids.p, gw.p, crow.p, cpos.p, cid.p, octs.p, st0);
         MPF_HIP(hipStreamSynchronize(st0));
@@ -124,7 +124,8 @@ bool ComplexModel::Impl::ensure_chip() {
         }
     } catch (const Error& e) {
         if (e.code != MPF_ENOMEM) throw;
-        cval.release();
+        cid.release(); octs.release(); cval.release(); chip_items.release(); progress.release();
+        for (auto& g : gst) g.release();
         return false;
     }
     return chip_ok = true;

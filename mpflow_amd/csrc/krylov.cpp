@@ -153,12 +153,23 @@ KrylovDriver::~KrylovDriver() {
     if (h_active) (void)hipHostFree(h_active);
     if (h_st) (void)hipHostFree(h_st);
     if (h_tiles) (void)hipHostFree(h_tiles);
+    drop_chip();
+}
+
+// the on-chip solver's tables, streams and events
+void KrylovDriver::drop_chip() {
     if (h_gst) (void)hipHostFree(h_gst);
     for (auto& c : chips) {
         if (c.done) (void)hipEventDestroy(c.done);
         if (c.stream) (void)hipStreamDestroy(c.stream);
     }
     if (chip_fork) (void)hipEventDestroy(chip_fork);
+    h_gst = nullptr;
+    chip_fork = nullptr;
+    chips.clear();
+    chip_meshes.clear();
+    cval.release(); chip_js.release(); progress.release();
+    for (auto& g : gst) g.release();
 }
 
 // Tables of the on-chip PCG (chip.hip), once per driver: the chip order and 16-bit matrix of
@@ -264,13 +275,12 @@ bool KrylovDriver::ensure_chip() {
         progress.alloc(total);
         MPF_HIP(hipMemsetAsync(gst[0].p, 0, gst[0].bytes(), s0));
         MPF_HIP(hipMemsetAsync(gst[1].p, 0, gst[1].bytes(), s0));
-        MPF_HIP(hipHostMalloc((void**)&h_gst, sizeof(int2) * total, hipHostMallocDefault));
+        h_gst = pinned_alloc<int2>(total);
         MPF_HIP(hipStreamSynchronize(s0));
     } catch (const Error& e) {
         if (e.code != MPF_ENOMEM) throw;
         // no room for the tables: the jobs are streamed
-        cval.release();
-        chip_meshes.clear();
+        drop_chip();
         return false;
     }
     chip_ok = true;

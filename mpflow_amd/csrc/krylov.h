@@ -88,6 +88,7 @@ class KrylovDriver {
         DBuf<uint8_t> octs;
     };
     bool ensure_chip();               // false: no job fits, or no room for the tables
+    void drop_chip();
     void run_chip();
     bool chip_tried = false, chip_ok = false;
     std::vector<ChipClass> chips;

@@ -373,7 +373,6 @@ void Mlp::ensure_batch(int B) {
             work.alloc(kSplitWork);
         } catch (const Error& e) {
             if (e.code != MPF_ENOMEM) throw;   // no room: no product is split
-            (void)hipGetLastError();
         }
     }
 }

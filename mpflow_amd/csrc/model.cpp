@@ -275,12 +275,13 @@ void Model::ensure_blocks() {
     try {
         bloc.alloc(block_inverse_floats(S.C, S.np));
         dneg.alloc(frames);
+        h_dneg = pinned_alloc<int>(frames);
     } catch (const Error& e) {
         if (e.code != MPF_ENOMEM) throw;
         bloc.release();
+        dneg.release();
         return;
     }
-    MPF_HIP(hipHostMalloc((void**)&h_dneg, dneg.bytes(), hipHostMallocDefault));
     DBuf<int> bad(1);
     int hbad = 0;
     bad.upload(&hbad, 1, st0);

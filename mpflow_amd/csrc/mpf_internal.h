@@ -45,6 +45,20 @@ struct Error : std::runtime_error {
 inline int ceil16(int n) { return (n % 16 == 0 || n == 1) ? n : (n / 16 + 1) * 16; }
 inline int round_up(int n, int m) { return (n + m - 1) / m * m; }
 
+// Out of memory: callers with another way handle it, so the runtime's record of the failed call goes
+// too (the check after the next kernel launch would report it as the launch's).
+[[noreturn]] inline void no_memory(const char* what) {
+    (void)hipGetLastError();
+    throw Error(MPF_ENOMEM, std::string(what) + " failed");
+}
+// pinned host memory of n elements, freed with hipHostFree
+template <class T>
+T* pinned_alloc(size_t n) {
+    T* p = nullptr;
+    if (hipHostMalloc((void**)&p, n * sizeof(T), hipHostMallocDefault) != hipSuccess) no_memory("hipHostMalloc");
+    return p;
+}
+
 // Device buffer with RAII.
 template <class T>
 struct DBuf {
@@ -62,7 +76,7 @@ struct DBuf {
         n = count;
         if (count) {
             hipError_t e = hipMalloc(&p, count * sizeof(T));
-            if (e != hipSuccess) { p = nullptr; n = 0; throw Error(MPF_ENOMEM, "hipMalloc failed"); }
+            if (e != hipSuccess) { p = nullptr; n = 0; no_memory("hipMalloc"); }
         }
     }
     void release() { if (p) (void)hipFree(p); p = nullptr; n = 0; }
