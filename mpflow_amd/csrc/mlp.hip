@@ -10,10 +10,9 @@
 #include <atomic>
 #include <cmath>
 #include <cstring>
-#include <system_error>
-#include <thread>
 
 #include "mlp.h"
+#include "threads.h"
 
 namespace mpf {
 
@@ -480,15 +479,7 @@ bool Mlp::read(const std::vector<Span>& spans) {
         }
         failed = (int)e;
     };
-    std::vector<std::thread> threads;
-    threads.reserve(kReadThreads);
-    try {
-        for (int t = 1; t < kReadThreads; ++t) threads.emplace_back(work, t);
-    } catch (const std::system_error&) {
-        // the threads there are share the chunks
-    }
-    work(0);
-    for (auto& t : threads) t.join();
+    on_threads(kReadThreads, work);
     MPF_HIP((hipError_t)failed.load());
     return true;
 }
