@@ -91,6 +91,12 @@ void* mpf_ctx_stream(mpf_ctx* ctx);
 int mpf_ctx_profile(mpf_ctx* ctx, int32_t enable);
 int mpf_ctx_profile_read(mpf_ctx* ctx, double out[3]);
 
+/* On-chip solves under the reference stop rule: the most polls (about a microsecond each,
+ * default 128) for which a lane group waits within a step for the group that decides.  A
+ * group that gives up goes on in a launch after the deciding one: results do not depend on
+ * the bound.  For tests and tuning; no counterpart in the reference. */
+int mpf_ctx_lead_polls(mpf_ctx* ctx, int32_t polls);
+
 /* HBM streaming reference for the rooflines (no counterpart in the reference): the best
  * rate in GB/s over `reps` timed launches (after one warm-up) of a grid-stride 128-bit
  * kernel of `blocks` 256-thread blocks with `loads` (1, 2, 4) float4 in flight per thread.
@@ -216,7 +222,11 @@ typedef struct mpf_solve_opts {
     int32_t refine_steps;         /* FP64 refinement passes (MPF_PREC_MIXED)        */
     double refine_tol;            /* inner tolerance of each refinement solve       */
     int32_t krylov;               /* MPF_KRYLOV_*                                   */
-    int32_t check_every;          /* iterations between host convergence polls (0 -> 16) */
+    int32_t check_every;          /* iterations between host convergence polls (0 -> 16).  Small
+                                     meshes (up to 20480 unknowns, 8192 with complex
+                                     conductivity; outside mpf_ctx_profile) solve in one
+                                     launch that polls nothing: neither this nor `graphs` has
+                                     an effect there, and it runs to max_iter at most */
     int32_t warm_start;           /* MPF_PREC_MIXED only: start from the model's previous FP64
                                      fields (a correction solve of the FP64 residual, stopped at
                                      tol * ||b||) instead of from zero; ignored on the first solve */

@@ -126,6 +126,14 @@ int mpf_ctx_profile_read(mpf_ctx* ctx, double out[3]) {
     });
 }
 
+int mpf_ctx_lead_polls(mpf_ctx* ctx, int32_t polls) {
+    return guarded([&] {
+        MPF_REQUIRE(ctx && polls >= 0, "mpf_ctx_lead_polls: null context or negative bound");
+        ctx->lead_polls = polls;
+        return MPF_OK;
+    });
+}
+
 int mpf_ctx_stream_probe(mpf_ctx* ctx, int32_t pattern, int32_t loads, const float* d_x, float* d_y, int64_t n,
                          int32_t blocks, int32_t reps, double* gbps) {
     return guarded([&] {

@@ -29,6 +29,9 @@ __host__ __device__ constexpr int chip_step(int k, int wave, int nw, int np) {
     return (wave + k * nw) * 64 < np ? k * nw * 64 : 0;
 }
 
+// polls (about a microsecond each) after which a lane group gives up its wait for the deciding group
+constexpr int kLeadPolls = 128;
+
 // gst flags of a lane group
 constexpr int kChipCapped = 1, kChipNan = 2, kChipEmpty = 4;
 
@@ -46,9 +49,10 @@ void launch_chip_pack(const JobDev* d_jobs, const int2* d_js, int njs, int max_n
 // one phase over `n` items (job, slice, lane group, index of the pair's first group state):
 // phase 0 runs every lane group from its start to its own stop test -- under the reference rule
 // to the step its pair's deciding group stops at, which that group publishes in progress (zeroed
-// by launch_chip_pack; at the pair's first index) -- and phase 1 takes the groups behind their
-// pair's largest step count (gin) on to it.  gout receives every group's (steps, flags).
+// by launch_chip_pack; at the pair's first index; waited for `polls` polls a step) -- and phase 1
+// takes the groups behind their pair's largest step count (gin) on to it.  gout receives every
+// group's (steps, flags).
 void launch_chip(const JobDev* d_jobs, const int4* d_items, int n, const ChipShape& c, const int2* gin, int2* gout,
-                 int* progress, int phase, hipStream_t st);
+                 int* progress, int polls, int phase, hipStream_t st);
 
 }  // namespace mpf

@@ -106,7 +106,7 @@ constexpr bool chip_dinv_in_lds() { return (size_t)NP * 4 * (G + 1) <= 140 * 102
 template <int G, int K, int NT, bool HOLD>
 __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restrict__ jobs, const int4* __restrict__ items,
                                                     const int2* __restrict__ gin, int2* __restrict__ gout,
-                                                    int* progress, int phase) {
+                                                    int* progress, int polls, int phase) {
     typedef typename ChipVec<G>::type VecG;
     constexpr int NP = K * NT, NA = NP / kAggRows;
     constexpr bool DLDS = chip_dinv_in_lds<G, NP>();
@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_pcg_chip(const JobDev* __restr
         for (int c = 0; c < G; ++c) { vz[c] = 0.0; vr[c] = 0.0; }
         precondition(vz, std::false_type());
         norms(vr);
-        if (follows && tid == 0) told = lead_word(word, steps + 1, seen);
+        if (follows && tid == 0) told = lead_word(word, steps + 1, seen, polls);
         block_sum(red2, vz, vr, true, rz, rr);
         // beta = rho' / rho (rho == 0 zeroes p)
         const float be = rho != 0.0 ? (float)(rz / rho) : 0.0f;
@@ -607,16 +607,16 @@ void launch_chip_pack(const JobDev* d_jobs, const int2* d_js, int njs, int max_n
 // kernels for MINK..MAXK rows per thread; up to MAXH the matrix may stay in registers
 template <int G, int NT, int MINK, int MAXK, int MAXH>
 static void chip_dispatch(const JobDev* d_jobs, const int4* d_items, int n, const ChipShape& c, const int2* gin,
-                          int2* gout, int* progress, int phase, hipStream_t st) {
+                          int2* gout, int* progress, int polls, int phase, hipStream_t st) {
 #define MPF_CHIP(k)                                                                                           \
     case k:                                                                                                   \
         if constexpr (k <= MAXH)                                                                              \
             if (c.hold) {                                                                                     \
-                k_pcg_chip<G, k, NT, true><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, phase); \
+                k_pcg_chip<G, k, NT, true><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, polls, phase); \
                 return;                                                                                       \
             }                                                                                                 \
         if constexpr (k >= MINK && k <= MAXK) {                                                               \
-            k_pcg_chip<G, k, NT, false><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, phase); \
+            k_pcg_chip<G, k, NT, false><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, polls, phase); \
             return;                                                                                           \
         }                                                                                                     \
         break;
@@ -630,15 +630,15 @@ static void chip_dispatch(const JobDev* d_jobs, const int4* d_items, int n, cons
 }
 
 void launch_chip(const JobDev* d_jobs, const int4* d_items, int n, const ChipShape& c, const int2* gin, int2* gout,
-                 int* progress, int phase, hipStream_t st) {
+                 int* progress, int polls, int phase, hipStream_t st) {
     if (!n) return;
-    if (c.G == 4) chip_dispatch<4, 512, 1, 10, 0>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
+    if (c.G == 4) chip_dispatch<4, 512, 1, 10, 0>(d_jobs, d_items, n, c, gin, gout, progress, polls, phase, st);
     else if (c.G == 2 && c.threads <= 512)
-        chip_dispatch<2, 512, 1, 20, 0>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
-    else if (c.G == 2) chip_dispatch<2, 1024, 1, 8, 0>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
+        chip_dispatch<2, 512, 1, 20, 0>(d_jobs, d_items, n, c, gin, gout, progress, polls, phase, st);
+    else if (c.G == 2) chip_dispatch<2, 1024, 1, 8, 0>(d_jobs, d_items, n, c, gin, gout, progress, polls, phase, st);
     else if (c.threads <= 512)
-        chip_dispatch<1, 512, 1, 5, 10>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
-    else chip_dispatch<1, 1024, 3, 20, 0>(d_jobs, d_items, n, c, gin, gout, progress, phase, st);
+        chip_dispatch<1, 512, 1, 5, 10>(d_jobs, d_items, n, c, gin, gout, progress, polls, phase, st);
+    else chip_dispatch<1, 1024, 3, 20, 0>(d_jobs, d_items, n, c, gin, gout, progress, polls, phase, st);
     check_launch();
 }
 

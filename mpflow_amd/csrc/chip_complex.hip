@@ -125,7 +125,7 @@ __device__ __forceinline__ void add_lanes(const double (&v)[Q], double (*red)[34
 template <int G, int K, int NT, bool HOLD, int RL>
 __global__ void __launch_bounds__(NT, NT / 256) k_c_chip(const CJob* __restrict__ jobs, const int4* __restrict__ items,
                                                          const int2* __restrict__ gin, int2* __restrict__ gout,
-                                                         int* progress, int phase) {
+                                                         int* progress, int polls, int phase) {
     static_assert(K == 4 || K == 8, "a wavefront owns one or two tiles");
     constexpr int NP = K * NT, W = 2 * G, NTL = NP / kTileRows;
     typedef typename ChipVec<W>::type VecW;        // G complex columns
@@ -457,7 +457,7 @@ __global__ void __launch_bounds__(NT, NT / 256) k_c_chip(const CJob* __restrict_
         });
         zd rz;
         double rr;
-        if (follows && tid == 0) told = lead_word(word, steps + 1, seen);
+        if (follows && tid == 0) told = lead_word(word, steps + 1, seen, polls);
         precondition(rz, rr);
         const bool rz0 = zzero(rho);
         const zd be = rz0 ? zmake(0.0) : by_rho.of(rz);
@@ -558,11 +558,11 @@ void launch_c_chip_pack(const CJob* d_jobs, const int2* d_js, int njs, int np, i
 
 template <int G, int K, int NT, bool HOLD>
 static void c_chip_dispatch(const CJob* d_jobs, const int4* d_items, int n, const ChipShape& c, int Rq,
-                            const int2* gin, int2* gout, int* progress, int phase, hipStream_t st) {
+                            const int2* gin, int2* gout, int* progress, int polls, int phase, hipStream_t st) {
     switch (Rq) {
 #define MPF_CHIP(rq, rl)                                                                                    \
     case rq:                                                                                                \
-        k_c_chip<G, K, NT, HOLD, rl><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, phase); \
+        k_c_chip<G, K, NT, HOLD, rl><<<n, c.threads, 0, st>>>(d_jobs, d_items, gin, gout, progress, polls, phase); \
         return
         MPF_CHIP(8, 6);
         MPF_CHIP(16, 5);
@@ -575,7 +575,7 @@ static void c_chip_dispatch(const CJob* d_jobs, const int4* d_items, int n, cons
 }
 
 void launch_c_chip(const CJob* d_jobs, const int4* d_items, int n, const ChipShape& c, int width, int Rq,
-                   const int2* gin, int2* gout, int* progress, int phase, hipStream_t st) {
+                   const int2* gin, int2* gout, int* progress, int polls, int phase, hipStream_t st) {
     // rows of one 8-slot group: the matrix stays in registers where they have room for it (20 per row;
     // 1280 rows 1.85 -> 1.54 ms per call, measured with the sums in the lanes' own order)
     const auto launch = c.K == 8 ? (c.threads > 512 ? c_chip_dispatch<1, 8, 1024, false>
@@ -583,7 +583,7 @@ void launch_c_chip(const CJob* d_jobs, const int4* d_items, int n, const ChipSha
                                                     : c_chip_dispatch<1, 8, 512, false>)
                         : width == 8 ? c_chip_dispatch<1, 4, 512, true>
                                      : c_chip_dispatch<1, 4, 512, false>;
-    launch(d_jobs, d_items, n, c, Rq, gin, gout, progress, phase, st);
+    launch(d_jobs, d_items, n, c, Rq, gin, gout, progress, polls, phase, st);
     check_launch();
 }
 

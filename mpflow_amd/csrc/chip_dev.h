@@ -147,10 +147,9 @@ __device__ __forceinline__ typename ChipVec<G>::type pack(const float (&v)[G]) {
 // Reference rule: the first column's group decides for its pair, and the others keep pace with it
 // instead of running after it.  After step k the leader publishes 2 k, or 2 k + 1 where it stops;
 // a follower ends step k only when it has seen that decision, so it never passes the leader's
-// last step.  The wait is bounded (about 0.1 ms): a follower that gives up keeps its state and goes
-// on in the next phase.  In place of leader first, followers after: forward solves of 817 nodes
-// 1.02 -> 0.58 ms, of two complex frames of 1261 nodes 1.57 -> 0.88 ms.
-constexpr int kLeadPolls = 128;
+// last step.  The wait is bounded (kLeadPolls: about 0.1 ms): a follower that gives up keeps its
+// state and goes on in the next phase.  In place of leader first, followers after: forward solves of
+// 817 nodes 1.02 -> 0.58 ms, of two complex frames of 1261 nodes 1.57 -> 0.88 ms.
 __device__ __forceinline__ int lead_seen(const int* progress) {
     return __hip_atomic_load(progress, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -158,9 +157,9 @@ __device__ __forceinline__ void lead_tell(int* progress, int v) {
     __hip_atomic_store(progress, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // the leader's word on `step` (`seen`: an earlier look); -1: none in time
-__device__ __forceinline__ int lead_word(const int* progress, int step, int seen) {
+__device__ __forceinline__ int lead_word(const int* progress, int step, int seen, int polls) {
     for (int i = 0; (seen >> 1) < step; ++i) {
-        if (i == kLeadPolls) return -1;
+        if (i >= polls) return -1;
         __builtin_amdgcn_s_sleep(1);
         seen = lead_seen(progress);
     }

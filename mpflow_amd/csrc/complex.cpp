@@ -137,11 +137,11 @@ void ComplexModel::Impl::run_chip() {
     hipStream_t st0 = ctx->stream;
     const int groups = Rq / shape.G, total = njs * groups;
     launch_c_chip_pack(jobs.p, js.p, njs, S.np, progress.p, total, st0);
-    launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, Rq, gst[1].p, gst[0].p, progress.p, 0, st0);
+    launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, Rq, gst[1].p, gst[0].p, progress.p, ctx->lead_polls, 0, st0);
     int in = 0;
     for (bool open = true; open;) {
-        launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, Rq, gst[in].p, gst[in ^ 1].p, progress.p, 1,
-                      st0);
+        launch_c_chip(jobs.p, chip_items.p, total, shape, S.wpad, Rq, gst[in].p, gst[in ^ 1].p, progress.p,
+                      ctx->lead_polls, 1, st0);
         in ^= 1;
         MPF_HIP(hipMemcpyAsync(h_gst, gst[in].p, sizeof(int2) * total, hipMemcpyDeviceToHost, st0));
         MPF_HIP(hipStreamSynchronize(st0));

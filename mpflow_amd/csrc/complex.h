@@ -91,7 +91,7 @@ void launch_c_chip_pack(const CJob* d_jobs, const int2* d_js, int njs, int np, i
 // one phase over `n` items (frame, slice, lane group, index of the pair's first group state), as
 // launch_chip
 void launch_c_chip(const CJob* d_jobs, const int4* d_items, int n, const ChipShape& c, int width, int Rq,
-                   const int2* gin, int2* gout, int* progress, int phase, hipStream_t st);
+                   const int2* gin, int2* gout, int* progress, int polls, int phase, hipStream_t st);
 void launch_c_voltages(const CJob* d_jobs, int njobs, const CMeasDev& md, float2* U32, zd* U64, hipStream_t st);
 void launch_c_jacobian(const CJob* d_jobs, int njobs, const CJacDev& jd, float2* J, hipStream_t st);
 // G_b = J_b J_b^T + shift I (complex symmetric, FP64 sums of the FP32 J, both triangles);

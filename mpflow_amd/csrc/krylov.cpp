@@ -299,8 +299,8 @@ void KrylovDriver::run_chip() {
         for (auto& c : chips) {
             hipStream_t s = c.stream ? c.stream : s0;
             if (c.stream) MPF_HIP(hipStreamWaitEvent(s, chip_fork, 0));
-            launch_chip(jobs.p, c.items.p, (int)c.h_items.size(), c.shape, gst[in].p, gst[in ^ 1].p, progress.p, ph,
-                        s);
+            launch_chip(jobs.p, c.items.p, (int)c.h_items.size(), c.shape, gst[in].p, gst[in ^ 1].p, progress.p,
+                        ctx->lead_polls, ph, s);
             if (c.stream) {
                 MPF_HIP(hipEventRecord(c.done, s));
                 MPF_HIP(hipStreamWaitEvent(s0, c.done, 0));

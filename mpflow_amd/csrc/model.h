@@ -21,6 +21,7 @@ struct mpf_ctx {
     double prof_bytes = 0.0;       // algorithmic bytes of the timed launches
     std::pair<hipEvent_t, hipEvent_t> next_events();
     void collect_events();
+    int lead_polls = mpf::kLeadPolls;   // on-chip solves: bound of a lane group's wait
     mpf::AutotuneCache tune;
 };
 

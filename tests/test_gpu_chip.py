@@ -66,3 +66,26 @@ def test_on_chip_matches_streamed(gpu_ctx, shape):
     b, sb = _solve(eit, g, gpu_ctx, True)
     assert abs(sa.steps - sb.steps) <= 0.1 * sb.steps + 4
     assert np.max(np.abs(a - b)) / np.max(np.abs(b)) < 1e-5
+
+
+@pytest.mark.parametrize("shape", [SHAPES[1], SHAPES[2], SHAPES[4], SHAPES[5]], ids=lambda s: "-".join(map(str, s)))
+def test_groups_that_give_up_waiting_take_the_same_steps(gpu_ctx, shape):
+    """Reference rule: with no polls allowed the lane groups stop waiting for the deciding one at once, keep
+    their state and go on in the launch after it: the same steps, the same bits."""
+    import torch
+    from mpflow_amd import capi
+    rings, L, C, p2, frames, z = shape
+    p = make_problem(rings, L, 1.6 / L, C=C, height=1.0 if C == 1 else 0.4, port_height=1.0 if C == 1 else 0.1, p2=p2)
+    eit = eit_of(p, gpu_ctx, frames=frames, contact_impedance=z)
+    g = torch.tensor(np.stack([ellipse_phantom(p["nodes"], p["elements"], frame_seed(2, f)) for f in range(frames)]),
+                     dtype=torch.float32)
+    for kw in (dict(), dict(max_iter=7), dict(preconditioner=1)):
+        print("case: on-chip without waiting %s %s" % (shape, kw), flush=True)
+        a, sa = _solve(eit, g, gpu_ctx, False, **kw)
+        capi.check(capi.lib().mpf_ctx_lead_polls(gpu_ctx.h, 0))
+        try:
+            b, sb = _solve(eit, g, gpu_ctx, False, **kw)
+        finally:
+            capi.check(capi.lib().mpf_ctx_lead_polls(gpu_ctx.h, 128))
+        assert (sa.steps, sa.max_steps, sa.not_converged) == (sb.steps, sb.max_steps, sb.not_converged)
+        assert np.isfinite(a).all() and np.array_equal(a, b)
