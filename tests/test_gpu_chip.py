@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from mpflow_amd.phantom import ellipse_phantom, frame_seed
-from tests.problems import eit_of, make_problem
+from tests.problems import eit_of, make_problem, oracle_of
 
 pytestmark = pytest.mark.gpu
 
@@ -89,3 +89,24 @@ def test_groups_that_give_up_waiting_take_the_same_steps(gpu_ctx, shape):
             capi.check(capi.lib().mpf_ctx_lead_polls(gpu_ctx.h, 128))
         assert (sa.steps, sa.max_steps, sa.not_converged) == (sb.steps, sb.max_steps, sb.not_converged)
         assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("shape", SHAPES[:7], ids=lambda s: "-".join(map(str, s)))
+def test_on_chip_matches_the_oracle(gpu_ctx, shape):
+    import torch
+    from mpflow_amd import capi
+    rings, L, C, p2, frames, z = shape
+    p = make_problem(rings, L, 1.6 / L, C=C, height=1.0 if C == 1 else 0.4, port_height=1.0 if C == 1 else 0.1, p2=p2)
+    eit, o = eit_of(p, gpu_ctx, frames=frames, contact_impedance=z), oracle_of(p, contact_impedance=z)
+    g = np.stack([ellipse_phantom(p["nodes"], p["elements"], frame_seed(2, f)) for f in range(frames)]).astype(np.float32)
+    u = np.stack([o.solve(x.astype(np.float64))[0] for x in g])
+    # FP64 refinement to 1e-8 of the right-hand side; FP32 to 1e-6 with the iteration's own error, as the
+    # forward solves' comparisons allow
+    mixed = dict(precision=capi.MPF_PREC_MIXED, tol=1e-5, refine_steps=2, refine_tol=1e-3)
+    for pre in (0, 1):
+        for kw, bound in ((mixed, 1e-6), (dict(tol=1e-6), 2e-5)):
+            print("case: on-chip against the oracle %s preconditioner %d" % (shape, pre), flush=True)
+            a, st = _solve(eit, torch.tensor(g), gpu_ctx, False, stop_rule=capi.MPF_STOP_TOLERANCE, preconditioner=pre, **kw)
+            err = np.max(np.abs(a - u)) / np.max(np.abs(u))
+            print("error %.2e" % err)
+            assert st.not_converged == 0 and err < bound
