@@ -441,7 +441,7 @@ __global__ void __launch_bounds__(256) k_c_gemv_t(int m, int E, const float2* __
     const zd* xv = x + b * stridex;
     zd a = zmake(0.0);
     for (int i = lane; i < m; i += 64) a += zf(col[i]) * xv[i];
-    for (int off = 32; off > 0; off >>= 1) a += Scal<zd>::shfl_xor(a, off);
+    for (int off = 32; off > 0; off >>= 1) a += zshfl_xor(a, off);
     if (lane == 0) {
         y[b * stridey + e] = a;
         if (gamma) {

@@ -49,29 +49,9 @@ __host__ __device__ inline zd zexp(zd a) {
 __host__ __device__ inline zd zf(float2 v) { return zd{(double)v.x, (double)v.y}; }
 __host__ __device__ inline float2 fz(zd v) { return make_float2((float)v.x, (float)v.y); }
 
-// Scalar traits shared by the real and complex instantiations of the dense kernels: the
-// formulas of an L L^T factorisation and its triangular solves are the same for real
-// symmetric positive definite and for complex symmetric (not Hermitian) matrices.
-template <class T> struct Scal;
-template <> struct Scal<double> {
-    __device__ static double zero() { return 0.0; }
-    __device__ static double one() { return 1.0; }
-    __device__ static double sqrt_(double a) { return sqrt(a); }
-    // a usable pivot: positive for the real factorisation
-    __device__ static bool pivot_ok(double a) { return a > 0.0; }
-    __device__ static double tiny() { return 1e-300; }
-    __device__ static double shfl(double v, int src) { return __shfl(v, src, 64); }
-    __device__ static double shfl_xor(double v, int m) { return __shfl_xor(v, m, 64); }
-};
-template <> struct Scal<zd> {
-    __device__ static zd zero() { return zd{0.0, 0.0}; }
-    __device__ static zd one() { return zd{1.0, 0.0}; }
-    __device__ static zd sqrt_(zd a) { return zsqrt(a); }
-    // a usable pivot: finite and nonzero (complex symmetric matrices have no sign test)
-    __device__ static bool pivot_ok(zd a) { return !zzero(a) && isfinite(a.x) && isfinite(a.y); }
-    __device__ static zd tiny() { return zd{1e-300, 0.0}; }
-    __device__ static zd shfl(zd v, int src) { return zd{__shfl(v.x, src, 64), __shfl(v.y, src, 64)}; }
-    __device__ static zd shfl_xor(zd v, int m) { return zd{__shfl_xor(v.x, m, 64), __shfl_xor(v.y, m, 64)}; }
-};
+// a usable pivot of a complex symmetric L L^T: finite and nonzero (there is no sign to test)
+__device__ inline bool zpivot_ok(zd a) { return !zzero(a) && isfinite(a.x) && isfinite(a.y); }
+__device__ inline zd zshfl(zd v, int src) { return zd{__shfl(v.x, src, 64), __shfl(v.y, src, 64)}; }
+__device__ inline zd zshfl_xor(zd v, int m) { return zd{__shfl_xor(v.x, m, 64), __shfl_xor(v.y, m, 64)}; }
 
 }  // namespace mpf

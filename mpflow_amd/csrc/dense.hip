@@ -674,25 +674,24 @@ constexpr int kCB = 32;
 // transposes, no conjugation); the real ones are factored in spd.hip.
 //
 // factor the diagonal block kb in place
-template <class T>
-__global__ void __launch_bounds__(256) k_potrf_diag(int n, T* __restrict__ A, size_t strideA, int kb,
+__global__ void __launch_bounds__(256) k_potrf_diag(int n, zd* __restrict__ A, size_t strideA, int kb,
                                                     int* __restrict__ info) {
-    T* a = A + blockIdx.z * strideA;
-    __shared__ T L[kCB][kCB + 1];
+    zd* a = A + blockIdx.z * strideA;
+    __shared__ zd L[kCB][kCB + 1];
     const int o = kb * kCB, nb = min(kCB, n - o);
     for (int i = threadIdx.x; i < kCB * kCB; i += 256) {
         const int r = i % kCB, c = i / kCB;
-        L[r][c] = (r < nb && c < nb) ? a[(o + r) + (size_t)(o + c) * n] : Scal<T>::zero();
+        L[r][c] = (r < nb && c < nb) ? a[(o + r) + (size_t)(o + c) * n] : zmake(0.0);
     }
     __syncthreads();
     for (int j = 0; j < nb; ++j) {
         if (threadIdx.x == 0) {
-            T d = L[j][j];
-            if (!Scal<T>::pivot_ok(d)) { atomicExch(info, 1); d = Scal<T>::tiny(); }
-            L[j][j] = Scal<T>::sqrt_(d);
+            zd d = L[j][j];
+            if (!zpivot_ok(d)) { atomicExch(info, 1); d = zmake(1e-300); }
+            L[j][j] = zsqrt(d);
         }
         __syncthreads();
-        const T djj = L[j][j];
+        const zd djj = L[j][j];
         for (int r = j + 1 + threadIdx.x; r < nb; r += 256) L[r][j] /= djj;
         __syncthreads();
         // trailing update of the block: L[r][c] -= L[r][j] L[c][j], c in (j, r]
@@ -709,27 +708,26 @@ __global__ void __launch_bounds__(256) k_potrf_diag(int n, T* __restrict__ A, si
 }
 
 // panel: A[ib, kb] <- A[ib, kb] L_kk^-T for every row block ib > kb (blockIdx.x)
-template <class T>
-__global__ void __launch_bounds__(256) k_potrf_panel(int n, T* __restrict__ A, size_t strideA, int kb) {
-    T* a = A + blockIdx.z * strideA;
+__global__ void __launch_bounds__(256) k_potrf_panel(int n, zd* __restrict__ A, size_t strideA, int kb) {
+    zd* a = A + blockIdx.z * strideA;
     const int o = kb * kCB;
     const int ib = kb + 1 + blockIdx.x;
     const int ro = ib * kCB;
     if (ro >= n) return;
     const int nr = min(kCB, n - ro), nb = min(kCB, n - o);
-    __shared__ T L[kCB][kCB + 1];
-    __shared__ T X[kCB][kCB + 1];
+    __shared__ zd L[kCB][kCB + 1];
+    __shared__ zd X[kCB][kCB + 1];
     for (int i = threadIdx.x; i < kCB * kCB; i += 256) {
         const int r = i % kCB, c = i / kCB;
-        L[r][c] = (r < nb && c < nb) ? a[(o + r) + (size_t)(o + c) * n] : Scal<T>::zero();
-        X[r][c] = (r < nr && c < nb) ? a[(ro + r) + (size_t)(o + c) * n] : Scal<T>::zero();
+        L[r][c] = (r < nb && c < nb) ? a[(o + r) + (size_t)(o + c) * n] : zmake(0.0);
+        X[r][c] = (r < nr && c < nb) ? a[(ro + r) + (size_t)(o + c) * n] : zmake(0.0);
     }
     __syncthreads();
     // each row r of X solves x L^T = a  (forward substitution over columns)
     if (threadIdx.x < nr) {
         const int r = threadIdx.x;
         for (int c = 0; c < nb; ++c) {
-            T s = X[r][c];
+            zd s = X[r][c];
             for (int t = 0; t < c; ++t) s -= X[r][t] * L[c][t];
             X[r][c] = s / L[c][c];
         }
@@ -742,26 +740,25 @@ __global__ void __launch_bounds__(256) k_potrf_panel(int n, T* __restrict__ A, s
 }
 
 // trailing update: A[ib, jb] -= L[ib, kb] L[jb, kb]^T for kb < jb <= ib
-template <class T>
-__global__ void __launch_bounds__(256) k_potrf_update(int n, T* __restrict__ A, size_t strideA, int kb,
+__global__ void __launch_bounds__(256) k_potrf_update(int n, zd* __restrict__ A, size_t strideA, int kb,
                                                       const int2* __restrict__ pairs) {
-    T* a = A + blockIdx.z * strideA;
+    zd* a = A + blockIdx.z * strideA;
     const int2 pr = pairs[blockIdx.x];
     const int ib = pr.x, jb = pr.y;
     const int o = kb * kCB, ro = ib * kCB, co = jb * kCB;
     const int nb = min(kCB, n - o), nr = min(kCB, n - ro), nc = min(kCB, n - co);
-    __shared__ T Li[kCB][kCB + 1];
-    __shared__ T Lj[kCB][kCB + 1];
+    __shared__ zd Li[kCB][kCB + 1];
+    __shared__ zd Lj[kCB][kCB + 1];
     for (int i = threadIdx.x; i < kCB * kCB; i += 256) {
         const int r = i % kCB, c = i / kCB;
-        Li[r][c] = (r < nr && c < nb) ? a[(ro + r) + (size_t)(o + c) * n] : Scal<T>::zero();
-        Lj[r][c] = (r < nc && c < nb) ? a[(co + r) + (size_t)(o + c) * n] : Scal<T>::zero();
+        Li[r][c] = (r < nr && c < nb) ? a[(ro + r) + (size_t)(o + c) * n] : zmake(0.0);
+        Lj[r][c] = (r < nc && c < nb) ? a[(co + r) + (size_t)(o + c) * n] : zmake(0.0);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < kCB * kCB; i += 256) {
         const int r = i % kCB, c = i / kCB;
         if (r < nr && c < nc && (ib != jb || r >= c)) {
-            T s = Scal<T>::zero();
+            zd s = zmake(0.0);
             for (int t = 0; t < nb; ++t) s += Li[r][t] * Lj[c][t];
             a[(ro + r) + (size_t)(co + c) * n] -= s;
         }
@@ -774,16 +771,15 @@ __global__ void __launch_bounds__(256) k_potrf_update(int n, T* __restrict__ A, 
 // wavefront read contiguous column segments of L and reduce them with shuffles.
 constexpr int kTrsvThreads = 1024;
 
-template <class T>
-__global__ void __launch_bounds__(kTrsvThreads) k_potrs(int n, const T* __restrict__ A, size_t strideA,
-                                                        const T* __restrict__ b, size_t strideb,
-                                                        T* __restrict__ y, size_t stridey) {
-    const T* a = A + blockIdx.x * strideA;
-    T* yv = y + blockIdx.x * stridey;
-    const T* bv = b + blockIdx.x * strideb;
+__global__ void __launch_bounds__(kTrsvThreads) k_potrs(int n, const zd* __restrict__ A, size_t strideA,
+                                                        const zd* __restrict__ b, size_t strideb,
+                                                        zd* __restrict__ y, size_t stridey) {
+    const zd* a = A + blockIdx.x * strideA;
+    zd* yv = y + blockIdx.x * stridey;
+    const zd* bv = b + blockIdx.x * strideb;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwave = kTrsvThreads / 64;
-    __shared__ T Lb[kCB][kCB + 1];
-    __shared__ T z[kCB];
+    __shared__ zd Lb[kCB][kCB + 1];
+    __shared__ zd z[kCB];
     for (int i = tid; i < n; i += kTrsvThreads) yv[i] = bv[i];
     __syncthreads();
     const int nblk = (n + kCB - 1) / kCB;
@@ -792,13 +788,13 @@ __global__ void __launch_bounds__(kTrsvThreads) k_potrs(int n, const T* __restri
         const int o = kb * kCB, nb = min(kCB, n - o);
         for (int i = tid; i < kCB * kCB; i += kTrsvThreads) {
             const int r = i % kCB, c = i / kCB;
-            Lb[r][c] = (r < nb && c < nb) ? a[(o + r) + (size_t)(o + c) * n] : (r == c ? Scal<T>::one() : Scal<T>::zero());
+            Lb[r][c] = (r < nb && c < nb) ? a[(o + r) + (size_t)(o + c) * n] : (r == c ? zmake(1.0) : zmake(0.0));
         }
         __syncthreads();
         if (wave == 0) {
-            T v = lane < nb ? yv[o + lane] : Scal<T>::zero();
+            zd v = lane < nb ? yv[o + lane] : zmake(0.0);
             for (int r = 0; r < nb; ++r) {
-                const T zr = Scal<T>::shfl(v, r) / Lb[r][r];
+                const zd zr = zshfl(v, r) / Lb[r][r];
                 if (lane == r) v = zr;
                 else if (lane > r && lane < nb) v -= Lb[lane][r] * zr;
             }
@@ -806,7 +802,7 @@ __global__ void __launch_bounds__(kTrsvThreads) k_potrs(int n, const T* __restri
         }
         __syncthreads();
         for (int r = o + nb + tid; r < n; r += kTrsvThreads) {
-            T s = Scal<T>::zero();
+            zd s = zmake(0.0);
             for (int t = 0; t < nb; ++t) s += a[r + (size_t)(o + t) * n] * z[t];
             yv[r] -= s;
         }
@@ -817,13 +813,13 @@ __global__ void __launch_bounds__(kTrsvThreads) k_potrs(int n, const T* __restri
         const int o = kb * kCB, nb = min(kCB, n - o);
         for (int i = tid; i < kCB * kCB; i += kTrsvThreads) {
             const int r = i % kCB, c = i / kCB;
-            Lb[r][c] = (r < nb && c < nb) ? a[(o + r) + (size_t)(o + c) * n] : (r == c ? Scal<T>::one() : Scal<T>::zero());
+            Lb[r][c] = (r < nb && c < nb) ? a[(o + r) + (size_t)(o + c) * n] : (r == c ? zmake(1.0) : zmake(0.0));
         }
         __syncthreads();
         if (wave == 0) {
-            T v = lane < nb ? yv[o + lane] : Scal<T>::zero();
+            zd v = lane < nb ? yv[o + lane] : zmake(0.0);
             for (int r = nb - 1; r >= 0; --r) {
-                const T zr = Scal<T>::shfl(v, r) / Lb[r][r];
+                const zd zr = zshfl(v, r) / Lb[r][r];
                 if (lane == r) v = zr;
                 else if (lane < r) v -= Lb[r][lane] * zr;
             }
@@ -832,8 +828,8 @@ __global__ void __launch_bounds__(kTrsvThreads) k_potrs(int n, const T* __restri
         __syncthreads();
         // y[c] -= sum_t L[o+t][c] z[t] for c < o: column segment a[o..o+nb, c] is contiguous
         for (int c = wave; c < o; c += nwave) {
-            T p = lane < nb ? a[(o + lane) + (size_t)c * n] * z[lane] : Scal<T>::zero();
-            for (int off = 32; off > 0; off >>= 1) p += Scal<T>::shfl_xor(p, off);
+            zd p = lane < nb ? a[(o + lane) + (size_t)c * n] * z[lane] : zmake(0.0);
+            for (int off = 32; off > 0; off >>= 1) p += zshfl_xor(p, off);
             if (lane == 0) yv[c] -= p;
         }
         __syncthreads();
@@ -1250,11 +1246,11 @@ void launch_cholesky_z(int n, zd* A, size_t strideA, int batch, int* d_info, int
     const int nblk = (n + kCB - 1) / kCB;
     k_chol_pairs<<<(nblk + 255) / 256, 256, 0, st>>>(nblk, d_pairs);
     for (int kb = 0; kb < nblk; ++kb) {
-        k_potrf_diag<zd><<<dim3(1, 1, batch), 256, 0, st>>>(n, A, strideA, kb, d_info);
+        k_potrf_diag<<<dim3(1, 1, batch), 256, 0, st>>>(n, A, strideA, kb, d_info);
         if (kb + 1 < nblk) {
-            k_potrf_panel<zd><<<dim3(nblk - kb - 1, 1, batch), 256, 0, st>>>(n, A, strideA, kb);
+            k_potrf_panel<<<dim3(nblk - kb - 1, 1, batch), 256, 0, st>>>(n, A, strideA, kb);
             const int p0 = chol_pair_start(nblk, kb), np = chol_pair_start(nblk, kb + 1) - p0;
-            k_potrf_update<zd><<<dim3(np, 1, batch), 256, 0, st>>>(n, A, strideA, kb, d_pairs + p0);
+            k_potrf_update<<<dim3(np, 1, batch), 256, 0, st>>>(n, A, strideA, kb, d_pairs + p0);
         }
     }
     check_launch();
@@ -1262,7 +1258,7 @@ void launch_cholesky_z(int n, zd* A, size_t strideA, int batch, int* d_info, int
 
 void launch_potrs_z(int n, const zd* A, size_t strideA, const zd* b, size_t strideb, zd* y, size_t stridey,
                     int batch, hipStream_t st) {
-    k_potrs<zd><<<batch, kTrsvThreads, 0, st>>>(n, A, strideA, b, strideb, y, stridey);
+    k_potrs<<<batch, kTrsvThreads, 0, st>>>(n, A, strideA, b, strideb, y, stridey);
     check_launch();
 }
 
