@@ -19,7 +19,9 @@
 // matrix with 32 columns 2.02 -> 0.56 ms.
 //
 // The recurrences, the FP64 scalars, the stop rules and the breakdown rules are those of the
-// streaming kernels (sparse.hip); sums run in a fixed order.
+// streaming kernels (sparse.hip); sums run in a fixed order.  One difference: a column that breaks
+// down (NaN) stops its lane group alone, not every column of its pair; the pair reports it all the
+// same.  A solve is one launch: it ends at its stop rule or after max_iter iterations.
 #include <climits>
 
 #include "chip_dev.h"

@@ -11,7 +11,8 @@
 // CPU: median 1.7e-7, worst 3.5e-6; one problem has 1.5e-7 in three orders and 3.2e-6 in the
 // fourth).  The streamed order is: a thread adds the rows rr, rr + rpp, ... of its tile (rpp =
 // 512 / Rq rows per pass), one lane adds the tile's rpp sums, then the tiles.  Hence a wavefront
-// owns whole tiles, its lane the rows l, l + 64, ...
+// owns whole tiles, its lane the rows l, l + 64, ...  (A column that breaks down stops its lane group
+// alone, not every column of its pair as there; the pair reports it all the same.)
 //
 // Bound by the chain of an iteration (two block sums with their barriers, two complex divisions,
 // the gathers), not by any pipe.  Measured (MI355X): two frames x 3 harmonics of 1261 nodes, 16

@@ -14,6 +14,10 @@
 // Tiles are 64 x 64, products on v_mfma_f64_16x16x4_f64.  Bound by the chain of n / 64 diagonal
 // factorisations for one frame (64 dependent columns each), by FP64 MFMA for many.
 //
+// Error against an extended-precision solve, n = 63, 200 and 321, condition 1e2 to 1e7: forward 1.0 to
+// 1.75 times that of factor and substitutions (1.4e-10 against 0.9e-10 at 1e7), residual 1 to 6 times
+// (7e-10 against 1e-10): far below what the normal equations carry in, which are FP32 sums.
+//
 // Measured (MI355X, n = 1024, against the 32-column factorisation in three launches per block
 // column and one-workgroup substitutions): the first diagonal tile 41 -> 24 us, a step's panel
 // 16.8 -> 7.4 us and update 48 -> 28 us (64 matrices 294 -> 138 us), the arrows from this file's
