@@ -1,6 +1,6 @@
 """The on-chip complex conjugate gradients (whole solves in one workgroup per lane group) against
 the streamed iteration of the same solve -- a profiled context streams every mesh -- at the edges
-of its shapes: one row per thread, a partial last tile, both lane-group sizes, rows wider than
+of its shapes: one tile, a partial last tile, both lane-group sizes, rows wider than
 8 entries, the largest mesh it takes and the first one it does not."""
 import numpy as np
 import pytest
@@ -11,11 +11,11 @@ pytestmark = pytest.mark.gpu
 
 # rings, electrodes, harmonics, P2, frames
 SHAPES = [
-    (5, 8, 1, False, 1),        # 91 nodes: one tile, 256 threads
-    (16, 16, 2, False, 1),      # 817 nodes: one row per thread
+    (5, 8, 1, False, 1),        # 91 nodes: one tile, one wavefront
+    (16, 16, 2, False, 1),      # 817 nodes: four tiles
     (18, 20, 3, False, 1),      # 1027 nodes: one row past 1024, 12 empty lanes
     (14, 16, 2, True, 1),       # P2: rows of 9 and 19 entries
-    (20, 16, 3, False, 8),      # two lanes, 1261 nodes
+    (20, 16, 3, False, 8),      # 1261 nodes, more groups than CUs
     (36, 16, 1, False, 20),     # two lanes, 3997 nodes
     (51, 16, 1, False, 1),      # 7957 nodes: the largest
     (52, 16, 1, False, 1),      # 8269 nodes: streamed
