@@ -84,6 +84,13 @@ ORDER = [
     (30, 8, 2, False, 20, False),     # stride 8, two lanes
     (51, 16, 1, False, 2, False),     # 32 tiles: 1024 threads
     (45, 12, 1, False, 1, False),     # 25 tiles: some wavefronts with one tile
+    (12, 8, 1, True, 2, False),       # P2, one tile per wavefront: stride 8
+    (12, 20, 1, True, 2, False),      # and stride 32
+    (30, 8, 1, False, 1, False),      # one lane, two tiles per wavefront: stride 8
+    (30, 32, 1, False, 1, False),     # stride 32
+    (30, 32, 1, False, 1, True),      # stride 64
+    (45, 8, 1, False, 1, False),      # 1024 threads: stride 8
+    (45, 24, 1, False, 1, False),     # stride 32
 ]
 
 
